@@ -15,12 +15,21 @@
 // are written in increasing offset (the reference's order comes from an atomic counter,
 // so any order is a valid instance of its format); padding bytes are zero.
 //
-// Kernels: a count pass (one workgroup per chunk, per box: existing points inside),
-// per-box scans of the counts and of the non-empty flags, then a write pass (one
-// workgroup per chunk, wave-ballot compaction keeps offsets ascending).  Unpack expands
-// a section into point records (key = packed coordinate - box start + destination
-// start) appended to the insert buffer; the finalize removes the queued boxes and
-// flushes with the unpacked properties taking the new values.
+// Kernels: a count pass (one wave per chunk, per box: existing points inside), one scan of
+// the counts and the non-empty flags of all boxes, then a write pass over all boxes (one
+// wave per chunk, ballot compaction keeps offsets ascending).  Unpack expands a section
+// into point records (key = packed coordinate - box start + destination start) appended to
+// the insert buffer; the finalize removes the queued boxes and flushes with the unpacked
+// properties taking the new values.
+//
+// Ghost layers are small (a few thousand points of a few per cent of the chunks), so these
+// calls are bound by launches, waits and the cost of passing over chunks that meet no box:
+// boxes travel as kernel arguments, one launch covers all boxes, totals and flags come back
+// through pinned words, and a wave leaves a chunk outside every box after some 60
+// instructions (a workgroup per chunk with 64-bit divisions in every thread took 106 us for
+// 22,000 chunks in each of the count and removal passes, and 16 us a box in the write pass).
+// Six ghost slabs of width 3 of a 250^3 sheet packed, removed and unpacked
+// (two FP32 fields, 25,000 chunks): 1.63 -> 0.47 ms, the flush that merges them included.
 #include "sg_internal.hpp"
 
 #include <algorithm>
@@ -33,26 +42,60 @@ constexpr int kWG = 256;
 
 struct Geom {
     int dim, edge, csz;
+    int sh;     // log2 of the edge, or -1
+    int ids32;  // row-major chunk ids (below 2^31): 32-bit divisions
     ChunkLin L;
 };
 
+// chunk coordinates of chunk id `id` (any value: ids of packed sections are not trusted)
+__device__ inline void chunk_coords_of(const Geom &G, const int64_t *bsz, int64_t id, int64_t *bc)
+{
+    if (G.ids32 && (uint64_t)id < ((uint64_t)1 << 31)) {
+        uint32_t t = (uint32_t)id;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (d >= G.dim) break;
+            const uint32_t b = (uint32_t)bsz[d], q = t / b;
+            bc[d] = (int64_t)(t - q * b);
+            t = q;
+        }
+        return;
+    }
+    ChunkLin L = G.L;
+    for (int d = 0; d < 3; ++d) L.bsz[d] = bsz[d];
+    chunk_coords(L, id, bc);
+}
+
 __device__ inline void chunk_origin(const Geom &G, int64_t id, int64_t *o)
 {
-    chunk_coords(G.L, id, o);
-    for (int d = 0; d < G.dim; ++d) o[d] *= G.edge;
+    chunk_coords_of(G, G.L.bsz, id, o);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= G.dim) break;
+        o[d] *= G.edge;
+    }
 }
 
 __device__ inline void local_coord(const Geom &G, int off, int64_t *l)
 {
-    for (int d = 0; d < G.dim; ++d) {
-        l[d] = off % G.edge;
-        off /= G.edge;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= G.dim) break;
+        if (G.sh >= 0) {
+            l[d] = off & (G.edge - 1);
+            off >>= G.sh;
+        } else {
+            l[d] = off % G.edge;
+            off /= G.edge;
+        }
     }
 }
 
+// up to kBoxes inclusive boxes, in the kernel arguments
+constexpr int kBoxes = 32;
 struct Boxes {
     int n;
-    const int32_t *lo, *hi;  // [n][dim]
+    int32_t lo[kBoxes * 3], hi[kBoxes * 3];  // [n][dim]
 };
 
 // property set of a grid for kernels that write or read every property
@@ -69,226 +112,440 @@ __device__ inline void copy_scalar(unsigned char *dst, const unsigned char *src,
     for (int b = 0; b < ts; ++b) dst[b] = src[b];
 }
 
+// little-endian values at any address (one load where it is aligned)
+__device__ inline uint32_t load_u16(const unsigned char *p)
+{
+    if (((uintptr_t)p & 1) == 0) return *(const uint16_t *)p;
+    return (uint32_t)p[0] | ((uint32_t)p[1] << 8);
+}
+__device__ inline uint32_t load_u32(const unsigned char *p)
+{
+    if (((uintptr_t)p & 3) == 0) return *(const uint32_t *)p;
+    return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
+}
+__device__ inline uint64_t load_u64(const unsigned char *p)
+{
+    return (uint64_t)load_u32(p) | ((uint64_t)load_u32(p + 4) << 32);
+}
+
+// one value of ts bytes where both addresses are multiples of ts
+__device__ inline void copy_aligned(unsigned char *dst, const unsigned char *src, int ts)
+{
+    switch (ts) {
+    case 8: *(uint64_t *)dst = *(const uint64_t *)src; break;
+    case 4: *(uint32_t *)dst = *(const uint32_t *)src; break;
+    case 2: *(uint16_t *)dst = *(const uint16_t *)src; break;
+    default: *dst = *src; break;
+    }
+}
+
 __device__ inline void clear_slot(const PropSet &P, uint8_t *mask, int64_t slot)
 {
     mask[slot] = 0;
     for (int q = 0; q < P.np; ++q)
-        copy_scalar((unsigned char *)P.p[q] + slot * P.ts[q], (const unsigned char *)&P.bg[q], P.ts[q]);
+        copy_aligned((unsigned char *)P.p[q] + slot * P.ts[q], (const unsigned char *)&P.bg[q], P.ts[q]);
 }
 
 __device__ inline bool chunk_meets_box(const Geom &G, const int64_t *org, const int32_t *lo, const int32_t *hi)
 {
-    for (int d = 0; d < G.dim; ++d)
-        if (org[d] + G.edge - 1 < lo[d] || org[d] > hi[d]) return false;
-    return true;
+    bool met = true;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= G.dim) break;
+        met = met && org[d] + G.edge - 1 >= lo[d] && org[d] <= hi[d];
+    }
+    return met;
 }
 
-__device__ inline bool point_in_box(const Geom &G, const int64_t *c, const int32_t *lo, const int32_t *hi)
+// The kernels over chunks give lane l of a wave the slots [l V, (l + 1) V) of its chunk, V =
+// ceil(csz / 64) <= 16: their mask bytes are one load (V a template parameter where csz = 64 V;
+// 0 otherwise, byte loads), and lane order is slot order.
+__device__ inline int lane_slots(const Geom &G, int V) { return V > 0 ? V : (G.csz + 63) / 64; }
+
+// the masks of the lane's slots (0 past the chunk's end) and a bit per slot with EXIST
+template <int V>
+__device__ inline uint32_t lane_masks(const uint8_t *__restrict__ mask, int64_t c, const Geom &G, int lane,
+                                      uint32_t (&m)[4])
 {
-    for (int d = 0; d < G.dim; ++d)
-        if (c[d] < lo[d] || c[d] > hi[d]) return false;
-    return true;
+    m[0] = m[1] = m[2] = m[3] = 0;
+    if constexpr (V == 1) m[0] = mask[c * 64 + lane];
+    else if constexpr (V == 2) m[0] = ((const uint16_t *)mask)[c * 64 + lane];
+    else if constexpr (V == 4) m[0] = ((const uint32_t *)mask)[c * 64 + lane];
+    else if constexpr (V == 8) {
+        const uint2 q = ((const uint2 *)mask)[c * 64 + lane];
+        m[0] = q.x;
+        m[1] = q.y;
+    } else if constexpr (V == 16) {
+        const uint4 q = ((const uint4 *)mask)[c * 64 + lane];
+        m[0] = q.x;
+        m[1] = q.y;
+        m[2] = q.z;
+        m[3] = q.w;
+    } else {
+        const int n = lane_slots(G, 0);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int o = lane * n + v;
+            if (v < n && o < G.csz) m[v >> 2] |= (uint32_t)mask[c * G.csz + o] << (8 * (v & 3));
+        }
+    }
+    uint32_t e = 0;
+#pragma unroll
+    for (int v = 0; v < (V > 0 ? V : 16); ++v) e |= ((m[v >> 2] >> (8 * (v & 3))) & SG_EXIST) << v;
+    return e;
 }
 
-// existing points of chunk c inside each box: cnt[k * stride + c], flag = cnt != 0
-// (calc_exist_points_with_boxes, SparseGridGpu_kernels.cuh:1351-1420)
+// bit v: slot lane V + v of the chunk at org lies in the inclusive box (lo, hi)
+template <int V>
+__device__ inline uint32_t lane_box_bits(const Geom &G, const int64_t *org, const int32_t *lo, const int32_t *hi, int lane)
+{
+    // the box in chunk coordinates, cut to [0, edge)
+    int a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= G.dim) break;
+        const int64_t l = lo[d] - org[d], h = hi[d] - org[d];
+        a[d] = l < 0 ? 0 : (l > G.edge ? G.edge : (int)l);
+        b[d] = h < 0 ? -1 : (h > G.edge ? G.edge : (int)h);
+    }
+    const int n = lane_slots(G, V);
+    uint32_t in = 0;
+#pragma unroll
+    for (int v = 0; v < (V > 0 ? V : 16); ++v) {
+        int o = lane * n + v;
+        bool ok = v < n;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (d >= G.dim) break;
+            const int q = G.sh >= 0 ? o >> G.sh : o / G.edge, x = o - q * G.edge;
+            ok = ok && x >= a[d] && x <= b[d];
+            o = q;
+        }
+        in |= (ok ? 1u : 0u) << v;
+    }
+    return in;
+}
+
+// bit k of the result: the chunk at org meets box k (the lanes of the wave test a box each)
+__device__ inline uint32_t boxes_met(const Geom &G, const Boxes &B, const int64_t *org, int lane)
+{
+    bool met = false;
+    if (lane < B.n) met = chunk_meets_box(G, org, B.lo + lane * G.dim, B.hi + lane * G.dim);
+    return (uint32_t)__ballot(met);
+}
+
+// existing points of every chunk inside each box of B and whether there are any: box k's
+// counts at cnt[k * stride + c], its flags at flag[k * stride + c], entry n of both 0
+// (calc_exist_points_with_boxes, SparseGridGpu_kernels.cuh:1351-1420).  One wave per chunk
+// c <= n.
+template <int V>
 __global__ __launch_bounds__(kWG) void pack_count_kernel(const int64_t *__restrict__ keys, int64_t n,
                                                         const uint8_t *__restrict__ mask, Geom G, Boxes B,
                                                         uint32_t *__restrict__ cnt, uint32_t *__restrict__ flag,
                                                         int64_t stride)
 {
-    __shared__ uint32_t s_cnt;
-    const int64_t c = blockIdx.x;
-    if (c >= n) return;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int64_t c = (int64_t)blockIdx.x * (kWG / 64) + w;
+    if (c > n) return;
     int64_t org[3] = {0, 0, 0};
-    chunk_origin(G, keys[c], org);
-    for (int k = 0; k < B.n; ++k) {
-        const int32_t *lo = B.lo + k * G.dim, *hi = B.hi + k * G.dim;
-        uint32_t mine = 0;
-        if (chunk_meets_box(G, org, lo, hi)) {
-            for (int o = threadIdx.x; o < G.csz; o += kWG) {
-                if (!(mask[c * G.csz + o] & SG_EXIST)) continue;
-                int64_t l[3] = {0, 0, 0}, p[3];
-                local_coord(G, o, l);
-                for (int d = 0; d < G.dim; ++d) p[d] = org[d] + l[d];
-                mine += point_in_box(G, p, lo, hi) ? 1u : 0u;
-            }
+    uint32_t met = 0;
+    if (c < n) {
+        chunk_origin(G, keys[c], org);
+        met = boxes_met(G, B, org, lane);
+    }
+    uint32_t mine = 0;  // lane k: the points in box k
+    if (met) {
+        uint32_t m[4];
+        const uint32_t e = lane_masks<V>(mask, c, G, lane, m);
+        for (uint32_t left = met; left; left &= left - 1) {
+            const int k = __builtin_ctz(left);
+            uint32_t s = (uint32_t)__popc(e & lane_box_bits<V>(G, org, B.lo + k * G.dim, B.hi + k * G.dim, lane));
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) s += (uint32_t)__shfl_xor((int)s, o, 64);
+            mine = (lane == k) ? s : mine;
         }
-        if (threadIdx.x == 0) s_cnt = 0;
-        __syncthreads();
-        if (mine) atomicAdd(&s_cnt, mine);
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            cnt[k * stride + c] = s_cnt;
-            flag[k * stride + c] = s_cnt ? 1u : 0u;
-        }
-        __syncthreads();
+    }
+    if (lane < B.n) {
+        cnt[lane * stride + c] = mine;
+        flag[lane * stride + c] = mine ? 1u : 0u;
     }
 }
 
-struct PackOut {
-    unsigned char *ids;     // indexT [n_cnk]
-    uint32_t *scan;         // [n_cnk + 1]
-    unsigned char *data[kMaxProps];  // per packed property [n_pnt]
-    int ts[kMaxProps];
-    const unsigned char *src[kMaxProps];  // grid property arrays
-    int nprop;
-    int16_t *offs;          // [n_pnt]
-    uint8_t *masks;         // [n_pnt]
-    int A;                  // sizeof(indexT)
+// scan: the exclusive scan of the count rows of all boxes followed by their flag rows (per =
+// boxes * stride entries each; sums wrap, differences inside a row are exact).  Box k has
+// tot[2k] points in tot[2k + 1] chunks.
+__global__ void pack_totals_kernel(const uint32_t *__restrict__ scan, int64_t per, int64_t stride, int nbox,
+                                   uint32_t *__restrict__ tot)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= nbox) return;
+    const uint32_t *p = scan + (int64_t)k * stride;
+    tot[2 * k] = p[stride - 1] - p[0];
+    tot[2 * k + 1] = p[per + stride - 1] - p[per];
+}
+
+// the sections of the boxes of one write launch: byte offset in the buffer, chunks, points
+struct PackSections {
+    int64_t at[kBoxes];
+    uint32_t nc[kBoxes], np[kBoxes];
 };
 
-// write the points of box (lo, hi) of chunk c at their packed positions
-// (get_exist_points_with_boxes + pack_data, SparseGridGpu_kernels.cuh:1437-1697)
-__global__ __launch_bounds__(kWG) void pack_write_kernel(const int64_t *__restrict__ keys, int64_t n,
-                                                        const uint8_t *__restrict__ mask, Geom G, const int32_t *lo,
-                                                        const int32_t *hi, const uint32_t *__restrict__ pscan,
-                                                        const uint32_t *__restrict__ cscan,
-                                                        const uint32_t *__restrict__ cnt, PackOut O)
+struct PackProps {
+    int n;
+    int ts[kMaxProps];
+    const unsigned char *src[kMaxProps];  // grid property arrays
+};
+
+// a: a power of two
+__host__ __device__ inline int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) & ~(a - 1); }
+
+// addresses of one section's arrays
+struct SectionPtrs {
+    unsigned char *ids, *scan, *data, *offs, *masks, *end;
+};
+
+__device__ inline SectionPtrs section_ptrs(unsigned char *s0, int dim, int A, int64_t nc, int64_t np, int psz)
 {
-    __shared__ uint32_t s_wave[kWG / 64];
-    __shared__ uint32_t s_run;
-    const int64_t c = blockIdx.x;
-    if (c >= n || cnt[c] == 0) return;
-    const uint32_t slot = cscan[c], start = pscan[c];
-    const int64_t key = keys[c];
-    if (threadIdx.x == 0) {
-        if (O.A == 8) copy_scalar(O.ids + (int64_t)slot * 8, (const unsigned char *)&key, 8);
-        else {
-            const int32_t k4 = (int32_t)key;
-            copy_scalar(O.ids + (int64_t)slot * 4, (const unsigned char *)&k4, 4);
+    SectionPtrs S;
+    S.ids = s0 + 8 + 8 * dim;
+    S.scan = S.ids + A * nc;
+    S.data = S.scan + align_up((nc + 1) * 4, A);
+    S.offs = S.data + align_up(np * psz, A);
+    S.masks = S.offs + align_up(np * 2, A);
+    S.end = S.masks + align_up(np, A);
+    return S;
+}
+
+// Write the points of every box of B at their packed positions (get_exist_points_with_boxes
+// + pack_data, SparseGridGpu_kernels.cuh:1437-1697).  One wave per chunk c < n; wave n + k
+// writes the header, the scan's last entry and the zero padding of box k's section.  pscan /
+// cscan: the boxes' rows of the scan.
+template <int V>
+__global__ __launch_bounds__(kWG) void pack_write_kernel(const int64_t *__restrict__ keys, int64_t n,
+                                                        const uint8_t *__restrict__ mask, Geom G, Boxes B,
+                                                        const uint32_t *__restrict__ pscan,
+                                                        const uint32_t *__restrict__ cscan, int64_t stride, PackProps P,
+                                                        int psz, int A, PackSections X, unsigned char *buf, int32_t sz0,
+                                                        int32_t sz1, int32_t sz2)
+{
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int64_t c = (int64_t)blockIdx.x * (kWG / 64) + w;
+    if (c >= n + B.n) return;
+    if (c >= n) {
+        const int k = (int)(c - n);
+        unsigned char *s0 = buf + X.at[k];
+        const int64_t nc = X.nc[k], np = X.np[k];
+        const SectionPtrs S = section_ptrs(s0, G.dim, A, nc, np, psz);
+        // sections start at multiples of 4 bytes only: byte stores
+        if (lane < 8) s0[lane] = (unsigned char)((uint64_t)nc >> (8 * lane));
+        const int32_t sz[3] = {sz0, sz1, sz2};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (d >= G.dim || lane >= 4) continue;
+            s0[8 + 4 * d + lane] = (unsigned char)((uint32_t)B.lo[k * G.dim + d] >> (8 * lane));
+            s0[8 + 4 * (G.dim + d) + lane] = (unsigned char)((uint32_t)sz[d] >> (8 * lane));
         }
-        O.scan[slot] = start;
-        s_run = 0;
+        unsigned char *last = S.scan + 4 * nc;
+        if (lane < 4) last[lane] = (unsigned char)((uint32_t)np >> (8 * lane));
+        if (last + 4 + lane < S.data) last[4 + lane] = 0;
+        if (S.data + np * psz + lane < S.offs) S.data[np * psz + lane] = 0;
+        if (S.offs + np * 2 + lane < S.masks) S.offs[np * 2 + lane] = 0;
+        if (S.masks + np + lane < S.end) S.masks[np + lane] = 0;
+        return;
     }
+    // lane k: chunk c's first point and place in box k's section
+    uint32_t start = 0, cnt = 0, slot = 0;
+    if (lane < B.n) {
+        const uint32_t *row = pscan + lane * stride;
+        const uint32_t v = row[c];
+        cnt = row[c + 1] - v;
+        start = v - row[0];
+        slot = cscan[lane * stride + c] - cscan[lane * stride];
+    }
+    const uint32_t any = (uint32_t)__ballot(cnt != 0);
+    if (any == 0) return;
+    const int64_t key = keys[c];
     int64_t org[3] = {0, 0, 0};
     chunk_origin(G, key, org);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __syncthreads();
-    for (int o0 = 0; o0 < G.csz; o0 += kWG) {
-        const int o = o0 + threadIdx.x;
-        bool has = false;
-        if (o < G.csz && (mask[c * G.csz + o] & SG_EXIST)) {
-            int64_t l[3] = {0, 0, 0}, p[3];
-            local_coord(G, o, l);
-            for (int d = 0; d < G.dim; ++d) p[d] = org[d] + l[d];
-            has = point_in_box(G, p, lo, hi);
+    uint32_t m[4];
+    const uint32_t e = lane_masks<V>(mask, c, G, lane, m);
+    for (uint32_t left = any; left; left &= left - 1) {
+        const int k = __builtin_ctz(left);
+        const uint32_t st = (uint32_t)__shfl((int)start, k, 64), sl = (uint32_t)__shfl((int)slot, k, 64);
+        const int64_t np = X.np[k];
+        const SectionPtrs S = section_ptrs(buf + X.at[k], G.dim, A, X.nc[k], np, psz);
+        if (lane < A) S.ids[(int64_t)sl * A + lane] = (unsigned char)((uint64_t)key >> (8 * lane));
+        if (lane < 4) S.scan[(int64_t)sl * 4 + lane] = (unsigned char)(st >> (8 * lane));
+        const uint32_t in = e & lane_box_bits<V>(G, org, B.lo + k * G.dim, B.hi + k * G.dim, lane);
+        // the lanes' first points: exclusive prefix of their counts
+        const uint32_t own = (uint32_t)__popc(in);
+        uint32_t inc = own;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t u = (uint32_t)__shfl_up((int)inc, o, 64);
+            if (lane >= o) inc += u;
         }
-        const uint64_t bal = __ballot(has);
-        if (lane == 0) s_wave[w] = (uint32_t)__popcll(bal);
-        __syncthreads();
-        uint32_t pre = s_run, tot = 0;
-        for (int q = 0; q < kWG / 64; ++q) {
-            if (q < w) pre += s_wave[q];
-            tot += s_wave[q];
-        }
-        if (has) {
-            const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-            const int64_t j = (int64_t)start + pre + (uint32_t)__popcll(bal & lt);
+        int64_t j = (int64_t)st + inc - own;
+        const int o0 = lane * lane_slots(G, V);
+        for (uint32_t b = in; b; b &= b - 1, ++j) {
+            const int v = __builtin_ctz(b), o = o0 + v;
             const int64_t slot_pt = c * G.csz + o;
-            for (int q = 0; q < O.nprop; ++q)
-                copy_scalar(O.data[q] + j * O.ts[q], O.src[q] + slot_pt * O.ts[q], O.ts[q]);
-            O.offs[j] = (int16_t)o;
-            O.masks[j] = mask[slot_pt];
+            unsigned char *d = S.data;
+            for (int q = 0; q < P.n; ++q) {
+                const int ts = P.ts[q];
+                // arrays follow each other without alignment
+                if (((uintptr_t)d & (uintptr_t)(ts - 1)) == 0) copy_aligned(d + j * ts, P.src[q] + slot_pt * ts, ts);
+                else copy_scalar(d + j * ts, P.src[q] + slot_pt * ts, ts);
+                d += np * ts;
+            }
+            const int16_t o16 = (int16_t)o;
+            if (((uintptr_t)S.offs & 1) == 0) ((int16_t *)S.offs)[j] = o16;
+            else copy_scalar(S.offs + 2 * j, (const unsigned char *)&o16, 2);
+            const uint32_t mw = v < 8 ? (v < 4 ? m[0] : m[1]) : (v < 12 ? m[2] : m[3]);
+            S.masks[j] = (uint8_t)(mw >> (8 * (v & 3)));
         }
-        __syncthreads();
-        if (threadIdx.x == 0) s_run += tot;
-        __syncthreads();
     }
 }
 
 struct UnpackIn {
-    const unsigned char *ids;
-    const uint32_t *scan;
-    const unsigned char *data[kMaxProps];  // per grid property: packed array or null
-    const int16_t *offs;
-    int A;
-    int64_t pbsz[3];   // chunk counts of the packing grid
-    int32_t shift[3];  // destination start - packed box start
+    const unsigned char *buf;
+    int64_t avail;
+    int A, psz;                 // bytes of a chunk id, of a point's packed values
+    int off[kMaxProps];         // per grid property: packed bytes per point before its array, -1: not packed
+    int32_t dst_lo[3];
 };
 
-// packed chunk i -> point records at base + scan[i] .. (copy_packed_data_to_chunks,
-// SparseGridGpu_kernels.cuh:1591-1632; mask |= EXIST)
-__global__ __launch_bounds__(kWG) void unpack_records_kernel(UnpackIn U, int64_t n_cnk, int64_t n_pnt, Geom G,
-                                                            int64_t sz0, int64_t sz1, int64_t sz2, PropSet P,
-                                                            int64_t *__restrict__ rkey, uint8_t *__restrict__ rmask,
-                                                            int *__restrict__ bad)
+// words of a section's report (pinned host memory)
+enum { kUpChunks = 0, kUpStart = 2, kUpSize = 5, kUpPoints = 8, kUpState = 9, kUpBad = 10 };
+
+// One packed section in device memory: packed chunk i -> point records at scan[i] .. of the
+// record arrays (copy_packed_data_to_chunks, SparseGridGpu_kernels.cuh:1591-1632; mask |=
+// EXIST), one wave per chunk (grid stride).  Every wave reads the header itself, so the host
+// needs no look at the section before the launch: it learns n_cnk, box start, grid size,
+// n_pnt, the state (bit 0: the chunk list and scan lie inside the section; bit 1: the
+// records were written, as they are when the section is whole and `room` takes its points)
+// and whether a record was bad from the report, in one wait.
+__global__ __launch_bounds__(kWG) void unpack_section_kernel(UnpackIn U, Geom G, int64_t sz0, int64_t sz1, int64_t sz2,
+                                                            PropSet P, int64_t *__restrict__ rkey,
+                                                            uint8_t *__restrict__ rmask, int64_t room,
+                                                            uint32_t *__restrict__ rep)
 {
-    const int64_t i = blockIdx.x;
-    if (i >= n_cnk) return;
-    int64_t id;
-    if (U.A == 8) copy_scalar((unsigned char *)&id, U.ids + i * 8, 8);
-    else {
-        int32_t k4;
-        copy_scalar((unsigned char *)&k4, U.ids + i * 4, 4);
-        id = k4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int64_t first = (int64_t)blockIdx.x * (kWG / 64) + w, hsz = 8 + 8 * G.dim;
+    // a section may start at any address
+    const uint64_t nc = load_u64(U.buf);
+    int32_t bstart[3] = {0, 0, 0}, psize[3] = {1, 1, 1};
+    bool sizes = true;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= G.dim) break;
+        bstart[d] = (int32_t)load_u32(U.buf + 8 + 4 * d);
+        psize[d] = (int32_t)load_u32(U.buf + 8 + 4 * (G.dim + d));
+        sizes = sizes && psize[d] > 0;
     }
-    // chunk coordinates in the packing grid (same linearizer, its own chunk counts)
-    ChunkLin PL = G.L;
-    for (int d = 0; d < 3; ++d) PL.bsz[d] = U.pbsz[d];
-    int64_t bc[3] = {0, 0, 0};
-    chunk_coords(PL, id, bc);
-    const int64_t sz[3] = {sz0, sz1, sz2};
-    // a malformed section (scan not starting at 0, not increasing or past n_pnt) is refused,
-    // not followed: the records [0, n_pnt) are then exactly the chunks' ranges
-    const int64_t j0 = U.scan[i], j1 = U.scan[i + 1];
-    if (j0 > j1 || j1 > n_pnt || (i == 0 && j0 != 0)) {
-        if (threadIdx.x == 0) *bad = 1;
-        return;
+    // the chunk list and the scan lie inside (nc < avail first: no overflow below)
+    const bool whole = nc < (uint64_t)U.avail && U.avail >= hsz + U.A * (int64_t)nc + ((int64_t)nc + 1) * 4;
+    const int64_t n_cnk = (int64_t)nc;
+    const uint32_t np = whole ? load_u32(U.buf + hsz + U.A * n_cnk + n_cnk * 4) : 0u;
+    const int64_t n_pnt = np;
+    const unsigned char *ids = U.buf + hsz, *scan = ids + U.A * n_cnk;
+    const unsigned char *data = scan + align_up((n_cnk + 1) * 4, U.A);
+    const unsigned char *offs = data + align_up(n_pnt * U.psz, U.A);
+    const unsigned char *end = offs + align_up(n_pnt * 2, U.A) + align_up(n_pnt, U.A);
+    const bool go = whole && sizes && end - U.buf <= U.avail && n_pnt <= room;
+    if (first == 0 && lane == 0) {
+        rep[kUpChunks] = (uint32_t)nc;
+        rep[kUpChunks + 1] = (uint32_t)(nc >> 32);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (d >= G.dim) break;
+            rep[kUpStart + d] = (uint32_t)bstart[d];
+            rep[kUpSize + d] = (uint32_t)psize[d];
+        }
+        rep[kUpPoints] = np;
+        rep[kUpState] = (whole ? 1u : 0u) | (go ? 2u : 0u);
     }
-    for (int64_t j = j0 + threadIdx.x; j < j1; j += kWG) {
-        const int off = (uint16_t)U.offs[j];
-        int64_t l[3] = {0, 0, 0}, c[3] = {0, 0, 0};
-        local_coord(G, off, l);
-        bool ok = off < G.csz;
-        for (int d = 0; d < G.dim; ++d) {
-            c[d] = bc[d] * G.edge + l[d] + U.shift[d];
-            ok = ok && c[d] >= 0 && c[d] < sz[d];
+    if (!go) return;
+    int64_t pbsz[3] = {1, 1, 1};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= G.dim) break;
+        pbsz[d] = ((int64_t)psize[d] + G.edge - 1) / G.edge;
+    }
+    const int64_t sz[3] = {sz0, sz1, sz2}, stride = (int64_t)gridDim.x * (kWG / 64);
+    for (int64_t i = first; i < n_cnk; i += stride) {
+        const int64_t id = U.A == 8 ? (int64_t)load_u64(ids + i * 8) : (int64_t)(int32_t)load_u32(ids + i * 4);
+        const int64_t j0 = load_u32(scan + 4 * i), j1 = load_u32(scan + 4 * i + 4);
+        // chunk coordinates in the packing grid (same linearizer, its own chunk counts)
+        int64_t bc[3] = {0, 0, 0};
+        chunk_coords_of(G, pbsz, id, bc);
+        // a malformed section (scan not starting at 0, not increasing or past n_pnt) is
+        // refused, not followed: the records [0, n_pnt) are then exactly the chunks' ranges
+        if (j0 > j1 || j1 > n_pnt || (i == 0 && j0 != 0)) {
+            if (lane == 0) rep[kUpBad] = 1;
+            return;
         }
-        if (!ok) {
-            *bad = 1;
-            rkey[j] = 0;
-            rmask[j] = 0;
-            continue;
-        }
-        int64_t cb[3] = {0, 0, 0}, lo = 0;
-        for (int d = G.dim - 1; d >= 0; --d) {
-            cb[d] = c[d] / G.edge;
-            lo = lo * G.edge + c[d] % G.edge;
-        }
-        rkey[j] = chunk_id(G.L, cb) * G.csz + lo;
-        rmask[j] = SG_EXIST;
-        for (int q = 0; q < P.np; ++q) {
-            unsigned char *dst = (unsigned char *)P.p[q] + (int64_t)j * P.ts[q];
-            if (U.data[q]) copy_scalar(dst, U.data[q] + (int64_t)j * P.ts[q], P.ts[q]);
-            else copy_scalar(dst, (const unsigned char *)&P.bg[q], P.ts[q]);
+        for (int64_t j = j0 + lane; j < j1; j += 64) {
+            const int off = (int)load_u16(offs + 2 * j);
+            int64_t l[3] = {0, 0, 0}, c[3] = {0, 0, 0};
+            local_coord(G, off, l);
+            bool ok = off < G.csz;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                if (d >= G.dim) break;
+                c[d] = bc[d] * G.edge + l[d] + ((int64_t)U.dst_lo[d] - bstart[d]);
+                ok = ok && c[d] >= 0 && c[d] < sz[d];
+            }
+            if (!ok) {
+                rep[kUpBad] = 1;
+                rkey[j] = 0;
+                rmask[j] = 0;
+                continue;
+            }
+            int64_t cb[3] = {0, 0, 0}, lo = 0;
+#pragma unroll
+            for (int d = 2; d >= 0; --d) {
+                if (d >= G.dim) continue;
+                cb[d] = G.sh >= 0 ? c[d] >> G.sh : c[d] / G.edge;
+                lo = lo * G.edge + (c[d] - cb[d] * G.edge);
+            }
+            rkey[j] = chunk_id(G.L, cb) * G.csz + lo;
+            rmask[j] = SG_EXIST;
+            for (int q = 0; q < P.np; ++q) {
+                const int ts = P.ts[q];
+                unsigned char *dst = (unsigned char *)P.p[q] + j * ts;
+                const unsigned char *src = data + n_pnt * U.off[q];
+                if (U.off[q] < 0) copy_aligned(dst, (const unsigned char *)&P.bg[q], ts);
+                else if (((uintptr_t)src & (uintptr_t)(ts - 1)) == 0) copy_aligned(dst, src + j * ts, ts);
+                else copy_scalar(dst, src + j * ts, ts);
+            }
         }
     }
 }
 
 // remove_points (SparseGridGpu_kernels.cuh:1301-1346): existing points inside a queued box
 // get mask 0 (and the background value)
+// one wave per chunk
+template <int V>
 __global__ __launch_bounds__(kWG) void remove_boxes_kernel(const int64_t *__restrict__ keys, int64_t n,
-                                                          uint8_t *__restrict__ mask, Geom G, Boxes B, PropSet P)
+                                                          uint8_t *mask, Geom G, Boxes B, PropSet P)
 {
-    const int64_t c = blockIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int64_t c = (int64_t)blockIdx.x * (kWG / 64) + w;
     if (c >= n) return;
     int64_t org[3] = {0, 0, 0};
     chunk_origin(G, keys[c], org);
-    bool any = false;
-    for (int k = 0; k < B.n; ++k) any = any || chunk_meets_box(G, org, B.lo + k * G.dim, B.hi + k * G.dim);
-    if (!any) return;
-    for (int o = threadIdx.x; o < G.csz; o += kWG) {
-        if (!(mask[c * G.csz + o] & SG_EXIST)) continue;
-        int64_t l[3] = {0, 0, 0}, p[3];
-        local_coord(G, o, l);
-        for (int d = 0; d < G.dim; ++d) p[d] = org[d] + l[d];
-        for (int k = 0; k < B.n; ++k)
-            if (point_in_box(G, p, B.lo + k * G.dim, B.hi + k * G.dim)) {
-                clear_slot(P, mask, c * G.csz + o);
-                break;
-            }
+    const uint32_t met = boxes_met(G, B, org, lane);
+    if (met == 0) return;
+    uint32_t m[4];
+    const uint32_t e = lane_masks<V>(mask, c, G, lane, m);
+    uint32_t in = 0;
+    for (uint32_t left = met; left; left &= left - 1) {
+        const int k = __builtin_ctz(left);
+        in |= lane_box_bits<V>(G, org, B.lo + k * G.dim, B.hi + k * G.dim, lane);
     }
+    const int64_t s0 = c * G.csz + lane * lane_slots(G, V);
+    for (uint32_t b = e & in; b; b &= b - 1) clear_slot(P, mask, s0 + __builtin_ctz(b));
 }
 
 __device__ inline int64_t lower_bound_keys(const int64_t *a, int64_t n, int64_t x)
@@ -320,7 +577,12 @@ Geom geom_of(const sg_grid *g)
     G.dim = g->dim;
     G.edge = g->edge;
     G.csz = g->csz;
+    G.sh = -1;
+    for (int b = 1; b < 11; ++b)
+        if ((1 << b) == g->edge) G.sh = b;
     G.L = chunk_lin(g);
+    // chunk counts below 2^31 (sg_create) give row-major ids below 2^31
+    G.ids32 = !G.L.zorder;
     return G;
 }
 
@@ -337,14 +599,13 @@ PropSet grid_props(sg_grid *g)
     return P;
 }
 
-int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
-
 int check_pack_args(const sg_grid *g, int nbox, const int32_t *lo, const int32_t *hi, int nprop,
                     const int32_t *props, int A)
 {
     if (nbox < 0 || nprop < 0) return fail(SG_E_ARG, "negative count");
     if (nbox > 0 && (!lo || !hi)) return fail(SG_E_ARG, "null boxes");
     if (nprop > 0 && !props) return fail(SG_E_ARG, "null property list");
+    if (nprop > kMaxProps) return fail(SG_E_ARG, "more properties than a grid can have");
     if (A != 4 && A != 8) return fail(SG_E_ARG, "index_bytes must be 4 or 8");
     for (int q = 0; q < nprop; ++q)
         if (props[q] < 0 || props[q] >= g->np) return fail(SG_E_ARG, "bad property");
@@ -365,140 +626,131 @@ int64_t section_bytes(const sg_grid *g, int64_t n_cnk, int64_t n_pnt, int64_t ps
            align_up(n_pnt * 2, A) + align_up(n_pnt, A);
 }
 
-// per box: point counts + their scan and the chunk flags + their scan, totals to the host
+// boxes [k0, k0 + kBoxes) of a list as kernel arguments
+Boxes box_args(int dim, int nbox, const int32_t *lo, const int32_t *hi, int k0)
+{
+    Boxes B;
+    B.n = std::min(kBoxes, nbox - k0);
+    memcpy(B.lo, lo + (size_t)k0 * dim, (size_t)B.n * dim * 4);
+    memcpy(B.hi, hi + (size_t)k0 * dim, (size_t)B.n * dim * 4);
+    return B;
+}
+
+// f(std::integral_constant<int, V>) for the lane runs of the grid's chunks
+template <typename F> void with_lane_run(const sg_grid *g, F &&f)
+{
+    switch (g->csz) {
+    case 64: f(std::integral_constant<int, 1>()); break;
+    case 128: f(std::integral_constant<int, 2>()); break;
+    case 256: f(std::integral_constant<int, 4>()); break;
+    case 512: f(std::integral_constant<int, 8>()); break;
+    case 1024: f(std::integral_constant<int, 16>()); break;
+    default: f(std::integral_constant<int, 0>()); break;
+    }
+}
+
+unsigned chunk_waves(int64_t n) { return (unsigned)((n + kWG / 64 - 1) / (kWG / 64)); }
+
+// Per box (rows of stride = chunks + 1 entries) the scan of the point counts, then (from
+// entry per = nbox * stride) of the non-empty flags, in one exclusive scan over all rows
+// (in place), and the boxes' totals.
 struct PackPlan {
-    int64_t stride = 0;
-    uint32_t *cnt = nullptr, *flag = nullptr, *pscan = nullptr, *cscan = nullptr;
-    const int32_t *d_lo = nullptr, *d_hi = nullptr;  // device copy of the boxes, [nbox][dim]
+    int64_t stride = 0, per = 0;
+    uint32_t *scan = nullptr;
     std::vector<int64_t> n_cnk, n_pnt;
 };
+
+// the counts of every box in pl.scan and, after the caller's scan of them, their totals in
+// d_tot [2 * nbox] (queued on the grid's stream)
+int pack_counts(sg_grid *g, int nbox, const int32_t *lo, const int32_t *hi, int64_t stride, uint32_t *rows)
+{
+    const int64_t n = g->nchunks, per = nbox * stride;
+    for (int k0 = 0; k0 < nbox; k0 += kBoxes) {
+        with_lane_run(g, [&](auto v) {
+            hipLaunchKernelGGL(pack_count_kernel<decltype(v)::value>, dim3(chunk_waves(n + 1)), dim3(kWG), 0, g->stream,
+                               g->d_keys, n, g->d_mask, geom_of(g), box_args(g->dim, nbox, lo, hi, k0),
+                               rows + k0 * stride, rows + per + k0 * stride, stride);
+        });
+        SG_HIP(hipGetLastError());
+    }
+    return SG_OK;
+}
 
 int plan_pack(sg_grid *g, int nbox, const int32_t *lo, const int32_t *hi, PackPlan &pl)
 {
     const int64_t n = g->nchunks;
     pl.stride = n + 1;
+    pl.per = nbox * pl.stride;
     pl.n_cnk.assign(nbox, 0);
     pl.n_pnt.assign(nbox, 0);
     if (nbox == 0) return SG_OK;
     int rc;
-    DevBuf &b_boxes = g->scratch[0], &b_cnt = g->scratch[1];
-    const size_t bb = (size_t)nbox * g->dim * 4;
-    if ((rc = ensure(g->pool, b_boxes, 2 * bb + 64))) return rc;
-    const size_t per = (size_t)nbox * pl.stride;
-    if ((rc = ensure(g->pool, b_cnt, per * 4 * sizeof(uint32_t) + 64))) return rc;
-    int32_t *d_lo = (int32_t *)b_boxes.p, *d_hi = d_lo + (size_t)nbox * g->dim;
-    SG_HIP(hipMemcpyAsync(d_lo, lo, bb, hipMemcpyHostToDevice, g->stream));
-    SG_HIP(hipMemcpyAsync(d_hi, hi, bb, hipMemcpyHostToDevice, g->stream));
-    pl.d_lo = d_lo;
-    pl.d_hi = d_hi;
-    pl.cnt = (uint32_t *)b_cnt.p;
-    pl.flag = pl.cnt + per;
-    pl.pscan = pl.flag + per;
-    pl.cscan = pl.pscan + per;
-    // the trailing entry of every box row is 0 (its scan is the row total)
-    SG_HIP(hipMemsetAsync(pl.cnt, 0, per * 2 * sizeof(uint32_t), g->stream));
-    if (n > 0) {
-        Boxes B{nbox, d_lo, d_hi};
-        hipLaunchKernelGGL(pack_count_kernel, dim3((unsigned)n), dim3(kWG), 0, g->stream, g->d_keys, n, g->d_mask,
-                           geom_of(g), B, pl.cnt, pl.flag, pl.stride);
-        SG_HIP(hipGetLastError());
-    }
+    DevBuf &b_cnt = g->scratch[1];
+    if ((rc = ensure(g->pool, b_cnt, (size_t)pl.per * 2 * sizeof(uint32_t) + (size_t)nbox * 2 * sizeof(uint32_t) + 64)))
+        return rc;
+    pl.scan = (uint32_t *)b_cnt.p;
+    if ((rc = pack_counts(g, nbox, lo, hi, pl.stride, pl.scan))) return rc;
+    if ((rc = exclusive_scan_u32(g, pl.scan, pl.scan, 2 * pl.per, nullptr))) return rc;
+    // totals: straight to the pinned words when they fit
+    uint32_t *hw = host_words(g);
+    if (!hw) return fail(SG_E_OOM, "pinned host allocation failed");
+    const bool pinned = nbox <= 8;
+    uint32_t *tot = pinned ? hw : pl.scan + 2 * pl.per;
+    hipLaunchKernelGGL(pack_totals_kernel, dim3(grid_1d(nbox, 64)), dim3(64), 0, g->stream, pl.scan, pl.per, pl.stride,
+                       nbox, tot);
+    SG_HIP(hipGetLastError());
+    std::vector<uint32_t> h(pinned ? 0 : 2 * (size_t)nbox);
+    if (!pinned)
+        SG_HIP(hipMemcpyAsync(h.data(), tot, (size_t)nbox * 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, g->stream));
+    SG_HIP(hipStreamSynchronize(g->stream));
+    const uint32_t *t = pinned ? hw : h.data();
     for (int k = 0; k < nbox; ++k) {
-        uint32_t tp = 0, tc = 0;
-        if ((rc = exclusive_scan_u32(g, pl.cnt + k * pl.stride, pl.pscan + k * pl.stride, pl.stride, &tp))) return rc;
-        if ((rc = exclusive_scan_u32(g, pl.flag + k * pl.stride, pl.cscan + k * pl.stride, pl.stride, &tc))) return rc;
-        pl.n_pnt[k] = tp;
-        pl.n_cnk[k] = tc;
+        pl.n_pnt[k] = t[2 * k];
+        pl.n_cnk[k] = t[2 * k + 1];
     }
     return SG_OK;
 }
 
-// header of one packed section: chunk count, box start and grid size, and the scan's last
-// entry (n_pnt); passed by value to the kernel that writes them, so nothing is staged on
-// the host
-struct SectionHead {
-    uint64_t nc;
-    uint32_t np;
-    int dim;
-    int32_t lo[3], sz[3];
-};
-
-__global__ void pack_header_kernel(unsigned char *s0, uint32_t *scan_last, SectionHead h)
-{
-    if (threadIdx.x != 0) return;
-    // sections start at multiples of 4 bytes only: byte copies
-    copy_scalar(s0, (const unsigned char *)&h.nc, 8);
-    for (int d = 0; d < h.dim; ++d) {
-        copy_scalar(s0 + 8 + 4 * d, (const unsigned char *)&h.lo[d], 4);
-        copy_scalar(s0 + 8 + 4 * (h.dim + d), (const unsigned char *)&h.sz[d], 4);
-    }
-    copy_scalar((unsigned char *)scan_last, (const unsigned char *)&h.np, 4);
-}
-
-// write the packed sections of the boxes to the device buffer buf (cap bytes) from a
-// plan: per box k, rows k * stride of cnt / pscan / cscan and corners d_lo / d_hi + k * dim
-// (device), lo + k * dim (host); queued on the grid's stream, allocates nothing
-int pack_sections(sg_grid *g, int nbox, const int32_t *lo, int nprop, const int32_t *props, int A,
-                  unsigned char *buf, int64_t cap, int64_t stride, const uint32_t *cnt, const uint32_t *pscan,
-                  const uint32_t *cscan, const int32_t *d_lo, const int32_t *d_hi, const int64_t *n_cnk,
+// write the packed sections of the boxes to the device buffer buf (cap bytes) from the
+// scanned rows of a plan; queued on the grid's stream, allocates nothing
+int pack_sections(sg_grid *g, int nbox, const int32_t *lo, const int32_t *hi, int nprop, const int32_t *props, int A,
+                  unsigned char *buf, int64_t cap, int64_t stride, const uint32_t *scan, const int64_t *n_cnk,
                   const int64_t *n_pnt)
 {
-    const int64_t psz = point_bytes(g, nprop, props);
+    const int64_t psz = point_bytes(g, nprop, props), n = g->nchunks, per = nbox * stride;
+    PackProps P;
+    P.n = nprop;
+    for (int q = 0; q < nprop; ++q) {
+        P.ts[q] = g->ts[props[q]];
+        P.src[q] = (const unsigned char *)g->d_prop[props[q]];
+    }
     int64_t at = 0;
-    const int64_t n = g->nchunks;
-    const int hsz = 8 + 2 * g->dim * 4;
-    for (int k = 0; k < nbox; ++k) {
-        const int64_t nc = n_cnk[k], np = n_pnt[k];
-        const int64_t sb = section_bytes(g, nc, np, psz, A);
-        if (at + sb > cap) return fail(SG_E_RANGE, "pack buffer too small");
-        unsigned char *s0 = buf + at;
-        SG_HIP(hipMemsetAsync(s0, 0, (size_t)sb, g->stream));
-        int64_t q = hsz;
-        PackOut O;
-        O.A = A;
-        O.ids = s0 + q;
-        q += A * nc;
-        O.scan = (uint32_t *)(s0 + q);
-        q += align_up((nc + 1) * 4, A);
-        SectionHead h{};
-        h.nc = (uint64_t)nc;
-        h.np = (uint32_t)np;
-        h.dim = g->dim;
-        for (int d = 0; d < g->dim; ++d) {
-            h.lo[d] = lo[k * g->dim + d];
-            h.sz[d] = (int32_t)g->sz[d];
+    for (int k0 = 0; k0 < nbox; k0 += kBoxes) {
+        const Boxes B = box_args(g->dim, nbox, lo, hi, k0);
+        PackSections X;
+        for (int k = 0; k < B.n; ++k) {
+            X.at[k] = at;
+            X.nc[k] = (uint32_t)n_cnk[k0 + k];
+            X.np[k] = (uint32_t)n_pnt[k0 + k];
+            at += section_bytes(g, n_cnk[k0 + k], n_pnt[k0 + k], psz, A);
+            if (at > cap) return fail(SG_E_RANGE, "pack buffer too small");
         }
-        hipLaunchKernelGGL(pack_header_kernel, dim3(1), dim3(64), 0, g->stream, s0, O.scan + nc, h);
+        with_lane_run(g, [&](auto v) {
+            hipLaunchKernelGGL(pack_write_kernel<decltype(v)::value>, dim3(chunk_waves(n + B.n)), dim3(kWG), 0, g->stream,
+                               g->d_keys, n, g->d_mask, geom_of(g), B, scan + k0 * stride, scan + per + k0 * stride,
+                               stride, P, (int)psz, A, X, buf, (int32_t)g->sz[0], (int32_t)g->sz[1], (int32_t)g->sz[2]);
+        });
         SG_HIP(hipGetLastError());
-        O.nprop = nprop;
-        int64_t dq = q;
-        for (int pi = 0; pi < nprop; ++pi) {
-            O.data[pi] = s0 + dq;
-            O.ts[pi] = g->ts[props[pi]];
-            O.src[pi] = (const unsigned char *)g->d_prop[props[pi]];
-            dq += np * g->ts[props[pi]];
-        }
-        q += align_up(np * psz, A);
-        O.offs = (int16_t *)(s0 + q);
-        q += align_up(np * 2, A);
-        O.masks = s0 + q;
-        if (n > 0 && np > 0) {
-            hipLaunchKernelGGL(pack_write_kernel, dim3((unsigned)n), dim3(kWG), 0, g->stream, g->d_keys, n, g->d_mask,
-                               geom_of(g), d_lo + (size_t)k * g->dim, d_hi + (size_t)k * g->dim, pscan + k * stride,
-                               cscan + k * stride, cnt + k * stride, O);
-            SG_HIP(hipGetLastError());
-        }
-        at += sb;
     }
     return SG_OK;
 }
 
 // the packed sections from a plan, complete when the call returns
-int pack_into_device(sg_grid *g, int nbox, const int32_t *lo, int nprop, const int32_t *props, int A,
+int pack_into_device(sg_grid *g, int nbox, const int32_t *lo, const int32_t *hi, int nprop, const int32_t *props, int A,
                      unsigned char *buf, int64_t cap, const PackPlan &pl)
 {
-    int rc = pack_sections(g, nbox, lo, nprop, props, A, buf, cap, pl.stride, pl.cnt, pl.pscan, pl.cscan, pl.d_lo,
-                           pl.d_hi, pl.n_cnk.data(), pl.n_pnt.data());
+    int rc = pack_sections(g, nbox, lo, hi, nprop, props, A, buf, cap, pl.stride, pl.scan, pl.n_cnk.data(),
+                           pl.n_pnt.data());
     if (rc) return rc;
     SG_HIP(hipStreamSynchronize(g->stream));
     return SG_OK;
@@ -534,8 +786,9 @@ int noalloc_scratch(void **out)
 
 constexpr size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// scratch bytes of a pack of nbox boxes over n chunks: the box corners, the four count /
-// scan rows of every box, the per-box totals and the scan workspace
+// scratch bytes a pack of nbox boxes over n chunks may use (the call's documented limit:
+// box corners, four rows of every box, per-box totals and a scan workspace); two rows of
+// every box, the totals and the workspace of one scan over the rows are in use
 size_t noalloc_pack_bytes(int nbox, int dim, int64_t n)
 {
     const size_t stride = (size_t)n + 1;
@@ -578,12 +831,12 @@ int sg_pack(sg_grid *g, int nbox, const int32_t *lo, const int32_t *hi, int npro
     for (int k = 0; k < nbox; ++k) tot += section_bytes(g, pl.n_cnk[k], pl.n_pnt[k], psz, index_bytes);
     if (tot > cap) return fail(SG_E_RANGE, "pack buffer too small");
     if (mem == SG_MEM_DEVICE) {
-        rc = pack_into_device(g, nbox, lo, nprop, props, index_bytes, (unsigned char *)buf, cap, pl);
+        rc = pack_into_device(g, nbox, lo, hi, nprop, props, index_bytes, (unsigned char *)buf, cap, pl);
         return rc;
     }
     DevBuf &st = g->scratch[2];
     if ((rc = ensure(g->pool, st, (size_t)tot + 64))) return rc;
-    if ((rc = pack_into_device(g, nbox, lo, nprop, props, index_bytes, (unsigned char *)st.p, tot, pl)))
+    if ((rc = pack_into_device(g, nbox, lo, hi, nprop, props, index_bytes, (unsigned char *)st.p, tot, pl)))
         return rc;
     SG_HIP(hipMemcpyAsync(buf, st.p, (size_t)tot, hipMemcpyDeviceToHost, g->stream));
     SG_HIP(hipStreamSynchronize(g->stream));
@@ -609,37 +862,20 @@ int sg_pack_noalloc(sg_grid *g, int nbox, const int32_t *lo, const int32_t *hi, 
     if (nbox == 0) return SG_OK;
     void *base = nullptr;
     if ((rc = noalloc_scratch(&base))) return rc;
-    // carve the scratch: corners | cnt, flag, pscan, cscan rows | totals | scan workspace
-    unsigned char *p = (unsigned char *)base;
-    const size_t bb = (size_t)nbox * g->dim * 4, per = (size_t)nbox * stride;
-    int32_t *d_lo = (int32_t *)p, *d_hi = d_lo + (size_t)nbox * g->dim;
-    p += round256(2 * bb);
-    uint32_t *cnt = (uint32_t *)p, *flag = cnt + per, *pscan = flag + per, *cscan = pscan + per;
-    p += round256(4 * per * 4);
-    uint32_t *d_tot = (uint32_t *)p;
-    p += round256((size_t)2 * nbox * 4);
-    uint32_t *ws = (uint32_t *)p;
-    const size_t ws_words = scan_ws_words(stride);
-
-    SG_HIP(hipMemcpyAsync(d_lo, lo, bb, hipMemcpyHostToDevice, g->stream));
-    SG_HIP(hipMemcpyAsync(d_hi, hi, bb, hipMemcpyHostToDevice, g->stream));
-    // the scratch keeps the previous call's contents: the rows' trailing entries (which the
-    // count pass does not write) must read 0
-    SG_HIP(hipMemsetAsync(cnt, 0, per * 2 * sizeof(uint32_t), g->stream));
-    if (n > 0) {
-        Boxes B{nbox, d_lo, d_hi};
-        hipLaunchKernelGGL(pack_count_kernel, dim3((unsigned)n), dim3(kWG), 0, g->stream, g->d_keys, n, g->d_mask,
-                           geom_of(g), B, cnt, flag, stride);
-        SG_HIP(hipGetLastError());
-    }
-    for (int k = 0; k < nbox; ++k) {
-        if ((rc = exclusive_scan_u32_ws(g->stream, cnt + k * stride, pscan + k * stride, stride, d_tot + 2 * k, ws,
-                                        ws_words)))
-            return rc;
-        if ((rc = exclusive_scan_u32_ws(g->stream, flag + k * stride, cscan + k * stride, stride, d_tot + 2 * k + 1,
-                                        ws, ws_words)))
-            return rc;
-    }
+    // carve the scratch: count and flag rows (scanned in place) | totals | scan workspace
+    const int64_t per = nbox * stride;
+    const size_t rows_bytes = round256((size_t)per * 2 * 4), tot_bytes = round256((size_t)2 * nbox * 4);
+    const size_t ws_words = scan_ws_words(2 * per);
+    if (rows_bytes + tot_bytes + ws_words * 4 > (size_t)SG_PACK_NOALLOC_SCRATCH_BYTES)
+        return fail(SG_E_RANGE, "sg_pack_noalloc: scratch too small");
+    uint32_t *scan = (uint32_t *)base;
+    uint32_t *d_tot = (uint32_t *)((unsigned char *)base + rows_bytes);
+    uint32_t *ws = (uint32_t *)((unsigned char *)base + rows_bytes + tot_bytes);
+    if ((rc = pack_counts(g, nbox, lo, hi, stride, scan))) return rc;
+    if ((rc = exclusive_scan_u32_ws(g->stream, scan, scan, 2 * per, nullptr, ws, ws_words))) return rc;
+    hipLaunchKernelGGL(pack_totals_kernel, dim3(grid_1d(nbox, 64)), dim3(64), 0, g->stream, scan, per, stride, nbox,
+                       d_tot);
+    SG_HIP(hipGetLastError());
     uint32_t h_tot[2 * SG_PACK_NOALLOC_MAX_BOXES];
     SG_HIP(hipMemcpyAsync(h_tot, d_tot, (size_t)2 * nbox * 4, hipMemcpyDeviceToHost, g->stream));
     SG_HIP(hipStreamSynchronize(g->stream));
@@ -652,8 +888,8 @@ int sg_pack_noalloc(sg_grid *g, int nbox, const int32_t *lo, const int32_t *hi, 
         tot += section_bytes(g, n_cnk[k], n_pnt[k], psz, index_bytes);
     }
     if (tot > cap) return fail(SG_E_RANGE, "pack buffer too small: " + std::to_string(tot) + " bytes needed");
-    if ((rc = pack_sections(g, nbox, lo, nprop, props, index_bytes, (unsigned char *)dev_buf, cap, stride, cnt, pscan,
-                            cscan, d_lo, d_hi, n_cnk, n_pnt)))
+    if ((rc = pack_sections(g, nbox, lo, hi, nprop, props, index_bytes, (unsigned char *)dev_buf, cap, stride, scan,
+                            n_cnk, n_pnt)))
         return rc;
     SG_HIP(hipStreamSynchronize(g->stream));
     *written = tot;
@@ -669,79 +905,84 @@ int sg_unpack(sg_grid *g, const void *buf, int64_t avail, int mem, const int32_t
     const int A = index_bytes;
     const int64_t hsz = 8 + 2 * g->dim * 4;
     if (avail < hsz) return fail(SG_E_RANGE, "packed section truncated");
-    const hipMemcpyKind kind = (mem == SG_MEM_DEVICE) ? hipMemcpyDeviceToHost : hipMemcpyHostToHost;
-    std::vector<unsigned char> hdr(hsz);
-    SG_HIP(hipMemcpyAsync(hdr.data(), buf, hsz, kind, g->stream));
-    SG_HIP(hipStreamSynchronize(g->stream));
-    uint64_t ncu;
-    memcpy(&ncu, hdr.data(), 8);
-    const int64_t nc = (int64_t)ncu;
-    int32_t bstart[3] = {0, 0, 0}, psize[3] = {1, 1, 1};
-    for (int d = 0; d < g->dim; ++d) {
-        memcpy(&bstart[d], hdr.data() + 8 + 4 * d, 4);
-        memcpy(&psize[d], hdr.data() + 8 + 4 * (g->dim + d), 4);
-        if (psize[d] <= 0) return fail(SG_E_RANGE, "bad packed grid size");
-    }
-    if (nc < 0 || avail < hsz + A * nc + (nc + 1) * 4) return fail(SG_E_RANGE, "packed section truncated");
-    uint32_t np32 = 0;
-    SG_HIP(hipMemcpyAsync(&np32, (const unsigned char *)buf + hsz + A * nc + nc * 4, 4, kind, g->stream));
-    SG_HIP(hipStreamSynchronize(g->stream));
-    const int64_t np = np32;
+    uint32_t *hw = host_words(g);
+    if (!hw) return fail(SG_E_OOM, "pinned host allocation failed");
     const int64_t psz = point_bytes(g, nprop, props);
+    UnpackIn U;
+    U.A = A;
+    U.psz = (int)psz;
+    for (int p = 0; p < kMaxProps; ++p) U.off[p] = -1;
+    for (int pi = 0, o = 0; pi < nprop; ++pi) {
+        U.off[props[pi]] = o;
+        o += g->ts[props[pi]];
+    }
+    for (int d = 0; d < 3; ++d) U.dst_lo[d] = d < g->dim ? dst_lo[d] : 0;
+    // records go to the insert buffer at `at` (room for `room` of them); values of the
+    // properties not unpacked are the background (the finalize keeps the old values there)
+    int64_t at = g->ins_n, room = g->ins_cap - g->ins_n;
+    if (g->cins_n > 0 || g->pins_n > 0) room = 0;  // converted to point records first, below
+    auto launch = [&](const unsigned char *s0, int64_t bytes) -> int {
+        PropSet R;
+        R.np = g->np;
+        for (int p = 0; p < g->np; ++p) {
+            R.p[p] = (unsigned char *)g->d_ins_val[p] + at * g->ts[p];
+            R.ts[p] = g->ts[p];
+            R.bg[p] = 0;
+            memcpy(&R.bg[p], g->bg[p], g->ts[p]);
+        }
+        U.buf = s0;
+        U.avail = bytes;
+        // the report: the flag is written only by a thread that meets a bad record
+        hw[kUpState] = hw[kUpBad] = 0;
+        const unsigned grid = std::min<unsigned>(1024, chunk_waves(std::max<int64_t>(1, bytes / (A + 4))));
+        hipLaunchKernelGGL(unpack_section_kernel, dim3(grid), dim3(kWG), 0, g->stream, U, geom_of(g), g->sz[0], g->sz[1],
+                           g->sz[2], R, g->d_ins_key + at, g->d_ins_mask + at, room, hw);
+        SG_HIP(hipGetLastError());
+        SG_HIP(hipStreamSynchronize(g->stream));
+        return SG_OK;
+    };
+    const unsigned char *s0 = (const unsigned char *)buf;
+    int64_t nc = 0, sec = avail;
+    uint32_t np32 = 0;
+    bool whole = false, sizes = true, done = false;
+    if (mem == SG_MEM_DEVICE) {
+        if ((rc = launch(s0, avail))) return rc;
+        nc = (int64_t)((uint64_t)hw[kUpChunks] | ((uint64_t)hw[kUpChunks + 1] << 32));
+        for (int d = 0; d < g->dim; ++d) sizes = sizes && (int32_t)hw[kUpSize + d] > 0;
+        np32 = hw[kUpPoints];
+        whole = (hw[kUpState] & 1) != 0;
+        done = (hw[kUpState] & 2) != 0;
+    } else {
+        memcpy(&nc, s0, 8);
+        for (int d = 0; d < g->dim; ++d) {
+            int32_t v;
+            memcpy(&v, s0 + 8 + 4 * (g->dim + d), 4);
+            sizes = sizes && v > 0;
+        }
+        whole = nc >= 0 && nc < avail && avail >= hsz + A * nc + (nc + 1) * 4;
+        if (whole) memcpy(&np32, s0 + hsz + A * nc + nc * 4, 4);
+    }
+    if (!sizes) return fail(SG_E_RANGE, "bad packed grid size");
+    if (!whole) return fail(SG_E_RANGE, "packed section truncated");
+    const int64_t np = np32;
     const int64_t sb = section_bytes(g, nc, np, psz, A);
     if (avail < sb) return fail(SG_E_RANGE, "packed section truncated");
     if (nc == 0 && np != 0) return fail(SG_E_RANGE, "malformed packed section: points without chunks");
     *consumed = sb;
     if (np == 0) return SG_OK;
-    // the section on the device
-    const unsigned char *s0 = (const unsigned char *)buf;
-    if (mem != SG_MEM_DEVICE) {
-        DevBuf &st = g->scratch[2];
-        if ((rc = ensure(g->pool, st, (size_t)sb + 64))) return rc;
-        SG_HIP(hipMemcpyAsync(st.p, buf, (size_t)sb, hipMemcpyHostToDevice, g->stream));
-        s0 = (const unsigned char *)st.p;
+    if (!done) {
+        if (mem != SG_MEM_DEVICE) {
+            DevBuf &st = g->scratch[2];
+            if ((rc = ensure(g->pool, st, (size_t)sb + 64))) return rc;
+            SG_HIP(hipMemcpyAsync(st.p, buf, (size_t)sb, hipMemcpyHostToDevice, g->stream));
+            s0 = (const unsigned char *)st.p;
+            sec = sb;
+        }
+        if ((rc = reserve_point_records(g, np, &at))) return rc;
+        room = np;
+        if ((rc = launch(s0, sec))) return rc;
     }
-    int64_t at = 0;
-    if ((rc = reserve_point_records(g, np, &at))) return rc;
-    UnpackIn U;
-    int64_t q = hsz;
-    U.A = A;
-    U.ids = s0 + q;
-    q += A * nc;
-    U.scan = (const uint32_t *)(s0 + q);
-    q += align_up((nc + 1) * 4, A);
-    for (int p = 0; p < kMaxProps; ++p) U.data[p] = nullptr;
-    int64_t dq = q;
-    for (int pi = 0; pi < nprop; ++pi) {
-        U.data[props[pi]] = s0 + dq;
-        dq += np * g->ts[props[pi]];
-    }
-    q += align_up(np * psz, A);
-    U.offs = (const int16_t *)(s0 + q);
-    for (int d = 0; d < 3; ++d) {
-        U.pbsz[d] = (d < g->dim) ? (psize[d] + g->edge - 1) / g->edge : 1;
-        U.shift[d] = (d < g->dim) ? dst_lo[d] - bstart[d] : 0;
-    }
-    // records go to the insert buffer at `at`; values of the properties not unpacked are
-    // the background (the finalize keeps the old values there)
-    PropSet R;
-    R.np = g->np;
-    for (int p = 0; p < g->np; ++p) {
-        R.p[p] = (unsigned char *)g->d_ins_val[p] + at * g->ts[p];
-        R.ts[p] = g->ts[p];
-        R.bg[p] = 0;
-        memcpy(&R.bg[p], g->bg[p], g->ts[p]);
-    }
-    if ((rc = ensure(g->pool, g->scratch[6], 64))) return rc;
-    int *bad = (int *)g->scratch[6].p;
-    SG_HIP(hipMemsetAsync(bad, 0, sizeof(int), g->stream));
-    hipLaunchKernelGGL(unpack_records_kernel, dim3((unsigned)std::max<int64_t>(nc, 1)), dim3(kWG), 0, g->stream, U,
-                       nc, np, geom_of(g), g->sz[0], g->sz[1], g->sz[2], R, g->d_ins_key + at, g->d_ins_mask + at, bad);
-    SG_HIP(hipGetLastError());
-    int hbad = 0;
-    SG_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-    SG_HIP(hipStreamSynchronize(g->stream));
-    if (hbad) return fail(SG_E_RANGE, "unpacked point outside the grid or malformed packed section");
+    if (hw[kUpBad]) return fail(SG_E_RANGE, "unpacked point outside the grid or malformed packed section");
     g->ins_n = at + np;
     return SG_OK;
 }
@@ -786,20 +1027,17 @@ int remove_queued_boxes(sg_grid *g)
 {
     const int nb = (int)(g->rem_lo.size() / std::max(1, g->dim));
     if (nb > 0 && g->nchunks > 0) {
-        const size_t bb = (size_t)nb * g->dim * 4;
-        int rc = ensure(g->pool, g->scratch[0], 2 * bb + 64);
-        if (rc) return rc;
-        int32_t *d_lo = (int32_t *)g->scratch[0].p, *d_hi = d_lo + (size_t)nb * g->dim;
-        SG_HIP(hipMemcpyAsync(d_lo, g->rem_lo.data(), bb, hipMemcpyHostToDevice, g->stream));
-        SG_HIP(hipMemcpyAsync(d_hi, g->rem_hi.data(), bb, hipMemcpyHostToDevice, g->stream));
-        Boxes B{nb, d_lo, d_hi};
         g->occ_tab_valid = false;
         g->ebits_valid = false;
-        hipLaunchKernelGGL(remove_boxes_kernel, dim3((unsigned)g->nchunks), dim3(kWG), 0, g->stream, g->d_keys,
-                           g->nchunks, g->d_mask, geom_of(g), B, grid_props(g));
-        SG_HIP(hipGetLastError());
+        for (int k0 = 0; k0 < nb; k0 += kBoxes) {
+            with_lane_run(g, [&](auto v) {
+                hipLaunchKernelGGL(remove_boxes_kernel<decltype(v)::value>, dim3(chunk_waves(g->nchunks)), dim3(kWG), 0,
+                                   g->stream, g->d_keys, g->nchunks, g->d_mask, geom_of(g),
+                                   box_args(g->dim, nb, g->rem_lo.data(), g->rem_hi.data(), k0), grid_props(g));
+            });
+            SG_HIP(hipGetLastError());
+        }
         g->ep_valid = false;
-        SG_HIP(hipStreamSynchronize(g->stream));  // the box vectors are cleared next
     }
     g->rem_lo.clear();
     g->rem_hi.clear();

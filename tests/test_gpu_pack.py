@@ -147,3 +147,74 @@ def test_unpack_outside_grid_fails(G):
         g.unpack(buf, (30, 30, 30), [0])  # the point would land at 32
     assert g.pending_inserts() == 0
     g.close()
+
+
+@pytest.mark.parametrize("nbox,dim,edge,lin,index_bytes", [(1, 3, 8, "smb", 8), (8, 3, 8, "smb", 4), (9, 3, 5, "smb", 8),
+                                                           (32, 2, 16, "smb", 8), (33, 3, 8, "zmb", 4), (70, 2, 6, "smb", 8)])
+def test_many_boxes(G, oracle, nbox, dim, edge, lin, index_bytes):
+    """Counts of boxes about what one launch and the pinned words take, chunk edges that are
+    no power of two, Morton ids, value arrays at every alignment, a device buffer at an odd
+    address: the oracle's bytes, and after unpacking and removing them its grid."""
+    import torch
+    rng = np.random.default_rng(nbox)
+    size = [int(rng.integers(5 * edge, 9 * edge)) for _ in range(dim)]
+    dtypes = [np.uint8, np.float64, np.uint16, np.float32]
+    pts = np.stack([rng.integers(0, s, 4000) for s in size], 1).astype(np.int32)
+    vals = [rng.integers(0, 200, 4000).astype(t) for t in dtypes]
+    boxes = []
+    for k in range(nbox):
+        lo = [int(rng.integers(0, s - 1)) for s in size]
+        boxes.append((lo, [int(rng.integers(l, min(s, l + 3 * edge))) for l, s in zip(lo, size)]))
+    boxes[-1] = ([0] * dim, [s - 1 for s in size])
+    grids = []
+    for cls in (G, oracle.SparseGridCpu):
+        pair = []
+        for part in (slice(None), slice(0, 1500)):
+            g = cls(dim, size, dtypes, block_edge=edge, linearizer=lin)
+            g.insert_coords(pts[part], [v[part] for v in vals])
+            g.flush(["smax"] * 4)
+            pair.append(g)
+        grids.append(pair)
+    (a, da), (b, db) = grids
+    want = b.pack(boxes, [0, 1, 2, 3], index_bytes)
+    assert a.pack_size(boxes, [0, 1, 2, 3], index_bytes) == len(want)
+    np.testing.assert_array_equal(a.pack(boxes, [0, 1, 2, 3], index_bytes), want)
+    dev = torch.full((len(want) + 9,), 0xAB, dtype=torch.uint8, device="cuda")
+    odd = dev[1:]
+    assert a.pack(boxes, [0, 1, 2, 3], index_bytes, out=odd) == len(want)
+    np.testing.assert_array_equal(odd.cpu().numpy()[:len(want)], want)
+    assert (dev.cpu().numpy()[[0] + list(range(len(want) + 1, len(want) + 9))] == 0xAB).all()
+    for g in (da, db):
+        for lo, hi in boxes[:-1]:
+            g.remove_box(lo, hi)
+        at = 0
+        for lo, _ in boxes[:-1][:12]:
+            at += g.unpack(odd if g is da else want, lo, [0, 1, 2, 3], index_bytes, offset=at)
+        g.remove_add_unpack_finalize([0, 1, 2, 3])
+    S.assert_same_state(da, db)
+
+
+def test_unpack_refuses_malformed_sections(G):
+    """Chunk counts and scans that lead outside the section are refused, host and device."""
+    import torch
+    from openfpm_data_amd._capi import SgError
+    g = G(3, (32, 32, 32), [np.float32], block_edge=8)
+    g.insert_coords([[1, 2, 3], [20, 20, 20]], [np.array([1.0, 2.0], np.float32)])
+    g.flush(["smax"])
+    good = g.pack([((0, 0, 0), (31, 31, 31))], [0])
+    head = 8 + 24
+    bad = [good[:head - 1], good[:head + 17], good[:-1]]
+    for at, v in ((0, 1 << 62), (0, len(good)), (0, (1 << 64) - 2)):
+        x = good.copy()
+        x[at:at + 8] = np.frombuffer(np.uint64(v).tobytes(), np.uint8)
+        bad.append(x)
+    x = good.copy()
+    x[head + 16:head + 20] = 1  # the scan starts past 0
+    bad.append(x)
+    for x in bad:
+        for buf in (x, torch.from_numpy(x.copy()).cuda()):
+            with pytest.raises(SgError):
+                g.unpack(buf, (0, 0, 0), [0])
+    assert g.pending_inserts() == 0
+    assert g.unpack(torch.from_numpy(good).cuda(), (0, 0, 0), [0]) == len(good)
+    g.close()
