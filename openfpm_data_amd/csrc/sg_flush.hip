@@ -350,10 +350,13 @@ __device__ inline uint32_t run_block_scan(uint32_t v, uint32_t *total)
     return pre + inc - v;
 }
 
-// the number of runs starting in each tile
+// the number of runs starting in each tile; with flag, *flag_out = *flag (a pinned word: the
+// host reads it with the totals)
 __global__ __launch_bounds__(kWG) void run_count_kernel(const uint32_t *__restrict__ sk, int64_t n,
-                                                       uint32_t *__restrict__ cnt)
+                                                       uint32_t *__restrict__ cnt, const int *__restrict__ flag,
+                                                       uint32_t *__restrict__ flag_out)
 {
+    if (flag && blockIdx.x == 0 && threadIdx.x == 0) *flag_out = (uint32_t)*flag;
     const int64_t i0 = (int64_t)blockIdx.x * kRunTile + (int64_t)threadIdx.x * kRunIPT;
     uint32_t k[kRunIPT], prev;
     run_items(sk, n, i0, k, prev);
@@ -369,10 +372,10 @@ __global__ __launch_bounds__(kWG) void run_count_kernel(const uint32_t *__restri
 }
 
 // each run's key and first item at the run's rank (off: exclusive scan of the tiles'
-// counts; start[nu] = n)
+// counts, *nu their sum; start[*nu] = n)
 __global__ __launch_bounds__(kWG) void run_emit_kernel(const uint32_t *__restrict__ sk, int64_t n,
                                                       const uint32_t *__restrict__ off, int64_t *__restrict__ key,
-                                                      uint32_t *__restrict__ start, uint32_t nu)
+                                                      uint32_t *__restrict__ start, const uint32_t *__restrict__ nu)
 {
     const int64_t i0 = (int64_t)blockIdx.x * kRunTile + (int64_t)threadIdx.x * kRunIPT;
     uint32_t k[kRunIPT], prev;
@@ -395,7 +398,7 @@ __global__ __launch_bounds__(kWG) void run_emit_kernel(const uint32_t *__restric
             ++u;
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) start[nu] = (uint32_t)n;
+    if (blockIdx.x == 0 && threadIdx.x == 0) start[*nu] = (uint32_t)n;
 }
 
 // unique points (construct_index_unique, src/util/cuda/kernels.cuh:34-54)
@@ -440,36 +443,37 @@ __device__ inline int64_t lower_bound_dev(const int64_t *a, int64_t n, int64_t x
     return lo;
 }
 
-// new chunk j: position in the old list or -1, and the brand-new flag
+// touched chunk j: its position in the old list or -1, the brand-new flag, and (lb != nullptr)
+// the number of old chunks before it.  With count the chunks are the first *count of the nn
+// entries (the others get flag 0), and *count_out = *count.
 __global__ void old_lookup_kernel(const int64_t *nkey, int64_t nn, const int64_t *okeys, int64_t m, int64_t *oldpos,
-                                  uint32_t *isnew)
+                                  uint32_t *isnew, int64_t *lb, const uint32_t *count, uint32_t *count_out)
 {
     int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (count && j == 0) *count_out = *count;
     if (j >= nn) return;
-    int64_t k = nkey[j];
-    int64_t lb = lower_bound_dev(okeys, m, k);
-    bool found = lb < m && okeys[lb] == k;
-    oldpos[j] = found ? lb : -1;
+    if (count && j >= (int64_t)*count) {
+        isnew[j] = 0;
+        return;
+    }
+    const int64_t k = nkey[j], p = lower_bound_dev(okeys, m, k);
+    const bool found = p < m && okeys[p] == k;
+    oldpos[j] = found ? p : -1;
     isnew[j] = found ? 0u : 1u;
+    if (lb) lb[j] = p;
 }
 
-__global__ void brand_new_kernel(const int64_t *nkey, const uint32_t *isnew, const uint32_t *nscan, int64_t nn,
-                                 int64_t *bn)
+// final position of each touched chunk in the union, cpos[j] (on entry the old chunks before
+// it): those plus the new chunks before it, which the scan of the flags counts, as the
+// touched chunks are sorted; and the new chunks' ids in order
+__global__ void place_chunks_kernel(const int64_t *nkey, const uint32_t *isnew, const uint32_t *nscan, int64_t nn,
+                                    const uint32_t *count, int64_t *cpos, int64_t *bn)
 {
     int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < nn && isnew[j]) bn[nscan[j]] = nkey[j];
-}
-
-// final chunk position of each new-touched chunk (merge-path rank in the union)
-__global__ void chunk_pos_kernel(const int64_t *nkey, const int64_t *oldpos, const uint32_t *nscan, int64_t nn,
-                                 const int64_t *okeys, int64_t m, const int64_t *bn, int64_t nb, int64_t *cpos)
-{
-    int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= nn) return;
-    int64_t k = nkey[j];
-    int64_t op = oldpos[j];
-    if (op >= 0) cpos[j] = op + lower_bound_dev(bn, nb, k);
-    else cpos[j] = (int64_t)nscan[j] + lower_bound_dev(okeys, m, k);
+    if (j >= nn || (count && j >= (int64_t)*count)) return;
+    const uint32_t s = nscan[j];
+    cpos[j] += s;
+    if (isnew[j]) bn[s] = nkey[j];
 }
 
 // scatter the old chunks into the enlarged arrays (copy_old_ker, BlockMapGpu_kernels.cuh:489-513)
@@ -2220,32 +2224,45 @@ void finish_merge(sg_grid *g, MergeDefer &df)
 }
 
 
-// brand-new chunks are placed by merge-path rank, the arrays grow (old chunks moved, new
-// ones mask 0 / background), and cpos[j] is the final position of nkey[j].
-int merge_chunk_set(sg_grid *g, const int64_t *nkey, int64_t nnew, int64_t **cpos_out, MergeDefer *df)
+// the touched chunks against the old chunk list (scratch arrays of `bound` entries)
+struct MergeLookup {
+    int64_t *oldpos, *cpos, *bn;
+    uint32_t *isnew, *nscan;
+};
+
+// Queues the lookup of the touched chunks nkey[0 .. nn) and their placing in the union: nn =
+// bound, or *count (device memory) when count is given; bound >= nn sizes the launches.  The
+// number of brand-new chunks goes to pinned word 0, *count to pinned word 1.
+int merge_lookup(sg_grid *g, const int64_t *nkey, int64_t bound, const uint32_t *count, uint32_t *hw, MergeLookup *L)
+{
+    DevBuf &b_c = g->scratch[5];
+    const int rc = ensure(g->pool, b_c, (size_t)bound * (8 + 4 + 4 + 8 + 8) + 128);
+    if (rc) return rc;
+    L->oldpos = (int64_t *)b_c.p;
+    L->isnew = (uint32_t *)(L->oldpos + bound);
+    L->nscan = L->isnew + bound;
+    L->cpos = (int64_t *)(((uintptr_t)(L->nscan + bound) + 15) & ~(uintptr_t)15);
+    L->bn = L->cpos + bound;
+    hipLaunchKernelGGL(old_lookup_kernel, dim3(grid_1d(bound, kWG)), dim3(kWG), 0, g->stream, nkey, bound, g->d_keys,
+                       g->nchunks, L->oldpos, L->isnew, L->cpos, count, hw + 1);
+    SG_HIP(hipGetLastError());
+    const int rs = exclusive_scan_u32_queued(g, L->isnew, L->nscan, bound, hw);
+    if (rs) return rs;
+    hipLaunchKernelGGL(place_chunks_kernel, dim3(grid_1d(bound, kWG)), dim3(kWG), 0, g->stream, nkey, L->isnew, L->nscan,
+                       bound, count, L->cpos, L->bn);
+    SG_HIP(hipGetLastError());
+    return SG_OK;
+}
+
+// the chunk set with the nb brand-new chunks of a lookup: the arrays grow (old chunks moved,
+// new ones mask 0 / background), and cpos[j] is the final position of touched chunk j (nnew)
+int merge_grow(sg_grid *g, const MergeLookup &L, int64_t nnew, int64_t nb, int64_t **cpos_out, MergeDefer *df)
 {
     const int csz = g->csz;
     const int64_t m = g->nchunks;
     int rc;
-    DevBuf &b_c = g->scratch[5];
-    if ((rc = ensure(g->pool, b_c, (size_t)nnew * (8 + 4 + 4 + 8 + 8) + 128))) return rc;
-    int64_t *oldpos = (int64_t *)b_c.p;
-    uint32_t *isnew = (uint32_t *)(oldpos + nnew);
-    uint32_t *nscan = isnew + nnew;
-    int64_t *cpos = (int64_t *)(((uintptr_t)(nscan + nnew) + 15) & ~(uintptr_t)15);
-    int64_t *bn = cpos + nnew;
-    hipLaunchKernelGGL(old_lookup_kernel, dim3(grid_1d(nnew, kWG)), dim3(kWG), 0, g->stream, nkey, nnew, g->d_keys,
-                       m, oldpos, isnew);
-    SG_HIP(hipGetLastError());
-    uint32_t nb32 = 0;
-    if ((rc = exclusive_scan_u32(g, isnew, nscan, nnew, &nb32))) return rc;
-    const int64_t nb = nb32;
-    hipLaunchKernelGGL(brand_new_kernel, dim3(grid_1d(nnew, kWG)), dim3(kWG), 0, g->stream, nkey, isnew, nscan, nnew,
-                       bn);
-    SG_HIP(hipGetLastError());
-    hipLaunchKernelGGL(chunk_pos_kernel, dim3(grid_1d(nnew, kWG)), dim3(kWG), 0, g->stream, nkey, oldpos, nscan, nnew,
-                       g->d_keys, m, bn, nb, cpos);
-    SG_HIP(hipGetLastError());
+    int64_t *oldpos = L.oldpos, *cpos = L.cpos, *bn = L.bn;
+    uint32_t *isnew = L.isnew;
     if (df) {
         df->oldpos = oldpos;
         df->isnew = isnew;
@@ -2400,6 +2417,19 @@ int merge_chunk_set(sg_grid *g, const int64_t *nkey, int64_t nnew, int64_t **cpo
     return SG_OK;
 }
 
+// both, for touched chunks whose number the host knows
+int merge_chunk_set(sg_grid *g, const int64_t *nkey, int64_t nnew, int64_t **cpos_out, MergeDefer *df)
+{
+    uint32_t *hw = host_words(g);
+    if (!hw) return fail(SG_E_OOM, "pinned host allocation failed");
+    hw[0] = 0;
+    MergeLookup L;
+    const int rc = merge_lookup(g, nkey, nnew, nullptr, hw, &L);
+    if (rc) return rc;
+    SG_HIP(hipStreamSynchronize(g->stream));
+    return merge_grow(g, L, nnew, hw[0], cpos_out, df);
+}
+
 // flush of whole-chunk records only: stable sort of (chunk id, record id), unique chunk
 // ids + segment starts, merge into the chunk map, one workgroup per touched chunk folds
 // its records slot by slot
@@ -2410,21 +2440,14 @@ int flush_chunks_impl(sg_grid *g, const int32_t *ops)
     const int csz = g->csz;
     const int64_t nblocks = key_limit(g) / csz;
     int rc;
-    {
-        if ((rc = ensure(g->pool, g->scratch[6], 64))) return rc;
-        int *bad = (int *)g->scratch[6].p;
-        SG_HIP(hipMemsetAsync(bad, 0, sizeof(int), g->stream));
-        hipLaunchKernelGGL(check_keys_kernel, dim3(grid_1d(n, kWG)), dim3(kWG), 0, g->stream, g->d_cins_id, n,
-                           nblocks, bad);
-        SG_HIP(hipGetLastError());
-        int hbad = 0;
-        SG_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-        SG_HIP(hipStreamSynchronize(g->stream));
-        if (hbad) {
-            g->cins_n = 0;
-            return fail(SG_E_RANGE, "chunk id outside the grid in the insert buffer");
-        }
-    }
+    // ids outside the grid: the flag comes back with the first scan total below (the grid is
+    // not touched before it is read; such ids only reorder scratch data)
+    uint32_t *hw = host_words(g);
+    if (!hw) return fail(SG_E_OOM, "pinned host allocation failed");
+    hw[8] = 0;
+    hipLaunchKernelGGL(check_keys_kernel, dim3(grid_1d(n, kWG)), dim3(kWG), 0, g->stream, g->d_cins_id, n, nblocks,
+                       (int *)(hw + 8));
+    SG_HIP(hipGetLastError());
     int bits = 0;
     while (bits < 63 && (((int64_t)1 << bits) < nblocks)) ++bits;
     const bool k32 = bits <= 32;
@@ -2470,6 +2493,10 @@ int flush_chunks_impl(sg_grid *g, const int32_t *ops)
     SG_HIP(hipGetLastError());
     uint32_t nu32 = 0;
     if ((rc = exclusive_scan_u32(g, head, hscan, n, &nu32))) return rc;
+    if (hw[8]) {
+        g->cins_n = 0;
+        return fail(SG_E_RANGE, "chunk id outside the grid in the insert buffer");
+    }
     const int64_t nu = nu32;
     if (k32)
         hipLaunchKernelGGL(unique_points_kernel<uint32_t>, dim3(grid_1d(n, kWG)), dim3(kWG), 0, g->stream,
@@ -2533,9 +2560,9 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
         staged = false;
     }
     const int64_t n = staged ? g->pins_n : g->ins_n;
-    if ((rc = ensure(g->pool, g->scratch[6], 64))) return rc;
-    int *bad = (int *)g->scratch[6].p;
-    SG_HIP(hipMemsetAsync(bad, 0, sizeof(int), g->stream));
+    // the range flags (pinned words 8: insert buffer, 9: staged pairs), read after the wait below
+    hw[0] = hw[8] = hw[9] = 0;
+    int *bad = (int *)(hw + 8);
 
     FoldProps F;
     F.np = g->np;
@@ -2572,20 +2599,39 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
                                     R.nv, n, cbits, &ck, &rec);
     }
     if (rc) return rc;
-    // the range flags, read with the scan total below
-    SG_HIP(hipMemcpyAsync(hw + 8, bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-    if (staged) SG_HIP(hipMemcpyAsync(hw + 9, g->d_pins_bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-    // touched chunks: runs of equal sorted chunk ids, counted per tile, tile offsets
-    // scanned, then each run's id and first record written at its offset
+    // Touched chunks: runs of equal sorted chunk ids, counted per tile, tile offsets scanned,
+    // then each run's id and first record written at its offset; then their lookup in the
+    // chunk list.  Up to kBound touched chunks can be expected (by the records and the
+    // domain), all of it is queued before the one wait of the flush, on arrays and launches of
+    // that bound; beyond, the host waits for their number first (2^20 entries are 46 MB of
+    // temporaries; a wait is some 15 us).  Ids outside the grid lead to no access outside the
+    // arrays: staged ones are one more distinct id, 0xffffffff.
     const int64_t rtiles = (n + kRunTile - 1) / kRunTile;
+    constexpr int64_t kBound = 1 << 20;
+    int64_t bound = std::min<int64_t>(n, limit / csz + 1);
+    const bool queued = bound <= kBound;
     DevBuf &b_h = g->scratch[4];
     if ((rc = ensure(g->pool, b_h, (size_t)rtiles * 8 + 64))) return rc;
-    uint32_t *rcnt = (uint32_t *)b_h.p, *roff = rcnt + rtiles;
+    uint32_t *rcnt = (uint32_t *)b_h.p, *roff = rcnt + rtiles, *d_nn = roff + rtiles;
     hipLaunchKernelGGL(run_count_kernel, dim3((unsigned)rtiles), dim3(kWG), 0, g->stream, (const uint32_t *)ck, n,
-                       rcnt);
+                       rcnt, staged ? g->d_pins_bad : nullptr, hw + 9);
     SG_HIP(hipGetLastError());
-    uint32_t nn32 = 0;
-    if ((rc = exclusive_scan_u32(g, rcnt, roff, rtiles, &nn32))) return rc;
+    if ((rc = exclusive_scan_u32_queued(g, rcnt, roff, rtiles, d_nn))) return rc;
+    if (!queued) {
+        SG_HIP(hipMemcpyAsync(hw + 1, d_nn, sizeof(uint32_t), hipMemcpyDeviceToHost, g->stream));
+        SG_HIP(hipStreamSynchronize(g->stream));
+        bound = hw[1];
+    }
+    // unique chunk ids and the first record of each (ustart[nnew] = n)
+    if ((rc = ensure(g->pool, g->scratch[12], (size_t)bound * 8 + (size_t)(bound + 1) * 4 + 64))) return rc;
+    int64_t *nkey = (int64_t *)g->scratch[12].p;
+    uint32_t *ustart = (uint32_t *)(nkey + bound);
+    hipLaunchKernelGGL(run_emit_kernel, dim3((unsigned)rtiles), dim3(kWG), 0, g->stream, (const uint32_t *)ck, n, roff,
+                       nkey, ustart, (const uint32_t *)d_nn);
+    SG_HIP(hipGetLastError());
+    MergeLookup ML;
+    if ((rc = merge_lookup(g, nkey, bound, d_nn, hw, &ML))) return rc;
+    SG_HIP(hipStreamSynchronize(g->stream));
     if (staged && hw[9]) {
         // the staged pairs, intact, through the insert buffer: the flush by chunk id over it
         // drops the records outside the grid and reports them
@@ -2599,21 +2645,14 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
         return fail(SG_E_RANGE, std::to_string(n - kept) + " inserted points outside the grid were dropped; the other " +
                                     std::to_string(kept) + " stay pending (flush again to merge them)");
     }
-    const int64_t nnew = nn32;
-    // unique chunk ids and the first record of each (ustart[nnew] = n)
-    if ((rc = ensure(g->pool, g->scratch[12], (size_t)nnew * 8 + (size_t)(nnew + 1) * 4 + 64))) return rc;
-    int64_t *nkey = (int64_t *)g->scratch[12].p;
-    uint32_t *ustart = (uint32_t *)(nkey + nnew);
-    hipLaunchKernelGGL(run_emit_kernel, dim3((unsigned)rtiles), dim3(kWG), 0, g->stream, (const uint32_t *)ck, n, roff,
-                       nkey, ustart, nn32);
-    SG_HIP(hipGetLastError());
+    const int64_t nnew = hw[1];
 
     MergeDefer df;
     // 8^3 chunks: the EXIST bit-planes are kept up to date when they are valid (or the
     // grid has no chunk yet): the fold writes those of the touched chunks
     df.planes = g->dim == 3 && g->edge == 8 && (g->ebits_valid || g->nchunks == 0);
     int64_t *cpos = nullptr;
-    if ((rc = merge_chunk_set(g, nkey, nnew, &cpos, &df))) return rc;
+    if ((rc = merge_grow(g, ML, nnew, hw[0], &cpos, &df))) return rc;
     const bool planes = df.planes;
     uint64_t *eb = planes ? g->d_ebits : nullptr;
     FusedImg I;
@@ -2731,10 +2770,8 @@ int flush_impl(sg_grid *g, const int32_t *ops)
     // grid is not touched before it is read; out-of-range keys only reorder scratch data)
     uint32_t *hw = host_words(g);
     if (!hw) return fail(SG_E_OOM, "pinned host allocation failed");
-    rc = ensure(g->pool, g->scratch[6], 64);
-    if (rc) return rc;
-    int *bad = (int *)g->scratch[6].p;
-    SG_HIP(hipMemsetAsync(bad, 0, sizeof(int), g->stream));
+    hw[8] = 0;
+    int *bad = (int *)(hw + 8);
     int bits = 0;
     while (bits < 63 && (((int64_t)1 << bits) < limit)) ++bits;
     const bool k32 = bits <= 32;
@@ -2767,8 +2804,6 @@ int flush_impl(sg_grid *g, const int32_t *ops)
         sk = ko;
     }
     if (rc) return rc;
-    // the range flag of the sort-key pass, read with the first scan total below
-    SG_HIP(hipMemcpyAsync(hw + 8, bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
     // the temporaries not holding the sorted result are free for reuse
     uint32_t *spare_a = (perm == (uint32_t *)b_vals.p) ? (uint32_t *)b_tv.p : (uint32_t *)b_vals.p;
 
@@ -2976,7 +3011,8 @@ int set_chunks_impl(sg_grid *g, int64_t n, const int64_t *ids, const uint8_t *ma
         SG_HIP(hipMemcpyAsync(nkeys, hid.data(), (size_t)n * 8, hipMemcpyHostToDevice, g->stream));
         SG_HIP(hipMemcpyAsync(nmask, masks, (size_t)n * csz, kind, g->stream));
         hipLaunchKernelGGL(old_lookup_kernel, dim3(grid_1d(n, kWG)), dim3(kWG), 0, g->stream, nkeys, n, g->d_keys,
-                           g->nchunks, oldpos, isnew);
+                           g->nchunks, oldpos, isnew, (int64_t *)nullptr, (const uint32_t *)nullptr,
+                           (uint32_t *)nullptr);
         SG_HIP(hipGetLastError());
     }
     SG_HIP(hipMemsetAsync(nmask + (size_t)n * csz, 0, csz, g->stream));

@@ -212,8 +212,8 @@ struct sg_grid {
     sg::DevicePool pool;
     sg::DevBuf scratch[14];  // flush / sort / scan temporaries
     sg::DevBuf hostlike;     // small device staging
-    // pinned host words for device -> host copies of flags and totals: queued without
-    // blocking the host, read after the next stream synchronisation
+    // pinned host words that kernels write flags and totals to, read after the next stream
+    // synchronisation
     uint32_t *h_words = nullptr;
     ~sg_grid()
     {
@@ -366,6 +366,9 @@ int restore_background_impl(sg_grid *g, int prop);
 // device-wide primitives (sg_primitives.hip)
 // exclusive scan of n uint32 values; *total (host) receives the sum when non-null
 int exclusive_scan_u32(sg_grid *g, const uint32_t *in, uint32_t *out, int64_t n, uint32_t *total);
+// the same without a wait: total (device or pinned host memory, may be null) receives the sum
+// when the stream gets there
+int exclusive_scan_u32_queued(sg_grid *g, const uint32_t *in, uint32_t *out, int64_t n, uint32_t *total);
 // the same on `stream` with a caller-provided workspace of ws_words >= scan_ws_words(n) words;
 // d_total (device, may be null) receives the sum; allocates nothing and does not wait
 size_t scan_ws_words(int64_t n);

@@ -302,41 +302,49 @@ int radix_sort_pairs(sg_grid *g, K *keys, uint32_t *vals, K *keys_tmp, uint32_t 
 constexpr int kRecIPT = 8;
 constexpr int kRecTile = kSortWG * kRecIPT;
 
-// the digit counts of kHistTiles consecutive tiles per workgroup (every key of the
-// workgroup loaded before the first is counted)
-constexpr int kHistTiles = 4;
+// the digit counts of HT consecutive tiles per workgroup (every key of the workgroup loaded
+// before the first is counted), D digits at most.  Four tiles a workgroup for long inputs
+// (33.6 us for 2^24 keys against 39 us with one); one where that leaves the chip idle: 98
+// tiles (200,000 keys) as 25 workgroups took 11.9 us, 25 tiles as 7 17.4 us, bound by the
+// 32 LDS atomics each thread issues one after the other (now 4.9 and 5.9 us).
+template <int HT, int D>
 __global__ __launch_bounds__(kSortWG) void radix_hist_rec_kernel(const uint32_t *keys, uint32_t *counts, int64_t n,
                                                                  int shift, uint32_t dmask, int ntiles)
 {
-    __shared__ uint32_t s_hist[kHistTiles][256];
+    __shared__ uint32_t s_hist[HT][D];
     const int t = threadIdx.x;
 #pragma unroll
-    for (int h = 0; h < kHistTiles; ++h) s_hist[h][t] = 0;
-    uint32_t d[kHistTiles][kRecIPT];
+    for (int h = 0; h < HT; ++h)
 #pragma unroll
-    for (int h = 0; h < kHistTiles; ++h) {
-        const int64_t base = ((int64_t)blockIdx.x * kHistTiles + h) * kRecTile;
+        for (int i = t; i < D; i += kSortWG) s_hist[h][i] = 0;
+    uint32_t d[HT][kRecIPT];
+#pragma unroll
+    for (int h = 0; h < HT; ++h) {
+        const int64_t base = ((int64_t)blockIdx.x * HT + h) * kRecTile;
 #pragma unroll
         for (int j = 0; j < kRecIPT; ++j) {
             const int64_t i = base + (int64_t)j * kSortWG + t;
-            d[h][j] = (i < n) ? (keys[i] >> shift) & dmask : 256u;
+            d[h][j] = (i < n) ? (keys[i] >> shift) & dmask : (uint32_t)D;
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int h = 0; h < kHistTiles; ++h)
+    for (int h = 0; h < HT; ++h)
 #pragma unroll
         for (int j = 0; j < kRecIPT; ++j)
-            if (d[h][j] < 256u) atomicAdd(&s_hist[h][d[h][j]], 1u);
+            if (d[h][j] < (uint32_t)D) atomicAdd(&s_hist[h][d[h][j]], 1u);
     __syncthreads();
 #pragma unroll
-    for (int h = 0; h < kHistTiles; ++h) {
-        const int64_t tile = (int64_t)blockIdx.x * kHistTiles + h;
-        if (tile < ntiles && (uint32_t)t <= dmask) counts[(int64_t)t * ntiles + tile] = s_hist[h][t];
+    for (int h = 0; h < HT; ++h) {
+        const int64_t tile = (int64_t)blockIdx.x * HT + h;
+#pragma unroll
+        for (int i = t; i < D; i += kSortWG)
+            if (tile < ntiles && (uint32_t)i <= dmask) counts[(int64_t)i * ntiles + tile] = s_hist[h][i];
     }
 }
 
-template <int NV>
+// D: the most digits of a pass (256, or 512 for short inputs; see radix_sort_records_u32)
+template <int NV, int D>
 __global__ __launch_bounds__(kSortWG) void radix_scatter_rec_kernel(const uint32_t *__restrict__ keys,
                                                                     const uint4 *__restrict__ recs,
                                                                     uint32_t *__restrict__ okeys,
@@ -345,20 +353,35 @@ __global__ __launch_bounds__(kSortWG) void radix_scatter_rec_kernel(const uint32
                                                                     const uint32_t *__restrict__ counts, int64_t n,
                                                                     int shift, int dbits, int ntiles)
 {
+    constexpr int DT = D / kSortWG;  // digits per thread: t DT .. t DT + DT - 1
     __shared__ uint32_t s_key[kRecTile];
     const uint32_t dmask = (1u << dbits) - 1u;
     __shared__ uint4 s_rec[kRecTile * NV];
-    __shared__ uint32_t s_gbase[256];
-    __shared__ uint32_t s_lstart[256];
-    __shared__ uint32_t s_wcnt[kSortWG / 64][256];
+    __shared__ uint32_t s_gbase[D];
+    __shared__ uint32_t s_lstart[D];
+    __shared__ uint32_t s_wcnt[kSortWG / 64][D];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     // the count table holds the 2^dbits digits of this pass
-    const bool dig = (uint32_t)t <= dmask;
-    s_gbase[t] = dig ? offsets[(int64_t)t * ntiles + blockIdx.x] : 0u;
-    uint32_t tot;
-    s_lstart[t] = block_exclusive_scan(dig ? counts[(int64_t)t * ntiles + blockIdx.x] : 0u, &tot);
+    uint32_t dc[DT], dsum = 0;
 #pragma unroll
-    for (int q = 0; q < kSortWG / 64; ++q) s_wcnt[q][t] = 0;
+    for (int k = 0; k < DT; ++k) {
+        const int i = t * DT + k;
+        const bool dig = (uint32_t)i <= dmask;
+        s_gbase[i] = dig ? offsets[(int64_t)i * ntiles + blockIdx.x] : 0u;
+        dc[k] = dig ? counts[(int64_t)i * ntiles + blockIdx.x] : 0u;
+        dsum += dc[k];
+    }
+    uint32_t tot;
+    uint32_t run0 = block_exclusive_scan(dsum, &tot);
+#pragma unroll
+    for (int k = 0; k < DT; ++k) {
+        s_lstart[t * DT + k] = run0;
+        run0 += dc[k];
+    }
+#pragma unroll
+    for (int q = 0; q < kSortWG / 64; ++q)
+#pragma unroll
+        for (int k = 0; k < DT; ++k) s_wcnt[q][t * DT + k] = 0;
     // Wave w owns the tile's items [w * 64 * IPT, (w + 1) * 64 * IPT), item j of a lane at
     // w * 64 * IPT + j * 64 + lane, so index order is (wave, j, lane): a wave ranks its
     // items among equal digits by ballots and a running count per digit of its own (LDS,
@@ -394,13 +417,14 @@ __global__ __launch_bounds__(kSortWG) void radix_scatter_rec_kernel(const uint32
         if (valid && lr == 0) s_wcnt[w][d] = before + (uint32_t)__popcll(peers);
     }
     __syncthreads();
-    {
+#pragma unroll
+    for (int k = 0; k < DT; ++k) {
         // per digit: the exclusive prefix of the waves' counts
         uint32_t run = 0;
 #pragma unroll
         for (int q = 0; q < kSortWG / 64; ++q) {
-            const uint32_t c = s_wcnt[q][t];
-            s_wcnt[q][t] = run;
+            const uint32_t c = s_wcnt[q][t * DT + k];
+            s_wcnt[q][t * DT + k] = run;
             run += c;
         }
     }
@@ -441,27 +465,43 @@ int radix_sort_records_u32(sg_grid *g, uint32_t *keys, uint4 *recs, uint32_t *ke
     if (n >= (int64_t)1 << 31) return fail(SG_E_RANGE, "radix sort supports fewer than 2^31 items");
     const int ntiles = (int)((n + kRecTile - 1) / kRecTile);
     DevBuf &cbuf = g->scratch[10];
-    int rc = ensure(g->pool, cbuf, (size_t)256 * ntiles * sizeof(uint32_t) * 2);
+    // 8-bit digits, or 9-bit ones for up to 2^20 items where that saves a pass: such an input
+    // stays in the caches, so the shorter runs cost less than a pass's launches (18 bits of
+    // 200,000 keys: a merge of them takes 327 us with 3 passes of 6 bits, 312 us with 2 of 9);
+    // longer inputs are bound by the partial lines that short runs write
+    const int most = (n <= (1 << 20) && (bits + 8) / 9 < (bits + 7) / 8) ? 9 : 8;
+    int rc = ensure(g->pool, cbuf, ((size_t)1 << most) * ntiles * sizeof(uint32_t) * 2);
     if (rc) return rc;
     uint32_t *counts = (uint32_t *)cbuf.p;
-    uint32_t *offs = counts + (size_t)256 * ntiles;
+    uint32_t *offs = counts + ((size_t)1 << most) * ntiles;
     uint32_t *src_k = keys, *dst_k = keys_tmp;
     uint4 *src_r = recs, *dst_r = recs_tmp;
-    // as few passes as 8-bit digits need, the bits shared evenly among them (21 bits: 3
+    // as few passes as those digits need, the bits shared evenly among them (21 bits: 3
     // passes of 7, so that a tile's run of one digit is twice as long as with 256 digits)
-    const int passes = (bits + 7) / 8, dbits = (bits + passes - 1) / passes;
+    const int passes = (bits + most - 1) / most, dbits = (bits + passes - 1) / passes;
+    const bool wide = dbits > 8;
     for (int shift = 0; shift < bits; shift += dbits) {
-        hipLaunchKernelGGL(radix_hist_rec_kernel, dim3((ntiles + kHistTiles - 1) / kHistTiles), dim3(kSortWG), 0,
-                           g->stream, src_k, counts, n, shift, (1u << dbits) - 1u, ntiles);
+        const uint32_t dmask = (1u << dbits) - 1u;
+        if (wide)
+            hipLaunchKernelGGL((radix_hist_rec_kernel<1, 512>), dim3(ntiles), dim3(kSortWG), 0, g->stream, src_k, counts, n,
+                               shift, dmask, ntiles);
+        else if (ntiles < 1024)
+            hipLaunchKernelGGL((radix_hist_rec_kernel<1, 256>), dim3(ntiles), dim3(kSortWG), 0, g->stream, src_k, counts, n,
+                               shift, dmask, ntiles);
+        else
+            hipLaunchKernelGGL((radix_hist_rec_kernel<4, 256>), dim3((ntiles + 3) / 4), dim3(kSortWG), 0, g->stream, src_k,
+                               counts, n, shift, dmask, ntiles);
         SG_HIP(hipGetLastError());
         rc = exclusive_scan_u32(g, counts, offs, ((int64_t)1 << dbits) * ntiles, nullptr);
         if (rc) return rc;
-        if (nv == 1)
-            hipLaunchKernelGGL(radix_scatter_rec_kernel<1>, dim3(ntiles), dim3(kSortWG), 0, g->stream, src_k, src_r,
-                               dst_k, dst_r, offs, counts, n, shift, dbits, ntiles);
-        else
-            hipLaunchKernelGGL(radix_scatter_rec_kernel<2>, dim3(ntiles), dim3(kSortWG), 0, g->stream, src_k, src_r,
-                               dst_k, dst_r, offs, counts, n, shift, dbits, ntiles);
+        auto scatter = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kSortWG), 0, g->stream, src_k, src_r, dst_k, dst_r, offs, counts, n,
+                               shift, dbits, ntiles);
+        };
+        if (nv == 1 && wide) scatter(radix_scatter_rec_kernel<1, 512>);
+        else if (nv == 1) scatter(radix_scatter_rec_kernel<1, 256>);
+        else if (wide) scatter(radix_scatter_rec_kernel<2, 512>);
+        else scatter(radix_scatter_rec_kernel<2, 256>);
         SG_HIP(hipGetLastError());
         std::swap(src_k, dst_k);
         std::swap(src_r, dst_r);
@@ -554,24 +594,29 @@ int exclusive_scan_u32_ws(hipStream_t stream, const uint32_t *in, uint32_t *out,
     return SG_OK;
 }
 
+int exclusive_scan_u32_queued(sg_grid *g, const uint32_t *in, uint32_t *out, int64_t n, uint32_t *total)
+{
+    if (n <= 0) return SG_OK;
+    const size_t words = scan_ws_words(n);
+    DevBuf &sb = g->scratch[11];
+    const int rc = ensure(g->pool, sb, (words + 2) * sizeof(uint32_t));
+    if (rc) return rc;
+    return exclusive_scan_u32_ws(g->stream, in, out, n, total, (uint32_t *)sb.p, words);
+}
+
 int exclusive_scan_u32(sg_grid *g, const uint32_t *in, uint32_t *out, int64_t n, uint32_t *total)
 {
     if (n <= 0) {
         if (total) *total = 0;
         return SG_OK;
     }
-    const size_t words = scan_ws_words(n) + 2;
-    DevBuf &sb = g->scratch[11];
-    int rc = ensure(g->pool, sb, words * sizeof(uint32_t));
+    // the scan writes the total to a pinned word: no copy, and words that earlier kernels
+    // wrote there need no wait of their own
+    uint32_t *hw = total ? host_words(g) : nullptr;
+    if (total && !hw) return fail(SG_E_OOM, "pinned host allocation failed");
+    const int rc = exclusive_scan_u32_queued(g, in, out, n, hw);
     if (rc) return rc;
-    uint32_t *d_total = (uint32_t *)sb.p + (words - 2);
-    if ((rc = exclusive_scan_u32_ws(g->stream, in, out, n, total ? d_total : nullptr, (uint32_t *)sb.p, words - 2)))
-        return rc;
     if (total) {
-        // through a pinned word, so that copies queued before it need no wait of their own
-        uint32_t *hw = host_words(g);
-        if (!hw) return fail(SG_E_OOM, "pinned host allocation failed");
-        SG_HIP(hipMemcpyAsync(hw, d_total, sizeof(uint32_t), hipMemcpyDeviceToHost, g->stream));
         SG_HIP(hipStreamSynchronize(g->stream));
         *total = hw[0];
     }
