@@ -694,10 +694,11 @@ __global__ __launch_bounds__(kWG) void fold_points_kernel(const int64_t *ukey, c
     omask[slot] = (uint8_t)(om | am);
 }
 
-__global__ void mark_positions_kernel(const int64_t *pos, int64_t n, uint8_t *flag)
+// only: nullptr, or the entries to mark
+__global__ void mark_positions_kernel(const int64_t *pos, int64_t n, uint8_t *flag, const uint32_t *only)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) flag[pos[i]] = 1;
+    if (i < n && (!only || only[i])) flag[pos[i]] = 1;
 }
 
 // LDS image of one chunk for the fused fold: property q at byte off[q], mask at moff,
@@ -1075,12 +1076,13 @@ __device__ inline void fold_batch_prop(int op, unsigned char *vals, const unsign
 }
 
 // one property of a touched chunk: old contents (OLD; the background for a new chunk)
-// combined with the folded records (fold_old) and written once at the final position
+// combined with the folded records (fold_old) and written once at the final position.
+// inplace: that is where the old contents are, so vectors without a record are left alone.
 template <typename T, bool OLD>
 __device__ inline void write_fold_prop(int op, T bgv, const unsigned char *__restrict__ vals,
                                        const uint8_t *__restrict__ seen, const uint8_t *__restrict__ am,
-                                       const T *__restrict__ src, const uint8_t *__restrict__ smask, T *__restrict__ dst,
-                                       int csz, int lane)
+                                       const T *src, const uint8_t *smask, T *dst, int csz, int lane,
+                                       bool inplace = false)
 {
     typedef unsigned int v4u __attribute__((ext_vector_type(4)));
     constexpr int PPV = 16 / (int)sizeof(T);
@@ -1101,14 +1103,26 @@ __device__ inline void write_fold_prop(int op, T bgv, const unsigned char *__res
                 v4u q;
                 T t[PPV];
             } u[G];
-            union {
+            union MaskV {
                 MaskW w;
                 uint8_t b[PPV];
-            } om[G];
+            } om[G], sw[G];
+            // the vectors' seen bytes in one LDS read each (most vectors receive no record)
+            bool any[G], need[G];
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 const int v = v0 + 64 * g;
-                if (OLD && v < nvec) {
+                need[g] = v < nvec;
+                sw[g].w = need[g] ? ((const MaskW *)seen)[v] : MaskW();
+                any[g] = false;
+#pragma unroll
+                for (int x = 0; x < PPV; ++x) any[g] = any[g] || sw[g].b[x] != 0;
+                if (OLD && inplace) need[g] = any[g];
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const int v = v0 + 64 * g;
+                if (OLD && need[g]) {
                     u[g].q = ((const v4u *)src)[v];
                     om[g].w = ((const MaskW *)smask)[v];
                 } else {
@@ -1122,20 +1136,11 @@ __device__ inline void write_fold_prop(int op, T bgv, const unsigned char *__res
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 const int v = v0 + 64 * g;
-                if (v >= nvec) break;
-                // the vector's seen bytes in one LDS read (most vectors receive no record)
-                union {
-                    MaskW w;
-                    uint8_t b[PPV];
-                } sw;
-                sw.w = ((const MaskW *)seen)[v];
-                bool any = false;
-#pragma unroll
-                for (int x = 0; x < PPV; ++x) any = any || sw.b[x] != 0;
-                if (any) {
+                if (!need[g]) continue;
+                if (any[g]) {
 #pragma unroll
                     for (int x = 0; x < PPV; ++x) {
-                        if (sw.b[x]) {
+                        if (sw[g].b[x]) {
                             const int s = v * PPV + x;
                             T o = u[g].t[x];
                             fold_old<T>(op, ((const T *)vals)[s], am[s], &o, om[g].b[x], bgv);
@@ -1143,12 +1148,15 @@ __device__ inline void write_fold_prop(int op, T bgv, const unsigned char *__res
                         }
                     }
                 }
-                __builtin_nontemporal_store(u[g].q, (v4u *)dst + v);
+                // a lone vector of a line goes through the caches, a whole chunk past them
+                if (OLD && inplace) ((v4u *)dst)[v] = u[g].q;
+                else __builtin_nontemporal_store(u[g].q, (v4u *)dst + v);
             }
         }
         return;
     }
     for (int s = lane; s < csz; s += 64) {
+        if (OLD && inplace && !seen[s]) continue;
         T o = OLD ? src[s] : bgv;
         if (seen[s]) fold_old<T>(op, ((const T *)vals)[s], am[s], &o, OLD ? smask[s] : (uint8_t)0, bgv);
         dst[s] = o;
@@ -1169,7 +1177,9 @@ __device__ inline uint32_t exist_byte(uint64_t row)
 // LDS; each lane's record is applied to the LDS state of its slot, records of one batch
 // that share a slot in lane order (one rank per round: ranks come from ballots over the
 // slot bits).  Then every array of the chunk is combined with the chunk's old contents
-// and written once, contiguously.
+// and written once, contiguously.  Where the chunk set did not grow the chunk stays in
+// place, and only the 16-byte vectors a record reached are read and written (the records
+// of fold_few_records_kernel's figures took 114 us with every chunk written whole, 101 us so).
 template <int NV>
 __global__ __launch_bounds__(256) void fold_chunk_records_kernel(const uint4 *__restrict__ rec,
                                                                  const uint32_t *__restrict__ ustart,
@@ -1179,117 +1189,126 @@ __global__ __launch_bounds__(256) void fold_chunk_records_kernel(const uint4 *__
                                                                  int csz, int obits, int waves, FoldState S,
                                                                  FoldProps F, RecLayout R, FusedImg I,
                                                                  uint8_t *__restrict__ omask, int skip_fresh,
-                                                                 uint64_t *__restrict__ eb)
+                                                                 uint64_t *__restrict__ eb,
+                                                                 const uint32_t *__restrict__ list)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_fold[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (w >= waves) return;  // waves are independent: no workgroup barrier
-    const int64_t j = (int64_t)blockIdx.x * waves + w;
-    if (j >= nnew) return;
-    if (skip_fresh && isnew[j] != 0) return;  // folded by fold_fresh_chunks_kernel
-    unsigned char *st = smem_fold + (size_t)w * S.bytes;
-    uint8_t *seen = st, *am = st + csz;
-    uint4 *stage = (uint4 *)(st + S.roff);  // the batch's records, lane l at stage[l * NV]
-    const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-    const uint32_t r0 = ustart[j], r1 = ustart[j + 1];
-    uint4 nxt[NV];
+    // the chunks of the list (list[0] of them, behind it), or every touched chunk
+    const int64_t todo = list ? (int64_t)list[0] : nnew;
+    for (int64_t at = (int64_t)blockIdx.x * waves + w; at < todo; at += (int64_t)gridDim.x * waves) {
+        const int64_t j = list ? (int64_t)list[1 + at] : at;
+        if (skip_fresh && isnew[j] != 0) continue;  // folded by fold_fresh_chunks_kernel
+        wave_sync_lds();  // the previous chunk's state is no longer read
+        unsigned char *st = smem_fold + (size_t)w * S.bytes;
+        uint8_t *seen = st, *am = st + csz;
+        uint4 *stage = (uint4 *)(st + S.roff);  // the batch's records, lane l at stage[l * NV]
+        const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+        const uint32_t r0 = ustart[j], r1 = ustart[j + 1];
+        uint4 nxt[NV];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) nxt[v] = (r0 + lane < r1) ? rec[(size_t)(r0 + lane) * NV + v] : make_uint4(0, 0, 0, 0);
-    {
-        const bool fresh = isnew[j] != 0;
-        const int64_t src = fresh ? 0 : oldpos[j], dst = cpos[j];
-        if (csz % 16 == 0) {
-            for (int v = lane; v < csz / 16; v += 64) ((uint4 *)seen)[v] = make_uint4(0, 0, 0, 0);
-        } else {
-            for (int s = lane; s < csz; s += 64) seen[s] = 0;
-        }
-        for (uint32_t b0 = r0; b0 < r1; b0 += 64) {
-            const uint32_t k = b0 + (uint32_t)lane;
-            const bool valid = k < r1;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) stage[lane * NV + v] = nxt[v];
-            // the next 64 records of the chunk, in flight while these are folded
-            const uint32_t kn = k + 64;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) nxt[v] = (kn < r1) ? rec[(size_t)kn * NV + v] : make_uint4(0, 0, 0, 0);
-            wave_sync_lds();
-            const unsigned char *rp = (const unsigned char *)(stage + lane * NV);
-            const int off = valid ? (int)*(const uint16_t *)rp : 0;
-            const uint8_t bm = rp[2];
-            uint64_t peers = __ballot(valid);
-            for (int b = 0; b < obits; ++b) {
-                const bool bit = (off >> b) & 1;
-                const uint64_t bal = __ballot(bit);
-                peers &= bit ? bal : ~bal;
+        for (int v = 0; v < NV; ++v) nxt[v] = (r0 + lane < r1) ? rec[(size_t)(r0 + lane) * NV + v] : make_uint4(0, 0, 0, 0);
+        {
+            const bool fresh = isnew[j] != 0;
+            const int64_t src = fresh ? 0 : oldpos[j], dst = cpos[j];
+            if (csz % 16 == 0) {
+                for (int v = lane; v < csz / 16; v += 64) ((uint4 *)seen)[v] = make_uint4(0, 0, 0, 0);
+            } else {
+                for (int s = lane; s < csz; s += 64) seen[s] = 0;
             }
-            const int rank = valid ? (int)__popcll(peers & lt) : -1;
-            int maxr = 0;
-            while (__ballot(rank > maxr) != 0) ++maxr;
-            // the mask pass, rank by rank: whether the record is its slot's first and the OR
-            // of the masks of the slot's earlier records
-            bool first = false;
-            uint8_t ao = 0;
-            for (int r = 0; r <= maxr; ++r) {
-                if (rank == r) {
-                    first = seen[off] == 0;
-                    ao = first ? (uint8_t)0 : am[off];
-                    am[off] = (uint8_t)(ao | bm);
-                    seen[off] = 0xff;
-                }
+            for (uint32_t b0 = r0; b0 < r1; b0 += 64) {
+                const uint32_t k = b0 + (uint32_t)lane;
+                const bool valid = k < r1;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) stage[lane * NV + v] = nxt[v];
+                // the next 64 records of the chunk, in flight while these are folded
+                const uint32_t kn = k + 64;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) nxt[v] = (kn < r1) ? rec[(size_t)kn * NV + v] : make_uint4(0, 0, 0, 0);
                 wave_sync_lds();
+                const unsigned char *rp = (const unsigned char *)(stage + lane * NV);
+                const int off = valid ? (int)*(const uint16_t *)rp : 0;
+                const uint8_t bm = rp[2];
+                uint64_t peers = __ballot(valid);
+                for (int b = 0; b < obits; ++b) {
+                    const bool bit = (off >> b) & 1;
+                    const uint64_t bal = __ballot(bit);
+                    peers &= bit ? bal : ~bal;
+                }
+                const int rank = valid ? (int)__popcll(peers & lt) : -1;
+                int maxr = 0;
+                while (__ballot(rank > maxr) != 0) ++maxr;
+                // the mask pass, rank by rank: whether the record is its slot's first and the OR
+                // of the masks of the slot's earlier records
+                bool first = false;
+                uint8_t ao = 0;
+                for (int r = 0; r <= maxr; ++r) {
+                    if (rank == r) {
+                        first = seen[off] == 0;
+                        ao = first ? (uint8_t)0 : am[off];
+                        am[off] = (uint8_t)(ao | bm);
+                        seen[off] = 0xff;
+                    }
+                    wave_sync_lds();
+                }
+                // the values, property by property (type and operator dispatched once per batch)
+                for (int q = 0; q < F.np; ++q) {
+                    unsigned char *vals = st + S.voff[q];
+                    const unsigned char *bp = rp + R.off[q];
+                    const int op = F.op[q];
+                    switch (F.dt[q]) {
+#define SG_CASE(CODE, T)                                                                                        \
+        case CODE: fold_batch_prop<T>(op, vals, bp, off, rank, maxr, first, ao, bm); break;
+                        SG_FOLD_TYPES(SG_CASE)
+#undef SG_CASE
+                    }
+                }
             }
-            // the values, property by property (type and operator dispatched once per batch)
+            const uint8_t *smask = fresh ? nullptr : I.smask + src * csz;
+            const bool inplace = !fresh && I.smask == omask && src == dst;
             for (int q = 0; q < F.np; ++q) {
-                unsigned char *vals = st + S.voff[q];
-                const unsigned char *bp = rp + R.off[q];
-                const int op = F.op[q];
+                const size_t cb = (size_t)csz * F.ts[q];
+                const unsigned char *sp = fresh ? nullptr : I.src[q] + src * cb;
+                unsigned char *dp = F.out[q] + dst * cb;
                 switch (F.dt[q]) {
 #define SG_CASE(CODE, T)                                                                                        \
-    case CODE: fold_batch_prop<T>(op, vals, bp, off, rank, maxr, first, ao, bm); break;
+        case CODE: {                                                                                                \
+            T bgv;                                                                                                  \
+            __builtin_memcpy(&bgv, &F.bg[q], sizeof(T));                                                            \
+            if (fresh)                                                                                              \
+                write_fold_prop<T, false>(F.op[q], bgv, st + S.voff[q], seen, am, nullptr, nullptr, (T *)dp, csz, lane); \
+            else                                                                                                    \
+                write_fold_prop<T, true>(F.op[q], bgv, st + S.voff[q], seen, am, (const T *)sp, smask, (T *)dp, csz,  \
+                                         lane, inplace);                                                            \
+            break;                                                                                                  \
+        }
                     SG_FOLD_TYPES(SG_CASE)
 #undef SG_CASE
                 }
             }
-        }
-        const uint8_t *smask = fresh ? nullptr : I.smask + src * csz;
-        for (int q = 0; q < F.np; ++q) {
-            const size_t cb = (size_t)csz * F.ts[q];
-            const unsigned char *sp = fresh ? nullptr : I.src[q] + src * cb;
-            unsigned char *dp = F.out[q] + dst * cb;
-            switch (F.dt[q]) {
-#define SG_CASE(CODE, T)                                                                                        \
-    case CODE: {                                                                                                \
-        T bgv;                                                                                                  \
-        __builtin_memcpy(&bgv, &F.bg[q], sizeof(T));                                                            \
-        if (fresh)                                                                                              \
-            write_fold_prop<T, false>(F.op[q], bgv, st + S.voff[q], seen, am, nullptr, nullptr, (T *)dp, csz, lane); \
-        else                                                                                                    \
-            write_fold_prop<T, true>(F.op[q], bgv, st + S.voff[q], seen, am, (const T *)sp, smask, (T *)dp, csz,  \
-                                     lane);                                                                     \
-        break;                                                                                                  \
-    }
-                SG_FOLD_TYPES(SG_CASE)
-#undef SG_CASE
-            }
-        }
-        // the mask: old | OR of the records
-        uint8_t *dm = omask + dst * csz;
-        if (csz % 16 == 0) {
-            typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-            for (int v = lane; v < csz / 16; v += 64) {
-                v4u q = smask ? ((const v4u *)smask)[v] : (v4u){0u, 0u, 0u, 0u};
-                // seen bytes are 0 or 0xff: the OR of the records' masks where a record came
-                q |= ((const v4u *)am)[v] & ((const v4u *)seen)[v];
-                __builtin_nontemporal_store(q, (v4u *)dm + v);
-                if (eb) {
-                    // 8^3 chunks: the vector holds rows 2v and 2v + 1, whose EXIST bits are
-                    // bytes 2v and 2v + 1 of the chunk's 64 plane bytes
-                    const uint64_t lo = ((uint64_t)q.y << 32) | q.x, hi = ((uint64_t)q.w << 32) | q.z;
-                    ((uint16_t *)eb)[dst * 32 + v] = (uint16_t)(exist_byte(lo) | (exist_byte(hi) << 8));
+            // the mask: old | OR of the records
+            uint8_t *dm = omask + dst * csz;
+            if (csz % 16 == 0) {
+                typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+                for (int v = lane; v < csz / 16; v += 64) {
+                    const v4u sn = ((const v4u *)seen)[v];
+                    if (inplace && (sn.x | sn.y | sn.z | sn.w) == 0u) continue;
+                    v4u q = smask ? ((const v4u *)smask)[v] : (v4u){0u, 0u, 0u, 0u};
+                    // seen bytes are 0 or 0xff: the OR of the records' masks where a record came
+                    q |= ((const v4u *)am)[v] & sn;
+                    if (inplace) ((v4u *)dm)[v] = q;
+                    else __builtin_nontemporal_store(q, (v4u *)dm + v);
+                    if (eb) {
+                        // 8^3 chunks: the vector holds rows 2v and 2v + 1, whose EXIST bits are
+                        // bytes 2v and 2v + 1 of the chunk's 64 plane bytes
+                        const uint64_t lo = ((uint64_t)q.y << 32) | q.x, hi = ((uint64_t)q.w << 32) | q.z;
+                        ((uint16_t *)eb)[dst * 32 + v] = (uint16_t)(exist_byte(lo) | (exist_byte(hi) << 8));
+                    }
                 }
+            } else {
+                for (int s = lane; s < csz; s += 64) dm[s] = (uint8_t)((smask ? smask[s] : 0) | (seen[s] ? am[s] : 0));
             }
-        } else {
-            for (int s = lane; s < csz; s += 64) dm[s] = (uint8_t)((smask ? smask[s] : 0) | (seen[s] ? am[s] : 0));
         }
     }
 }
@@ -1550,6 +1569,141 @@ __global__ __launch_bounds__(256) void fold_fresh_chunks_kernel(const uint4 *__r
         const v4u *s = (const v4u *)mimg;
         v4u *d = (v4u *)(omask + dst * csz);
         for (int v = lane; v < csz / 16; v += 64) __builtin_nontemporal_store(s[v], d + v);
+    }
+}
+
+// ---- fold of a few records into old chunks, in place ---------------------------------
+// Touched chunks with at most kFewRecords records: 8 lanes per chunk, a record per lane, no
+// LDS.  The first lane of a slot folds the later records of that slot in lane (= insertion)
+// order from the other lanes' registers, then the old value, and writes the slot's values
+// and mask.  Chunks with more records go to the list (list[0]: their number, zero on
+// entry) for fold_chunk_records_kernel; new chunks are the fresh fold's.  The chunk arrays
+// hold the old contents at the chunks' final positions.
+// A wave per chunk with 2 or 3 records spends its time on a chain of six dependent loads
+// and LDS steps (200,000 records, mostly 1 to 4 a chunk, two 4-byte properties: 101 us);
+// here a wave takes 8 chunks through a chain of four loads: 43 us, and 23 us for the chunks
+// of the list.
+constexpr int kFewRecords = 8;
+
+template <typename T> __device__ inline T bits_to(uint64_t u)
+{
+    T t;
+    __builtin_memcpy(&t, &u, sizeof(T));
+    return t;
+}
+
+template <int NV, int NP>
+__global__ __launch_bounds__(256) void fold_few_records_kernel(const uint4 *__restrict__ rec,
+                                                               const uint32_t *__restrict__ ustart,
+                                                               const int64_t *__restrict__ cpos,
+                                                               const uint32_t *__restrict__ isnew, int64_t nnew, int csz,
+                                                               FoldProps F, RecLayout R, uint8_t *__restrict__ mask,
+                                                               uint32_t *__restrict__ eb, uint32_t *__restrict__ list)
+{
+    constexpr int L = kFewRecords;
+    const int np = NP > 0 ? NP : F.np;
+    const int lane = threadIdx.x & 63, i = lane & (L - 1), first = lane & ~(L - 1);
+    const int64_t j = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
+    uint32_t r0 = 0, len = 0;
+    if (j < nnew && isnew[j] == 0) {
+        r0 = ustart[j];
+        len = ustart[j + 1] - r0;
+        if (len > (uint32_t)L) {
+            if (i == 0) list[1 + atomicAdd(list, 1u)] = (uint32_t)j;
+            len = 0;
+        }
+    }
+    if (__ballot(len != 0) == 0) return;
+    const bool valid = (uint32_t)i < len;
+    uint4 rr[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) rr[v] = valid ? rec[(size_t)(r0 + i) * NV + v] : make_uint4(0, 0, 0, 0);
+    const int64_t base = len ? cpos[j] * csz : 0;
+    // slot and mask of the lane's record; slot 0xffff: none
+    const uint32_t key = valid ? (rr[0].x & 0xffffffu) : 0xffffu;
+    const uint32_t off = key & 0xffffu;
+    int longest = 1;
+    while (longest < L && __ballot(len > (uint32_t)longest) != 0) ++longest;
+    // same: the lanes of the chunk with a record of the slot; am: the OR of the masks
+    uint32_t same = 0, am = 0;
+    uint64_t masks = 0;  // byte k: lane k's record's mask
+    for (int k = 0; k < longest; ++k) {
+        const uint32_t o = (uint32_t)__shfl((int)key, first + k, 64);
+        if ((o & 0xffffu) == off) {
+            same |= 1u << k;
+            am |= o >> 16;
+        }
+        masks |= (uint64_t)(o >> 16) << (8 * k);
+    }
+    const bool lead = valid && (same & ((1u << i) - 1u)) == 0;
+    const int64_t slot = base + (lead ? off : 0);
+    // the old mask and values, all loaded before the first is folded
+    const uint8_t om = lead ? mask[slot] : (uint8_t)0;
+    uint64_t old[NP > 0 ? NP : 1];
+    auto load_old = [&](int q) -> uint64_t {
+        const unsigned char *p = F.out[q];
+        switch (F.ts[q]) {
+        case 8: return ((const uint64_t *)p)[slot];
+        case 4: return ((const uint32_t *)p)[slot];
+        case 2: return ((const uint16_t *)p)[slot];
+        default: return p[slot];
+        }
+    };
+    if constexpr (NP > 0) {
+#pragma unroll
+        for (int q = 0; q < NP; ++q) old[q] = lead ? load_old(q) : 0ull;
+    }
+    auto fold_prop = [&](int q) {
+        const int op = F.op[q];
+        switch (F.dt[q]) {
+#define SG_CASE(CODE, T)                                                                                        \
+    case CODE: {                                                                                                \
+        T bgv;                                                                                                  \
+        __builtin_memcpy(&bgv, &F.bg[q], sizeof(T));                                                            \
+        const T own = rec_value<T, NV>(rr, R.off[q]);                                                           \
+        T a = own;                                                                                              \
+        uint32_t ao = key >> 16;                                                                                \
+        for (int k = 1; k < longest; ++k) {                                                                     \
+            T b;                                                                                                \
+            if constexpr (sizeof(T) == 8) {                                                                     \
+                uint64_t u;                                                                                     \
+                __builtin_memcpy(&u, &own, 8);                                                                  \
+                const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)u, first + k, 64);                          \
+                const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(u >> 32), first + k, 64);                  \
+                b = bits_to<T>((uint64_t)lo | ((uint64_t)hi << 32));                                            \
+            } else {                                                                                            \
+                uint32_t u = 0;                                                                                 \
+                __builtin_memcpy(&u, &own, sizeof(T));                                                          \
+                b = bits_to<T>((uint64_t)(uint32_t)__shfl((int)u, first + k, 64));                              \
+            }                                                                                                   \
+            if (k > i && ((same >> k) & 1u)) {                                                                  \
+                const uint32_t bm = (uint32_t)(masks >> (8 * k)) & 0xffu;                                       \
+                const bool aE = ao & 1u, bE = bm & 1u;                                                          \
+                if (op == SG_OP_NONE) a = bE ? b : a;                                                           \
+                else if (aE && bE) a = dev_reduce<T>(op, a, b);                                                 \
+                else if (bE) a = b;                                                                             \
+                ao |= bm;                                                                                       \
+            }                                                                                                   \
+        }                                                                                                       \
+        if (lead) {                                                                                             \
+            uint64_t raw;                                                                                       \
+            if constexpr (NP > 0) raw = old[q];                                                                 \
+            else raw = load_old(q);                                                                             \
+            T o = bits_to<T>(raw);                                                                              \
+            fold_old<T>(op, a, (uint8_t)am, &o, om, bgv);                                                       \
+            ((T *)F.out[q])[slot] = o;                                                                          \
+        }                                                                                                       \
+        break;                                                                                                  \
+    }
+            SG_FOLD_TYPES(SG_CASE)
+#undef SG_CASE
+        }
+    };
+    for_props<NP>(np, fold_prop);
+    if (lead) {
+        mask[slot] = (uint8_t)(om | am);
+        // 8^3 chunks: the slot's bit of the EXIST bit-planes (bit slot % 32 of word slot / 32)
+        if (eb && (am & 1u) && !(om & 1u)) atomicOr(eb + (slot >> 5), 1u << (slot & 31));
     }
 }
 
@@ -2205,6 +2359,8 @@ struct MergeDefer {
     const int64_t *oldpos = nullptr;  // [nnew] old position of each touched chunk
     const uint32_t *isnew = nullptr;  // [nnew] 1: brand-new chunk
     int64_t nfresh = 0;               // brand-new chunks among the nnew
+    // in: the touched old chunks move with the others (the fold then works in place)
+    bool copy_touched = false;
     // in: keep the EXIST bit-planes (8^3 chunks) through the merge, the caller's fold
     // writing those of the touched chunks; out: false when they could not be kept
     bool planes = false;
@@ -2344,12 +2500,12 @@ int merge_grow(sg_grid *g, const MergeLookup &L, int64_t nnew, int64_t nb, int64
         } else if (flat) {
             uint8_t *skip = nullptr;
             if (df) {
-                // the touched chunks are written whole by the caller's fused fold
+                // the touched chunks (or only the new ones) are written whole by the caller's fold
                 skip = (uint8_t *)(src_of + (m + nb));
                 hipLaunchKernelGGL(fill_u8_kernel, dim3(grid_1d(total, kWG)), dim3(kWG), 0, g->stream, skip, (uint8_t)0,
                                    total);
                 hipLaunchKernelGGL(mark_positions_kernel, dim3(grid_1d(nnew, kWG)), dim3(kWG), 0, g->stream, cpos,
-                                   nnew, skip);
+                                   nnew, skip, df->copy_touched ? isnew : nullptr);
                 SG_HIP(hipGetLastError());
             }
             hipLaunchKernelGGL(build_union_kernel, dim3(2048), dim3(kWG), 0, g->stream, U, src_of, total + 1, skip);
@@ -2651,6 +2807,11 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
     // 8^3 chunks: the EXIST bit-planes are kept up to date when they are valid (or the
     // grid has no chunk yet): the fold writes those of the touched chunks
     df.planes = g->dim == 3 && g->edge == 8 && (g->ebits_valid || g->nchunks == 0);
+    // few records a touched chunk (8 on average at most) and old chunks among them: those are
+    // folded slot by slot in place, after the old chunks have moved if the set grows.  With more
+    // records a chunk a wave per chunk reads and writes it whole at the copy's rate.
+    const bool few = n <= kFewRecords * nnew && (int64_t)hw[0] < nnew && ((csz % 16) == 0 || hw[0] == 0);
+    df.copy_touched = few;
     int64_t *cpos = nullptr;
     if ((rc = merge_grow(g, ML, nnew, hw[0], &cpos, &df))) return rc;
     const bool planes = df.planes;
@@ -2666,6 +2827,11 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
     // brand-new chunks: folded in an image of the chunk (csz % 16 == 0, image <= 64 KB)
     FreshArgs A;
     bool fresh_ok = (csz % 16) == 0 && df.nfresh > 0;
+    if (few) {
+        // the old contents are at the final positions
+        I.smask = g->d_mask;
+        for (int p = 0; p < g->np; ++p) I.src[p] = F.out[p];
+    }
     {
         size_t at = 0;
         A.np = g->np;
@@ -2719,21 +2885,52 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
         }
         SG_HIP(hipGetLastError());
     }
+    const bool use_few = few && (df.nfresh == 0 || fresh_ok);
+    uint32_t *list = nullptr;
+    if (use_few) {
+        if ((rc = ensure(g->pool, g->scratch[8], (size_t)(nnew + 1) * 4))) return rc;
+        list = (uint32_t *)g->scratch[8].p;
+        hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(1), dim3(64), 0, g->stream, list, 0u, (int64_t)1);
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(grid_1d(nnew, 256 / kFewRecords)), dim3(256), 0, g->stream, rec, ustart, cpos,
+                               df.isnew, nnew, csz, F, R, g->d_mask, (uint32_t *)eb, list);
+        };
+        if (R.nv == 1) {
+            switch (g->np) {
+            case 1: launch(fold_few_records_kernel<1, 1>); break;
+            case 2: launch(fold_few_records_kernel<1, 2>); break;
+            case 3: launch(fold_few_records_kernel<1, 3>); break;
+            case 4: launch(fold_few_records_kernel<1, 4>); break;
+            default: launch(fold_few_records_kernel<1, 0>); break;
+            }
+        } else {
+            switch (g->np) {
+            case 1: launch(fold_few_records_kernel<2, 1>); break;
+            case 2: launch(fold_few_records_kernel<2, 2>); break;
+            case 3: launch(fold_few_records_kernel<2, 3>); break;
+            case 4: launch(fold_few_records_kernel<2, 4>); break;
+            default: launch(fold_few_records_kernel<2, 0>); break;
+            }
+        }
+        SG_HIP(hipGetLastError());
+    }
     if (!fresh_ok || df.nfresh < nnew) {
         // chunks that existed before (and new ones when the image path is not taken)
         const int waves = std::max(1, std::min(4, 65536 / S.bytes));
         // one wave per touched chunk (a wave's loop then runs once)
-        const int64_t groups = (nnew + waves - 1) / waves;
+        // (with a list: at most n / (kFewRecords + 1) chunks are on it, waves loop over it)
+        const int64_t most = list ? std::min<int64_t>(2048 * waves, n / (kFewRecords + 1) + 1) : nnew;
+        const int64_t groups = (most + waves - 1) / waves;
         const dim3 fgrid((unsigned)groups), fblk(64 * waves);
         const int skip_fresh = fresh_ok ? 1 : 0;
         if (R.nv == 1)
             hipLaunchKernelGGL(fold_chunk_records_kernel<1>, fgrid, fblk, (size_t)waves * S.bytes, g->stream, rec,
-                               ustart, cpos, df.oldpos, df.isnew, nnew, csz, obits, waves, S, F, R, I, g->d_mask,
-                               skip_fresh, eb);
+                               ustart, cpos, few ? cpos : df.oldpos, df.isnew, nnew, csz, obits, waves, S, F, R, I,
+                               g->d_mask, skip_fresh, eb, (const uint32_t *)list);
         else
             hipLaunchKernelGGL(fold_chunk_records_kernel<2>, fgrid, fblk, (size_t)waves * S.bytes, g->stream, rec,
-                               ustart, cpos, df.oldpos, df.isnew, nnew, csz, obits, waves, S, F, R, I, g->d_mask,
-                               skip_fresh, eb);
+                               ustart, cpos, few ? cpos : df.oldpos, df.isnew, nnew, csz, obits, waves, S, F, R, I,
+                               g->d_mask, skip_fresh, eb, (const uint32_t *)list);
         SG_HIP(hipGetLastError());
     }
     finish_merge(g, df);

@@ -1032,3 +1032,51 @@ def test_flush_known_answers_of_the_reference(G):
     with old data, merge maps, conflict resolution), end to end through insert + flush on
     the GPU, against the transcribed answers."""
     S.check_flush_known_answers(G)
+
+
+@pytest.mark.parametrize("dim,edge,grow", [(3, 8, False), (3, 8, True), (2, 16, True), (3, 4, False), (3, 5, False),
+                                           (2, 6, True)])
+@pytest.mark.parametrize("dtypes", [[np.int32, np.float32], [np.float64, np.uint16, np.int8], [np.uint8],
+                                    [np.float64, np.int64, np.uint32], [np.int16, np.uint8, np.int8, np.uint16, np.float32]])
+def test_flush_few_records_per_chunk(G, oracle, dim, edge, grow, dtypes):
+    """A few records a touched chunk, folded slot by slot in place: runs of 1 to 8 records and
+    of 9 and 30 (the per-chunk kernel's, by list), duplicates, masks 0 to 3, every operator;
+    into chunks that exist, and with new ones among them; the EXIST planes kept or stale."""
+    rng = np.random.default_rng(edge * 10 + len(dtypes))
+    size = [6 * edge + 1] * dim
+    cs = edge ** dim
+    nchunk = int(np.prod([-(-s // edge) for s in size]))
+    old = np.sort(rng.choice(nchunk, nchunk if not grow else nchunk // 2, replace=False)).astype(np.int64)
+    steps = []
+    keys = (np.repeat(old, 12) * cs + rng.integers(0, cs, 12 * len(old))).astype(np.int64)
+    steps.append((keys, ["smax"] * len(dtypes)))
+    for f in range(4):
+        touched = rng.choice(nchunk if grow else old, max(4, nchunk // 3), replace=False).astype(np.int64)
+        runs = rng.integers(1, 5, len(touched))
+        runs[:4] = [8, 9, 30, 7]
+        slots = rng.integers(0, max(2, cs // 8), int(runs.sum()))  # few slots: duplicates
+        keys = np.repeat(touched, runs) * cs + slots
+        ops = [str(rng.choice(["smax", "smin", "sadd", "sright", "sleft", "none"] +
+                              (["sor"] if np.issubdtype(dt, np.integer) else []))) for dt in dtypes]
+        steps.append((keys[rng.permutation(len(keys))], ops))
+    gs = []
+    for cls in (G, oracle.SparseGridCpu):
+        r = np.random.default_rng(3)
+        g = cls(dim, size, dtypes, block_edge=edge)
+        for p in range(len(dtypes)):
+            g.set_background_value(p, p + 1)
+        for k, (keys, ops) in enumerate(steps):
+            vals = [S._rand_vals(r, dt, len(keys)) for dt in dtypes]
+            g.insert(keys, vals, r.choice(np.array([1, 1, 1, 3, 2, 0], np.uint8), len(keys)))
+            g.flush(ops)
+            if cls is G and k == 3:
+                g.device_ptr(-1)  # planes stale from here on
+            if k != 2:
+                g.tag_boundaries(C.NN_STAR)
+        gs.append(g)
+    S.assert_same_state(gs[0], gs[1])
+    a = gs[0]
+    assert a.count_existing_elements() == gs[1].count_existing_elements()
+    m = a.masks()
+    for p in range(len(dtypes)):
+        assert (a.prop(p)[m == 0] == p + 1).all()
