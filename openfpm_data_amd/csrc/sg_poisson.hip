@@ -41,7 +41,21 @@ struct PGrid {
     double omega;
     int64_t n;            // chunks
     int32_t nsweeps;      // sweeps of this grid in the current inner block
+    // fused sweeps (mixed form): x's second buffer, the chunks' 18 neighbours, and whether both
+    // are still to be set up
+    float *x2;
+    int32_t *nb;
+    int32_t prep;
 };
+
+// A pointer of a grid descriptor in memory, read as one into global memory: as far as the
+// compiler knows a plain one may point anywhere, and its accesses become flat ones, which
+// also count as LDS accesses, wait for them, and take 64-bit addresses per lane.
+template <typename T> __device__ __forceinline__ T *as_global(T *const &field)
+{
+    typedef __attribute__((address_space(1))) T *G;
+    return (T *)*(const G *)&field;
+}
 
 template <typename T> struct R8 {
     T v[8];
@@ -137,11 +151,11 @@ __device__ inline void neighbour_rows(const T *tile, int lane, R8<T> &ym, R8<T> 
 // rows are stored; values of the other colour are written back unchanged (no other wave
 // changes them in this half sweep).
 template <typename T>
-__device__ inline void sweep_tile(const PGrid &g, int64_t c, T *tile, int lane, int color, int zero_x)
+__device__ __forceinline__ void sweep_tile(const PGrid &g, int64_t c, T *tile, int lane, int color, int zero_x)
 {
-    T *x = (T *)g.x;
-    const T *rhs = (const T *)g.rhs;
-    const uint64_t mrow = *(const uint64_t *)(g.mask + c * 512 + lane * 8);
+    T *x = (T *)as_global(g.x);
+    const T *rhs = (const T *)as_global(g.rhs);
+    const uint64_t mrow = *(const uint64_t *)(as_global(g.mask) + c * 512 + lane * 8);
     R8<T> b;
     ld8(b, rhs + c * 512 + lane * 8);
     R8<T> own, ym, yp, zm, zp;
@@ -151,7 +165,7 @@ __device__ inline void sweep_tile(const PGrid &g, int64_t c, T *tile, int lane, 
         for (int i = 0; i < 8; ++i) own.v[i] = ym.v[i] = yp.v[i] = zm.v[i] = zp.v[i] = (T)0;
     } else {
         int64_t nbp[6];
-        const int32_t *row = g.nn + c * 8;
+        const int32_t *row = as_global(g.nn) + c * 8;
 #pragma unroll
         for (int k = 0; k < 6; ++k) nbp[k] = row[k];
         stage<T>(x, c, nbp, tile, lane, own, xm, xp);
@@ -210,6 +224,321 @@ __global__ __launch_bounds__(64 * WAVES) void rbsor_batch_kernel(const PGrid *__
     }
 }
 
+// ---- both colours of a sweep in one pass (FP32) ---------------------------------------
+// A half sweep reads and writes every value of x for an update of half of them, so a sweep
+// of two launches moves 26 B a slot.  Here a wave updates the first colour on its chunk and,
+// a second time, on the ring of first-colour points of the six neighbour chunks' faces,
+// which the chunk's second colour then uses: each value is computed from the same inputs by
+// the same operations as in the neighbour's own wave, so the iterates keep their bits.  The
+// ring's update needs a second layer of x, the ring's right-hand side and masks, and the
+// values beside it in the 12 edge neighbours (those at nb[6 ..]).  x alternates between two
+// buffers from sweep to sweep, the last sweep of a block writing the property (PGrid::x).
+// Moved: 13 B a slot plus the ring, which other waves load as well (cache hits mostly), and
+// half the launches.  The kernel is bound by instructions (about 400 vector ones a chunk,
+// against 2 x 363 of two half sweeps); before the rows were kept split by colour, with a
+// select for every operand, it had 680 and a sweep of 48 grids took 115 us.  Those 48 grids
+// (58,600 chunks): 2 x 64 us a sweep in half sweeps, 74 us here; 152 chunks 2 x 4.8 -> 4.3 us.
+// 4 waves a workgroup (1: 12.2 ms a solve of the 48 instead of 11.3); plain stores 11.9 ms;
+// registers for 5 waves a SIMD spill (14.2 ms).
+constexpr int kNb = 20;  // entries per chunk: -x +x -y +y -z +z, xy, xz, yz edges, 2 unused
+// LDS row of the 10 x 10 rows of a chunk and its ring: the 4 points of the first colour, the 4
+// of the second, then x = -1 and x = 8 at 8 and 9.  Point j of a colour is at x = 2 j + s, s
+// the row's parity for it; the rows above, below, before and behind have the other parity, so
+// their points j of the other colour are its neighbours there: a row is updated from one
+// 16-byte read of each of the four, with no selection.
+constexpr int kFS = 12;
+
+// neighbour tables and zeroed second buffers of the grids that joined the batch (one wave
+// per chunk): edge neighbour (a, b) is b's neighbour of a's neighbour, or where that is
+// missing a's of b's; the background chunk where neither exists
+__global__ __launch_bounds__(256) void fused_prep_kernel(const PGrid *__restrict__ grids,
+                                                         const int64_t *__restrict__ prefix,
+                                                         const int32_t *__restrict__ tile_grid, int64_t ntiles)
+{
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int64_t t = (int64_t)blockIdx.x * 4 + w;
+    if (t >= ntiles) return;
+    const int gi = tile_grid[t];
+    const PGrid &g = grids[gi];
+    if (!g.prep) return;
+    const int64_t c = t - prefix[gi];
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 *p = (float4 *)(g.x2 + c * 512);
+    p[lane] = zero;
+    p[64 + lane] = zero;
+    if (c == 0) {
+        float4 *b = (float4 *)(g.x2 + g.n * 512);
+        b[lane] = zero;
+        b[64 + lane] = zero;
+    }
+    if (lane >= kNb) return;
+    int32_t v = (int32_t)g.n;
+    if (lane < 6) {
+        v = g.nn[c * 8 + lane];
+    } else if (lane < 18) {
+        const int k = (lane - 6) >> 2, q = (lane - 6) & 3;
+        const int a = (k == 2 ? 2 : 0) + (q & 1), b = (k == 0 ? 2 : 4) + (q >> 1);
+        const int32_t na = g.nn[c * 8 + a], nc = g.nn[c * 8 + b];
+        if (na != v) v = g.nn[(int64_t)na * 8 + b];
+        else if (nc != v) v = g.nn[(int64_t)nc * 8 + a];
+    }
+    g.nb[c * kNb + lane] = v;
+}
+
+__device__ __forceinline__ float sel(bool m, float a, float b) { return m ? a : b; }
+
+// a / 6 correctly rounded: with y the rounded 1 / 6 (off by 2^-25 of it), a y is within one
+// unit in the last place of a / 6, its remainder a - 6 q is exact, and one correction by it
+// gives the rounded quotient (Markstein).  That needs a quotient in the normal range: *small
+// is set where it is subnormal, and the caller divides.  Zeros, infinities and NaN are the
+// fixup's.  5 instructions instead of 12.
+__device__ __forceinline__ float div6(float a, bool *small)
+{
+    const float y = 1.0f / 6.0f;
+    const float q = a * y;
+    const float r = __builtin_fmaf(-6.0f, q, a);
+    // class mask: negative and positive subnormals
+    *small = *small || __builtin_amdgcn_classf(q, (1 << 4) | (1 << 7));
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(r, y, q), 6.0f, a);
+}
+
+// x + w ((b + nbs) / 6 - x) as sweep_tile computes it, where the point is active (mask m);
+// EXACT: by true division
+template <bool EXACT>
+__device__ __forceinline__ float sor_value(float cur, float b, float px, float py, float pz, float wgt, uint32_t m,
+                                           bool *small)
+{
+    float nbs = 0.0f;
+    nbs = nbs + px;
+    nbs = nbs + py;
+    nbs = nbs + pz;
+    const float a = b + nbs;
+    const float gs = EXACT ? a / 6.0f : div6(a, small);
+    const float x = cur + wgt * (gs - cur);
+    return (m & (SG_EXIST | SG_PADDING)) == SG_EXIST ? x : cur;
+}
+
+// One colour on the lane's row: its points c[4], the other colour's o[4], the value end beside
+// the row that points of parity s have (x = 8 for s, else x = -1), the neighbour rows' points
+// of the other colour at p (LDS).  m: the row's masks.
+template <bool EXACT>
+__device__ __forceinline__ void sor_row(float (&c)[4], const float (&o)[4], const float (&b)[4], float end, bool s,
+                                        const float *p, uint64_t m, float wgt, bool *small)
+{
+    const float4 ym = *(const float4 *)(p - kFS), yp = *(const float4 *)(p + kFS);
+    const float4 zm = *(const float4 *)(p - 10 * kFS), zp = *(const float4 *)(p + 10 * kFS);
+    const uint64_t ms = s ? m >> 8 : m;
+    // l + r: o[j] on one side, o[j + 1] or o[j - 1] on the other
+    const float x0 = o[0] + sel(s, o[1], end), x1 = o[1] + sel(s, o[2], o[0]);
+    const float x2 = o[2] + sel(s, o[3], o[1]), x3 = o[3] + sel(s, end, o[2]);
+    const uint32_t m0 = (uint32_t)ms, m1 = (uint32_t)(ms >> 32);
+    c[0] = sor_value<EXACT>(c[0], b[0], x0, ym.x + yp.x, zm.x + zp.x, wgt, m0, small);
+    c[1] = sor_value<EXACT>(c[1], b[1], x1, ym.y + yp.y, zm.y + zp.y, wgt, m0 >> 16, small);
+    c[2] = sor_value<EXACT>(c[2], b[2], x2, ym.z + yp.z, zm.z + zp.z, wgt, m1, small);
+    c[3] = sor_value<EXACT>(c[3], b[3], x3, ym.w + yp.w, zm.w + zp.w, wgt, m1 >> 16, small);
+}
+
+// the points of parity s (first) and the others of 8 values
+__device__ __forceinline__ void split8(float (&a)[4], float (&b)[4], const R8<float> &v, bool s)
+{
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        a[j] = sel(s, v.v[2 * j + 1], v.v[2 * j]);
+        b[j] = sel(s, v.v[2 * j], v.v[2 * j + 1]);
+    }
+}
+
+template <typename V> __device__ __forceinline__ V ld_at(const void *base, uint32_t byte)
+{
+    return *(const V *)((const char *)base + byte);
+}
+
+// per-lane values of one chunk for both colours
+struct FusedIn {
+    uint64_t mrow;                    // masks of the row
+    float c0[4], c1[4], b0[4], b1[4]; // first and second colour of the row, their right-hand sides
+    float xmm, xm, xp, xpp;           // x = -2, -1, 8, 9 of the row
+    // the lane's half row of a y / z face of the ring: first colour, right-hand side, second
+    // layer (beside the first colour), second colour, masks
+    float2 r0, rb, rl, r1;
+    uint32_t rm;
+    float sb;     // right-hand side and mask of the ring's first-colour point beside the row
+    uint32_t sm;
+};
+
+// Everything after the loads: EXACT divides truly; otherwise *small asks for that.  c0 and c1
+// are updated.
+template <bool EXACT>
+__device__ __forceinline__ void fused_compute(FusedIn &in, float *tile, int lane, float wgt, bool *small)
+{
+    const int y = lane & 7, z = lane >> 3, face = lane >> 4, idx = (lane >> 1) & 7, half = lane & 1;
+    const bool s = ((y + z) & 1) != 0;
+    const int own = ((z + 1) * 10 + y + 1) * kFS, trow = g_tile_row(lane) * kFS;
+    const bool yface = face < 2, rs = ((idx + ((face & 1) ? 0 : 1)) & 1) != 0;
+    // the ring's half row
+    float2 rn;
+    {
+        const int inner = (yface ? (idx + 1) * 10 + (face == 0 ? 1 : 8) : (face == 2 ? 10 : 80) + idx + 1) * kFS;
+        const int d = (yface ? 10 : 1) * kFS, at = 4 + 2 * half;
+        const float2 ip = *(const float2 *)(tile + inner + at);
+        const float2 lo = *(const float2 *)(tile + trow - d + at), hi = *(const float2 *)(tile + trow + d + at);
+        // the second colour's point beyond the half row that its parity has as a neighbour
+        const float e = tile[trow + (rs ? (half ? 9 : 6) : (half ? 5 : 8))];
+        const float n0 = in.rl.x + ip.x, n1 = in.rl.y + ip.y, a0 = lo.x + hi.x, a1 = lo.y + hi.y;
+        rn.x = sor_value<EXACT>(in.r0.x, in.rb.x, in.r1.x + sel(rs, in.r1.y, e), sel(yface, n0, a0),
+                                sel(yface, a0, n0), wgt, rs ? in.rm >> 8 : in.rm, small);
+        rn.y = sor_value<EXACT>(in.r0.y, in.rb.y, in.r1.y + sel(rs, e, in.r1.x), sel(yface, n1, a1),
+                                sel(yface, a1, n1), wgt, rs ? in.rm >> 24 : in.rm >> 16, small);
+    }
+    // the ring's point beside the row: x = -1 for rows of parity s, else x = 8
+    const int sl = s ? 8 : 9;
+    const float py = tile[own - kFS + sl] + tile[own + kFS + sl];
+    const float pz = tile[own - 10 * kFS + sl] + tile[own + 10 * kFS + sl];
+    const float xn = sor_value<EXACT>(sel(s, in.xm, in.xp), in.sb, sel(s, in.xmm, in.xpp) + sel(s, in.c1[0], in.c1[3]),
+                                      py, pz, wgt, in.sm, small);
+    // the row: first-colour points of parity s end beside x = 8, the others beside x = -1
+    sor_row<EXACT>(in.c0, in.c1, in.b0, sel(s, in.xp, in.xm), s, tile + own + 4, in.mrow, wgt, small);
+    wave_sync_lds();
+    *(float4 *)(tile + own) = make_float4(in.c0[0], in.c0[1], in.c0[2], in.c0[3]);
+    *(float2 *)(tile + trow + 2 * half) = rn;
+    wave_sync_lds();
+    // second-colour points have the other parity: they end beside the updated ring point
+    sor_row<EXACT>(in.c1, in.c0, in.b1, xn, !s, tile + own, in.mrow, wgt, small);
+}
+
+// both colours on chunk c of grid g (fewer than 2^21 chunks: 32-bit byte offsets): src -> dst
+__device__ __forceinline__ void fused_tile(const PGrid &g, uint32_t c, float *tile, int lane, int zero_x,
+                                           const float *src, float *dst)
+{
+    const int32_t *nb = as_global(g.nb) + (size_t)c * kNb;
+    const float *rhs = (const float *)as_global(g.rhs);
+    const uint8_t *mask = as_global(g.mask);
+    const int y = lane & 7, z = lane >> 3, face = lane >> 4, idx = (lane >> 1) & 7, half = lane & 1;
+    const bool s = ((y + z) & 1) != 0, rs = ((idx + ((face & 1) ? 0 : 1)) & 1) != 0;
+    const int own = ((z + 1) * 10 + y + 1) * kFS, trow = g_tile_row(lane) * kFS;
+    // source rows of the ring's half row in the neighbour: first and second layer
+    const int row1 = g_src_row(lane);
+    const int row2 = face < 2 ? idx * 8 + (face == 0 ? 6 : 1) : (face == 2 ? 48 : 8) + idx;
+    const uint32_t n0 = (uint32_t)nb[0], n1 = (uint32_t)nb[1];
+    const uint32_t nf = (uint32_t)(face < 2 ? (face == 0 ? nb[2] : nb[3]) : (face == 2 ? nb[4] : nb[5]));
+    const uint32_t at = c * 2048u + (uint32_t)lane * 32u, atf = nf * 2048u + (uint32_t)half * 16u;
+    // the ring's first-colour point beside the row
+    const uint32_t side = (s ? n0 : n1) * 512u + (uint32_t)lane * 8u + (s ? 7u : 0u);
+
+    FusedIn in;
+    in.mrow = ld_at<uint64_t>(mask, c * 512u + (uint32_t)lane * 8u);
+    R8<float> b, u;
+    ld8(b, (const float *)((const char *)rhs + at));
+    const float4 bh = ld_at<float4>(rhs, atf + (uint32_t)row1 * 32u);
+    in.rm = ld_at<uint32_t>(mask, nf * 512u + (uint32_t)row1 * 8u + (uint32_t)half * 4u);
+    in.sb = ld_at<float>(rhs, side * 4u);
+    in.sm = mask[side];
+    float4 h1 = make_float4(0.f, 0.f, 0.f, 0.f), h2 = h1, ye = h1;
+    float2 xm = make_float2(0.f, 0.f), xp = xm;
+    float xe = 0.f;
+    // edge values: lanes (e, i) -> value i of xy / xz edge e, one each; lanes 0 - 7 -> half rows
+    // of the 4 yz edges
+    const int ek = lane >> 5, es = (lane >> 4) & 1, ex = (lane >> 3) & 1, ei = lane & 7;
+    const int erow = ek == 0 ? ei * 8 + (es ? 0 : 7) : (es ? 0 : 56) + ei;
+    const int etile = (ek == 0 ? (ei + 1) * 10 + (es ? 9 : 0) : (es ? 90 : 0) + ei + 1) * kFS;
+    const int ys = (lane >> 1) & 1, zs = (lane >> 2) & 1;
+    if (zero_x) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) u.v[i] = 0.f;
+    } else {
+        ld8(u, (const float *)((const char *)src + at));
+        h1 = ld_at<float4>(src, atf + (uint32_t)row1 * 32u);
+        h2 = ld_at<float4>(src, atf + (uint32_t)row2 * 32u);
+        xm = ld_at<float2>(src, n0 * 2048u + (uint32_t)lane * 32u + 24u);
+        xp = ld_at<float2>(src, n1 * 2048u + (uint32_t)lane * 32u);
+        const uint32_t ne = (uint32_t)(ek == 0 ? (es ? (ex ? nb[9] : nb[8]) : (ex ? nb[7] : nb[6]))
+                                               : (es ? (ex ? nb[13] : nb[12]) : (ex ? nb[11] : nb[10])));
+        xe = ld_at<float>(src, ne * 2048u + (uint32_t)(erow * 8 + (ex ? 0 : 7)) * 4u);
+        if (lane < 8) {
+            const uint32_t ny = (uint32_t)(zs ? (ys ? nb[17] : nb[16]) : (ys ? nb[15] : nb[14]));
+            ye = ld_at<float4>(src, ny * 2048u + (uint32_t)((zs ? 0 : 56) + (ys ? 0 : 7)) * 32u + (uint32_t)half * 16u);
+        }
+    }
+    split8(in.c0, in.c1, u, s);
+    split8(in.b0, in.b1, b, s);
+    in.xmm = xm.x;
+    in.xm = xm.y;
+    in.xp = xp.x;
+    in.xpp = xp.y;
+    in.r0 = make_float2(sel(rs, h1.y, h1.x), sel(rs, h1.w, h1.z));
+    in.r1 = make_float2(sel(rs, h1.x, h1.y), sel(rs, h1.z, h1.w));
+    in.rl = make_float2(sel(rs, h2.y, h2.x), sel(rs, h2.w, h2.z));
+    in.rb = make_float2(sel(rs, bh.y, bh.x), sel(rs, bh.w, bh.z));
+    // the first colour's update reads second-colour points only
+    *(float4 *)(tile + own + 4) = make_float4(in.c1[0], in.c1[1], in.c1[2], in.c1[3]);
+    *(float2 *)(tile + own + 8) = make_float2(in.xm, in.xp);
+    *(float2 *)(tile + trow + 4 + 2 * half) = in.r1;
+    tile[etile + 8 + ex] = xe;
+    if (lane < 8) {
+        const bool cs = ys != zs;  // parity of the edge row (y and z are -1 or 8)
+        *(float2 *)(tile + ((zs ? 90 : 0) + (ys ? 9 : 0)) * kFS + 4 + 2 * half) =
+            make_float2(sel(cs, ye.x, ye.y), sel(cs, ye.z, ye.w));
+    }
+    wave_sync_lds();
+
+    const float wgt = (float)g.omega;
+    bool small = false;
+    float k0[4], k1[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        k0[j] = in.c0[j];
+        k1[j] = in.c1[j];
+    }
+    fused_compute<false>(in, tile, lane, wgt, &small);
+    if (__ballot(small) != 0) {
+        // subnormal quotients somewhere in the chunk: again with true divisions.  The LDS rows'
+        // second-colour points are as they were, the first colour's are rewritten.
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            in.c0[j] = k0[j];
+            in.c1[j] = k1[j];
+        }
+        wave_sync_lds();
+        fused_compute<true>(in, tile, lane, wgt, &small);
+    }
+    const uint64_t rows = __ballot(in.mrow != 0);
+    wave_sync_lds();
+    // back in row order, and out as lane-contiguous 16-byte stores of the rows with a point
+    *(float4 *)(tile + lane * 8) = make_float4(sel(s, in.c1[0], in.c0[0]), sel(s, in.c0[0], in.c1[0]),
+                                               sel(s, in.c1[1], in.c0[1]), sel(s, in.c0[1], in.c1[1]));
+    *(float4 *)(tile + lane * 8 + 4) = make_float4(sel(s, in.c1[2], in.c0[2]), sel(s, in.c0[2], in.c1[2]),
+                                                   sel(s, in.c1[3], in.c0[3]), sel(s, in.c0[3], in.c1[3]));
+    wave_sync_lds();
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int v = k * 64 + lane;
+        if ((rows >> (v >> 1)) & 1ull) copy16_nt((float *)((char *)dst + c * 2048u + (uint32_t)v * 16u), tile + v * 4);
+    }
+    // the next tile of this wave restages the LDS tile: finish reading it first
+    wave_sync_lds();
+}
+
+// sweep `sweep` of the live grids, both colours (work list as for rbsor_batch_kernel)
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void rbsor_fused_kernel(const PGrid *__restrict__ grids,
+                                                                const int64_t *__restrict__ prefix,
+                                                                const int32_t *__restrict__ tile_grid,
+                                                                const int64_t *__restrict__ act, int zero_x, int sweep)
+{
+    __shared__ __attribute__((aligned(16))) float tiles[WAVES][100 * kFS];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int64_t nact = act[sweep];
+    const int64_t nwaves = (int64_t)gridDim.x * WAVES;
+    for (int64_t t = (int64_t)blockIdx.x * WAVES + w; t < nact; t += nwaves) {
+        const int gi = tile_grid[t];
+        const PGrid &g = grids[gi];
+        // the block's last sweep writes x
+        const bool to2 = ((g.nsweeps - 1 - sweep) & 1) != 0;
+        float *x = (float *)as_global(g.x), *x2 = as_global(g.x2);
+        fused_tile(g, (uint32_t)(t - prefix[gi]), tiles[w], lane, zero_x, to2 ? x : x2, to2 ? x2 : x);
+    }
+}
+
 // tile -> grid map of a work list
 __global__ __launch_bounds__(256) void tile_grid_kernel(const int64_t *__restrict__ prefix, int32_t *__restrict__ tg)
 {
@@ -231,7 +560,16 @@ __global__ __launch_bounds__(256) void defect_batch_kernel(const PGrid *__restri
     const int64_t t = (int64_t)blockIdx.x * 4 + w;
     if (t >= ntiles) return;
     const int gi = tile_grid[t];
-    const PGrid g = grids[gi];
+    const PGrid &gd = grids[gi];
+    struct {
+        const int32_t *nn;
+        const uint8_t *mask;
+        const double *u_in, *f;
+        double *u_out;
+        const float *e;
+        float *r32;
+    } g = {as_global(gd.nn), as_global(gd.mask), as_global(gd.u_in), as_global(gd.f),
+           as_global(gd.u_out), as_global(gd.e), as_global(gd.r32)};
     const int64_t c = t - prefix[gi];
     int64_t nbp[6];
     const int32_t *row = g.nn + c * 8;
@@ -356,6 +694,11 @@ struct sg_batch {
         double rel = 1.0;
         int inner = 0;  // inner sweeps for the next outer iteration
         double tol = 0.0;
+        // fused sweeps: second x buffer and neighbour table (from the batch's pool; null: the
+        // grid cannot take them), still to be set up
+        float *x2 = nullptr;
+        int32_t *nb = nullptr;
+        bool prep = false;
     };
     std::vector<Entry> live;
     std::vector<std::pair<int64_t, sg_poisson_result>> done;
@@ -403,6 +746,9 @@ int upload_worklist(sg_batch *b, bool defect_view, const std::vector<int> &order
         d.omega = en.omega;
         d.nsweeps = en.inner;
         d.f = (const double *)g->d_prop[b->p.f_prop];
+        d.x2 = en.x2;
+        d.nb = en.nb;
+        d.prep = en.prep ? 1 : 0;
         if (mixed) {
             d.x = g->d_prop[b->p.e_prop];
             d.rhs = g->d_prop[b->p.r_prop];
@@ -475,6 +821,24 @@ template <typename T> int launch_sweep(sg_batch *b, unsigned nblk, int color, in
     }
 }
 
+template <int W> int launch_fused_kernel(sg_batch *b, unsigned nblk, int zx, int s)
+{
+    hipLaunchKernelGGL((rbsor_fused_kernel<W>), dim3(nblk), dim3(64 * W), 0, b->stream, (const PGrid *)b->d_grids.p,
+                       (const int64_t *)b->d_prefix.p, (const int32_t *)b->d_tg.p, (const int64_t *)b->d_act.p, zx, s);
+    SG_HIP(hipGetLastError());
+    return SG_OK;
+}
+
+// every live grid can take fused sweeps (a grid that cannot makes the step run half sweeps
+// for all: e ends in its property either way)
+bool fused_ok(const sg_batch *b, bool first_zero)
+{
+    if (b->p.mode != SG_POISSON_MIXED || !first_zero) return false;
+    for (const auto &en : b->live)
+        if (!en.x2) return false;
+    return true;
+}
+
 int launch_sweeps(sg_batch *b, int sweeps, bool first_zero)
 {
     const int64_t nt = b->h_act.empty() ? 0 : b->h_act[0];
@@ -482,6 +846,20 @@ int launch_sweeps(sg_batch *b, int sweeps, bool first_zero)
     int64_t nblk = (nt + b->waves - 1) / b->waves;
     if (b->max_wgs > 0) nblk = std::min(nblk, b->max_wgs);
     const bool mixed = b->p.mode == SG_POISSON_MIXED;
+    if (fused_ok(b, first_zero)) {
+        for (int s = 0; s < sweeps; ++s) {
+            const int zx = s == 0 ? 1 : 0;
+            int rc;
+            switch (b->waves) {
+            case 1: rc = launch_fused_kernel<1>(b, (unsigned)nblk, zx, s); break;
+            case 2: rc = launch_fused_kernel<2>(b, (unsigned)nblk, zx, s); break;
+            case 8: rc = launch_fused_kernel<8>(b, (unsigned)nblk, zx, s); break;
+            default: rc = launch_fused_kernel<4>(b, (unsigned)nblk, zx, s); break;
+            }
+            if (rc) return rc;
+        }
+        return SG_OK;
+    }
     for (int s = 0; s < sweeps; ++s) {
         for (int color = 0; color < 2; ++color) {
             const int zx = (first_zero && s == 0 && color == 0) ? 1 : 0;
@@ -527,6 +905,14 @@ int defect_and_norms(sg_batch *b, std::vector<double> &norms, bool defect_view)
     if (rc) return rc;
     const int64_t nt = b->h_prefix[ng];
     norms.assign(2 * ng, 0.0);
+    bool prep = false;
+    for (const auto &en : b->live) prep = prep || en.prep;
+    if (prep) {
+        hipLaunchKernelGGL(fused_prep_kernel, dim3((unsigned)((nt + 3) / 4)), dim3(256), 0, b->stream,
+                           (const PGrid *)b->d_grids.p, (const int64_t *)b->d_prefix.p, (const int32_t *)b->d_tg.p, nt);
+        SG_HIP(hipGetLastError());
+        for (auto &en : b->live) en.prep = false;
+    }
     if (nt > 0) {
         hipLaunchKernelGGL(defect_batch_kernel, dim3((unsigned)((nt + 3) / 4)), dim3(256), 0, b->stream,
                            (const PGrid *)b->d_grids.p, (const int64_t *)b->d_prefix.p, (const int32_t *)b->d_tg.p,
@@ -571,6 +957,11 @@ void retire(sg_batch *b, size_t i, int converged)
     r.omega = en.omega;
     r.solution_prop = en.cur_u;
     b->done.emplace_back(en.tag, r);
+    // stream order: reused only by work queued on the batch's stream after this
+    b->pool.free(en.x2);
+    b->pool.free(en.nb);
+    en.x2 = nullptr;
+    en.nb = nullptr;
 }
 
 }  // namespace
@@ -637,6 +1028,21 @@ int sg_batch_add(sg_batch *b, sg_grid *g, int64_t tag, double tol)
     en.omega = (p.omega > 0.0) ? p.omega : p.omega0;
     en.inner = p.first_sweeps;
     en.tol = (tol > 0.0) ? tol : p.tol;
+    // Fused sweeps keep e = 0 where no point is (as the second buffer has it), and take
+    // 2.1 KB a chunk of the batch's memory; a grid that does not fit makes its steps run half
+    // sweeps.
+    static const unsigned char zero[8] = {};
+    if (mixed && g->nchunks > 0 && g->nchunks < (1 << 21) - 1 && memcmp(g->bg[p.e_prop], zero, sizeof(float)) == 0) {
+        en.x2 = (float *)b->pool.alloc((size_t)(g->nchunks + 1) * 512 * sizeof(float));
+        en.nb = (int32_t *)b->pool.alloc((size_t)g->nchunks * kNb * sizeof(int32_t));
+        if (!en.x2 || !en.nb) {
+            b->pool.free(en.x2);
+            b->pool.free(en.nb);
+            en.x2 = nullptr;
+            en.nb = nullptr;
+        }
+        en.prep = en.x2 != nullptr;
+    }
     b->live.push_back(en);
     b->dirty = true;
     ++b->version;

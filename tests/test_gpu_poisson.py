@@ -149,3 +149,63 @@ def test_launch_shapes_identical(P, waves, max_wgs):
     for a, b, x, y in zip(ga, gb, ra, rb):
         assert x["sweeps"] == y["sweeps"] and y["converged"]
         np.testing.assert_array_equal(a.prop(x["solution_prop"]), b.prop(y["solution_prop"]))
+
+
+@pytest.mark.parametrize("scale", [1.0, 4e-38, 2e-44])
+@pytest.mark.parametrize("shape,sweeps,waves", [("points", 1, 4), ("points", 2, 1), ("points", 5, 4), ("block", 6, 2),
+                                                ("one", 3, 4), ("diagonal", 4, 8)])
+def test_fused_sweeps_match_oracle(P, oracle, shape, sweeps, waves, scale):
+    """Both colours of a sweep in one pass, bit for bit the oracle's half sweeps: ragged point
+    sets with padding-tagged points, a full block (every edge neighbour exists), a lone chunk,
+    chunks that touch at edges and corners only (edge neighbours without a face neighbour);
+    odd and even sweep counts (the last one writes e); right-hand sides whose quotients by 6
+    are subnormal, ties among them (the true-division path)."""
+    from openfpm_data_amd import SparseGridGpu
+    import torch
+    rng = np.random.default_rng(len(shape) + sweeps)
+    n = 40
+    if shape == "points":
+        pts = W.shell_points(n, 6.0, 17.0)
+        pts = pts[rng.random(len(pts)) < 0.9]
+    else:
+        lo = {"block": [(0, 0, 0), (24, 24, 24)], "one": [(8, 16, 8), (16, 24, 16)]}.get(shape)
+        boxes = [lo] if lo else [((8 * i, 8 * j, 8 * k), (8 * i + 8, 8 * j + 8, 8 * k + 8))
+                                 for i in range(4) for j in range(4) for k in range(4) if (i + j + k) % 2 == 0]
+        pts = np.concatenate([np.stack(np.meshgrid(*[np.arange(a, b) for a, b in zip(*bx)], indexing="ij"), -1).reshape(-1, 3)
+                              for bx in boxes])
+    f = (rng.integers(-1000, 1000, len(pts)) * scale).astype(np.float32).astype(np.float64)
+    z = np.zeros(len(pts))
+    g = SparseGridGpu(3, (n,) * 3, P.POISSON_PROPS)
+    g.insert_coords(pts.astype(np.int32), [z, z, f, z.astype(np.float32), z.astype(np.float32)])
+    g.flush(["sright"] * 5)
+    o = oracle.SparseGridCpu(3, (n,) * 3, [np.float32, np.float32], block_edge=8)
+    o.insert_coords(pts.astype(np.int32), [z.astype(np.float32), f.astype(np.float32)])
+    o.flush(["sright"] * 2)
+    if shape == "points":
+        g.tag_boundaries()
+        o.tag_boundaries()
+    torch.cuda.synchronize()
+    r = P.solve([g], P.make_params(tol=1e-300, omega=1.37, first_sweeps=sweeps, max_outer=1, use_graph=sweeps % 2 == 0),
+                tuning={C.TUNE_BATCH_WAVES: waves})[0]
+    assert r["sweeps"] == sweeps
+    for _ in range(sweeps):
+        o.rbsor_sweep(0, 1, 1.37, 0)
+        o.rbsor_sweep(0, 1, 1.37, 1)
+    np.testing.assert_array_equal(g.masks(), o.masks())
+    want = o.prop(0)
+    assert want[want != 0].size > 0
+    np.testing.assert_array_equal(g.prop(P.E).view(np.uint32), want.view(np.uint32))
+    np.testing.assert_array_equal(g.prop(r["solution_prop"]), 0.0 + want.astype(np.float64))
+
+
+def test_grids_without_fused_sweeps(P, oracle):
+    """A background of e other than 0 (read where no point is) makes the step run half sweeps,
+    for its batch mates as well: the mates' solutions keep their bits."""
+    specs = _small_grids(2, 5, 48)
+    alone = [P.poisson_grid(s["size"], s["chunk_ids"], s["f"]) for s in specs]
+    ra = [P.solve([g], P.make_params(tol=1e-8))[0] for g in alone]
+    mixed = [P.poisson_grid(s["size"], s["chunk_ids"], s["f"]) for s in specs]
+    mixed[1].set_background_value(P.E, 0.5)
+    rm = P.solve(mixed, P.make_params(tol=1e-8, max_outer=30))
+    assert ra[0]["converged"] and rm[0]["converged"] and ra[0]["sweeps"] == rm[0]["sweeps"]
+    np.testing.assert_array_equal(alone[0].prop(ra[0]["solution_prop"]), mixed[0].prop(rm[0]["solution_prop"]))
