@@ -50,7 +50,76 @@ void free_idle(int dev)
     }
 }
 
+// pinned blocks given back, oldest first
+constexpr size_t kPinnedBlocks = 16, kPinnedBytes = 1 << 20;
+std::mutex g_pinned_mu;
+std::vector<PinnedBlock> g_pinned;
+size_t g_pinned_bytes = 0;
+
+void free_pinned(int dev)
+{
+    std::lock_guard<std::mutex> lk(g_pinned_mu);
+    for (size_t i = 0; i < g_pinned.size();) {
+        if (g_pinned[i].dev != dev) {
+            ++i;
+            continue;
+        }
+        (void)hipHostFree(g_pinned[i].p);
+        g_pinned_bytes -= g_pinned[i].bytes;
+        g_pinned.erase(g_pinned.begin() + (ptrdiff_t)i);
+    }
+}
+
 }  // namespace
+
+bool pinned_take(PinnedBlock &b, size_t bytes)
+{
+    bytes = std::max<size_t>(4096, (bytes + 4095) & ~(size_t)4095);
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    {
+        // the smallest kept block that fits and is not more than four times as large
+        std::lock_guard<std::mutex> lk(g_pinned_mu);
+        size_t best = g_pinned.size();
+        for (size_t i = 0; i < g_pinned.size(); ++i) {
+            const PinnedBlock &k = g_pinned[i];
+            if (k.dev == dev && k.bytes >= bytes && k.bytes <= 4 * bytes &&
+                (best == g_pinned.size() || k.bytes < g_pinned[best].bytes))
+                best = i;
+        }
+        if (best < g_pinned.size()) {
+            b = g_pinned[best];
+            g_pinned_bytes -= b.bytes;
+            g_pinned.erase(g_pinned.begin() + (ptrdiff_t)best);
+            return true;
+        }
+    }
+    void *p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    b.p = p;
+    b.bytes = bytes;
+    b.dev = dev;
+    return true;
+}
+
+void pinned_give(PinnedBlock &b)
+{
+    if (!b.p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_pinned_mu);
+        if (g_pinned.size() < kPinnedBlocks && g_pinned_bytes + b.bytes <= kPinnedBytes) {
+            g_pinned.push_back(b);
+            g_pinned_bytes += b.bytes;
+            b = PinnedBlock();
+            return;
+        }
+    }
+    (void)hipHostFree(b.p);
+    b = PinnedBlock();
+}
 
 void *DevicePool::alloc(size_t bytes)
 {
@@ -136,6 +205,7 @@ void DevicePool::trim()
     int dev = 0;
     (void)hipGetDevice(&dev);
     free_idle(dev);
+    free_pinned(dev);
 }
 
 size_t DevicePool::held_bytes() const

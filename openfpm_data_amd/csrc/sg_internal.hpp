@@ -77,6 +77,19 @@ private:
     size_t live_ = 0;
 };
 
+// Pinned host memory.  A block per grid, allocated and freed with it, made up some 50 us of
+// the 480 us that setting up and reading back a grid of 24,000 points takes, so blocks given
+// back are kept for the next taker of the process (per device; at most 16 blocks and 1 MB
+// together, the rest is freed; sg_trim frees all of them).  A block may only be given back
+// once no queued work uses it.  Safe with several threads.
+struct PinnedBlock {
+    void *p = nullptr;
+    size_t bytes = 0;
+    int dev = 0;
+};
+bool pinned_take(PinnedBlock &b, size_t bytes);
+void pinned_give(PinnedBlock &b);
+
 // a device buffer owned by a pool, grown on demand
 struct DevBuf {
     void *p = nullptr;
@@ -214,11 +227,8 @@ struct sg_grid {
     sg::DevBuf hostlike;     // small device staging
     // pinned host words that kernels write flags and totals to, read after the next stream
     // synchronisation
-    uint32_t *h_words = nullptr;
-    ~sg_grid()
-    {
-        if (h_words) (void)hipHostFree(h_words);
-    }
+    sg::PinnedBlock h_words;
+    ~sg_grid() { sg::pinned_give(h_words); }
 
     int nnn(int type) const { return type == SG_NN_STAR ? (1 << dim) : (dim == 2 ? 9 : 27); }
 };

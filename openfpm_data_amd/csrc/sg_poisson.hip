@@ -53,8 +53,9 @@ struct PGrid {
 // also count as LDS accesses, wait for them, and take 64-bit addresses per lane.
 template <typename T> __device__ __forceinline__ T *as_global(T *const &field)
 {
-    typedef __attribute__((address_space(1))) T *G;
-    return (T *)*(const G *)&field;
+    __attribute__((address_space(1))) T *g;
+    __builtin_memcpy(&g, &field, sizeof(g));
+    return (T *)g;
 }
 
 template <typename T> struct R8 {
@@ -704,20 +705,30 @@ struct sg_batch {
     std::vector<std::pair<int64_t, sg_poisson_result>> done;
     // device work list (rebuilt when the live set changes)
     sg::DevicePool pool;
-    sg::DevBuf d_grids, d_prefix, d_partial, d_norms, d_tg, d_act;
+    sg::DevBuf d_list, d_partial, d_tg;
+    // the work list's parts in d_list
+    sg::PGrid *d_grids = nullptr;
+    int64_t *d_prefix = nullptr, *d_act = nullptr;
     bool dirty = true;
     std::vector<int64_t> h_prefix, h_act;
-    // launch shape of the sweep kernel: waves per workgroup (1, 2, 4, 8) and a cap on the
-    // workgroups of one launch (0: one tile per wave); set by sg_batch_set_tuning
-    int waves = 4;
+    // pinned staging of the work lists (one for the defect's, one for the sweeps', so that a
+    // list is rewritten only after a wait for the norms that follow its copy) and of the norms,
+    // which their kernel writes there
+    sg::PinnedBlock h_list[2], h_norms;
+    // launch shape of the sweep kernel: waves per workgroup (1, 2, 4, 8; 0: by the number of
+    // tiles) and a cap on the workgroups of one launch (0: one tile per wave); set by
+    // sg_batch_set_tuning
+    int waves = 0;
     int64_t max_wgs = 0;
-    // graph of the inner sweep sequence for the current live set
+    // graph of the inner sweep sequence for a live set and sweep count, and the last sequence
+    // that was launched without one
     hipGraphExec_t graph = nullptr;
-    int graph_sweeps = -1;
-    uint64_t graph_version = 0, version = 0;
+    int graph_sweeps = -1, last_sweeps = -1;
+    uint64_t graph_version = 0, last_version = 0, version = 0;
     ~sg_batch()
     {
         if (graph) (void)hipGraphExecDestroy(graph);
+        for (sg::PinnedBlock *h : {&h_list[0], &h_list[1], &h_norms}) sg::pinned_give(*h);
         pool.release();
     }
 };
@@ -726,16 +737,32 @@ namespace {
 
 using namespace sg;
 
+int ensure_pinned(PinnedBlock &h, size_t bytes)
+{
+    if (h.bytes >= bytes) return SG_OK;
+    pinned_give(h);
+    return pinned_take(h, bytes + bytes / 2) ? SG_OK : fail(SG_E_OOM, "pinned host allocation failed");
+}
+
 // Device work list of the live grids in the order `order` (indices into live): grid
 // descriptors, prefix sums of chunk counts, the tile -> grid map and, for the sweeps, the
 // active tile count per sweep index (order must then be by decreasing inner count).
 int upload_worklist(sg_batch *b, bool defect_view, const std::vector<int> &order)
 {
     const int ng = (int)order.size();
-    std::vector<PGrid> gd(ng);
+    int max_inner = 1;
+    for (const auto &en : b->live) max_inner = std::max(max_inner, en.inner);
+    // one pinned block and one copy: descriptors | prefix sums | active tiles per sweep
+    const size_t at_prefix = sizeof(PGrid) * (size_t)std::max(ng, 1), at_act = at_prefix + sizeof(int64_t) * (ng + 1);
+    const size_t bytes = at_act + sizeof(int64_t) * (size_t)max_inner;
+    PinnedBlock &hl = b->h_list[defect_view ? 0 : 1];
+    const void *const had = b->d_list.p;
+    int rc;
+    if ((rc = ensure_pinned(hl, bytes)) || (rc = ensure(b->pool, b->d_list, bytes))) return rc;
+    if (b->d_list.p != had) ++b->version;  // a captured sequence reads the old list
+    PGrid *gd = (PGrid *)hl.p;
     b->h_prefix.assign(ng + 1, 0);
     const bool mixed = b->p.mode == SG_POISSON_MIXED;
-    int max_inner = 0;
     for (int i = 0; i < ng; ++i) {
         sg_batch::Entry &en = b->live[order[i]];
         sg_grid *g = en.g;
@@ -767,10 +794,9 @@ int upload_worklist(sg_batch *b, bool defect_view, const std::vector<int> &order
             d.r32 = nullptr;
         }
         b->h_prefix[i + 1] = b->h_prefix[i] + g->nchunks;
-        max_inner = std::max(max_inner, en.inner);
     }
     // act[s] = tiles of the grids with more than s sweeps (a prefix of the ordered list)
-    b->h_act.assign(std::max(max_inner, 1), 0);
+    b->h_act.assign(max_inner, 0);
     if (!defect_view) {
         int k = ng;
         for (int sw = 0; sw < max_inner; ++sw) {
@@ -779,41 +805,45 @@ int upload_worklist(sg_batch *b, bool defect_view, const std::vector<int> &order
         }
     }
     const int64_t nt = b->h_prefix[ng];
-    int rc;
-    if ((rc = ensure(b->pool, b->d_grids, sizeof(PGrid) * std::max(ng, 1))) ||
-        (rc = ensure(b->pool, b->d_prefix, sizeof(int64_t) * (ng + 1))) ||
-        (rc = ensure(b->pool, b->d_partial, sizeof(double) * 2 * std::max<int64_t>(nt, 1))) ||
-        (rc = ensure(b->pool, b->d_norms, sizeof(double) * 2 * std::max(ng, 1))) ||
-        (rc = ensure(b->pool, b->d_tg, sizeof(int32_t) * std::max<int64_t>(nt, 1))) ||
-        (rc = ensure(b->pool, b->d_act, sizeof(int64_t) * b->h_act.size())))
+    if ((rc = ensure(b->pool, b->d_partial, sizeof(double) * 2 * std::max<int64_t>(nt, 1))) ||
+        (rc = ensure_pinned(b->h_norms, sizeof(double) * 2 * std::max(ng, 1))) ||
+        (rc = ensure(b->pool, b->d_tg, sizeof(int32_t) * std::max<int64_t>(nt, 1))))
         return rc;
-    SG_HIP(hipMemcpyAsync(b->d_grids.p, gd.data(), sizeof(PGrid) * ng, hipMemcpyHostToDevice, b->stream));
-    SG_HIP(hipMemcpyAsync(b->d_prefix.p, b->h_prefix.data(), sizeof(int64_t) * (ng + 1), hipMemcpyHostToDevice,
-                          b->stream));
-    SG_HIP(hipMemcpyAsync(b->d_act.p, b->h_act.data(), sizeof(int64_t) * b->h_act.size(), hipMemcpyHostToDevice,
-                          b->stream));
+    memcpy((char *)hl.p + at_prefix, b->h_prefix.data(), sizeof(int64_t) * (ng + 1));
+    memcpy((char *)hl.p + at_act, b->h_act.data(), sizeof(int64_t) * b->h_act.size());
+    b->d_grids = (PGrid *)b->d_list.p;
+    b->d_prefix = (int64_t *)((char *)b->d_list.p + at_prefix);
+    b->d_act = (int64_t *)((char *)b->d_list.p + at_act);
+    SG_HIP(hipMemcpyAsync(b->d_list.p, hl.p, bytes, hipMemcpyHostToDevice, b->stream));
     if (ng > 0) {
-        hipLaunchKernelGGL(tile_grid_kernel, dim3((unsigned)ng), dim3(256), 0, b->stream,
-                           (const int64_t *)b->d_prefix.p, (int32_t *)b->d_tg.p);
+        hipLaunchKernelGGL(tile_grid_kernel, dim3((unsigned)ng), dim3(256), 0, b->stream, (const int64_t *)b->d_prefix,
+                           (int32_t *)b->d_tg.p);
         SG_HIP(hipGetLastError());
     }
-    // host vectors are reused on the next call: wait for the copies
-    SG_HIP(hipStreamSynchronize(b->stream));
     return SG_OK;
+}
+
+// waves per workgroup of the sweeps: 4 (neighbour chunks share a CU's cache: 48 grids 11.3 ms,
+// 12.2 ms with 1), or 1 while the tiles are fewer than would give every CU 4 waves (152
+// tiles: 4.3 us a sweep with 4 waves on 38 CUs, 3.9 us with 1 on 152)
+int sweep_waves(const sg_batch *b, int64_t nt)
+{
+    if (b->waves > 0) return b->waves;
+    return nt <= 1024 ? 1 : 4;
 }
 
 template <typename T, int W> int launch_sweep_kernel(sg_batch *b, unsigned nblk, int color, int zx, int s)
 {
     hipLaunchKernelGGL((rbsor_batch_kernel<T, W>), dim3(nblk), dim3(64 * W), 0, b->stream,
-                       (const PGrid *)b->d_grids.p, (const int64_t *)b->d_prefix.p, (const int32_t *)b->d_tg.p,
-                       (const int64_t *)b->d_act.p, color, zx, s);
+                       (const PGrid *)b->d_grids, (const int64_t *)b->d_prefix, (const int32_t *)b->d_tg.p,
+                       (const int64_t *)b->d_act, color, zx, s);
     SG_HIP(hipGetLastError());
     return SG_OK;
 }
 
-template <typename T> int launch_sweep(sg_batch *b, unsigned nblk, int color, int zx, int s)
+template <typename T> int launch_sweep(sg_batch *b, int waves, unsigned nblk, int color, int zx, int s)
 {
-    switch (b->waves) {
+    switch (waves) {
     case 1: return launch_sweep_kernel<T, 1>(b, nblk, color, zx, s);
     case 2: return launch_sweep_kernel<T, 2>(b, nblk, color, zx, s);
     case 8: return launch_sweep_kernel<T, 8>(b, nblk, color, zx, s);
@@ -823,8 +853,8 @@ template <typename T> int launch_sweep(sg_batch *b, unsigned nblk, int color, in
 
 template <int W> int launch_fused_kernel(sg_batch *b, unsigned nblk, int zx, int s)
 {
-    hipLaunchKernelGGL((rbsor_fused_kernel<W>), dim3(nblk), dim3(64 * W), 0, b->stream, (const PGrid *)b->d_grids.p,
-                       (const int64_t *)b->d_prefix.p, (const int32_t *)b->d_tg.p, (const int64_t *)b->d_act.p, zx, s);
+    hipLaunchKernelGGL((rbsor_fused_kernel<W>), dim3(nblk), dim3(64 * W), 0, b->stream, (const PGrid *)b->d_grids,
+                       (const int64_t *)b->d_prefix, (const int32_t *)b->d_tg.p, (const int64_t *)b->d_act, zx, s);
     SG_HIP(hipGetLastError());
     return SG_OK;
 }
@@ -843,14 +873,15 @@ int launch_sweeps(sg_batch *b, int sweeps, bool first_zero)
 {
     const int64_t nt = b->h_act.empty() ? 0 : b->h_act[0];
     if (nt == 0) return SG_OK;
-    int64_t nblk = (nt + b->waves - 1) / b->waves;
+    const int waves = sweep_waves(b, nt);
+    int64_t nblk = (nt + waves - 1) / waves;
     if (b->max_wgs > 0) nblk = std::min(nblk, b->max_wgs);
     const bool mixed = b->p.mode == SG_POISSON_MIXED;
     if (fused_ok(b, first_zero)) {
         for (int s = 0; s < sweeps; ++s) {
             const int zx = s == 0 ? 1 : 0;
             int rc;
-            switch (b->waves) {
+            switch (waves) {
             case 1: rc = launch_fused_kernel<1>(b, (unsigned)nblk, zx, s); break;
             case 2: rc = launch_fused_kernel<2>(b, (unsigned)nblk, zx, s); break;
             case 8: rc = launch_fused_kernel<8>(b, (unsigned)nblk, zx, s); break;
@@ -863,18 +894,26 @@ int launch_sweeps(sg_batch *b, int sweeps, bool first_zero)
     for (int s = 0; s < sweeps; ++s) {
         for (int color = 0; color < 2; ++color) {
             const int zx = (first_zero && s == 0 && color == 0) ? 1 : 0;
-            int rc = mixed ? launch_sweep<float>(b, (unsigned)nblk, color, zx, s)
-                           : launch_sweep<double>(b, (unsigned)nblk, color, zx, s);
+            int rc = mixed ? launch_sweep<float>(b, waves, (unsigned)nblk, color, zx, s)
+                           : launch_sweep<double>(b, waves, (unsigned)nblk, color, zx, s);
             if (rc) return rc;
         }
     }
     return SG_OK;
 }
 
-// run `sweeps` inner sweeps for the whole live set, through a cached hipGraph when asked
+// run `sweeps` inner sweeps for the whole live set, through a cached hipGraph when asked: the
+// sequence is captured when the same one comes a second time (capturing and instantiating 40
+// launches takes the host longer than queuing them while the first already run)
 int run_sweeps(sg_batch *b, int sweeps, bool first_zero)
 {
-    if (!b->p.use_graph) return launch_sweeps(b, sweeps, first_zero);
+    const bool have = b->graph && b->graph_sweeps == sweeps && b->graph_version == b->version;
+    const bool again = b->last_sweeps == sweeps && b->last_version == b->version;
+    if (!b->p.use_graph || (!have && !again)) {
+        b->last_sweeps = sweeps;
+        b->last_version = b->version;
+        return launch_sweeps(b, sweeps, first_zero);
+    }
     if (!b->graph || b->graph_sweeps != sweeps || b->graph_version != b->version) {
         if (b->graph) {
             SG_HIP(hipGraphExecDestroy(b->graph));
@@ -909,20 +948,20 @@ int defect_and_norms(sg_batch *b, std::vector<double> &norms, bool defect_view)
     for (const auto &en : b->live) prep = prep || en.prep;
     if (prep) {
         hipLaunchKernelGGL(fused_prep_kernel, dim3((unsigned)((nt + 3) / 4)), dim3(256), 0, b->stream,
-                           (const PGrid *)b->d_grids.p, (const int64_t *)b->d_prefix.p, (const int32_t *)b->d_tg.p, nt);
+                           (const PGrid *)b->d_grids, (const int64_t *)b->d_prefix, (const int32_t *)b->d_tg.p, nt);
         SG_HIP(hipGetLastError());
         for (auto &en : b->live) en.prep = false;
     }
     if (nt > 0) {
         hipLaunchKernelGGL(defect_batch_kernel, dim3((unsigned)((nt + 3) / 4)), dim3(256), 0, b->stream,
-                           (const PGrid *)b->d_grids.p, (const int64_t *)b->d_prefix.p, (const int32_t *)b->d_tg.p,
+                           (const PGrid *)b->d_grids, (const int64_t *)b->d_prefix, (const int32_t *)b->d_tg.p,
                            nt, (double *)b->d_partial.p);
         SG_HIP(hipGetLastError());
         hipLaunchKernelGGL(norm_reduce_kernel, dim3((unsigned)ng), dim3(256), 0, b->stream,
-                           (const double *)b->d_partial.p, (const int64_t *)b->d_prefix.p, ng, (double *)b->d_norms.p);
+                           (const double *)b->d_partial.p, (const int64_t *)b->d_prefix, ng, (double *)b->h_norms.p);
         SG_HIP(hipGetLastError());
-        SG_HIP(hipMemcpyAsync(norms.data(), b->d_norms.p, sizeof(double) * 2 * ng, hipMemcpyDeviceToHost, b->stream));
         SG_HIP(hipStreamSynchronize(b->stream));
+        memcpy(norms.data(), b->h_norms.p, sizeof(double) * 2 * ng);
     }
     return SG_OK;
 }

@@ -625,9 +625,8 @@ int exclusive_scan_u32(sg_grid *g, const uint32_t *in, uint32_t *out, int64_t n,
 
 uint32_t *host_words(sg_grid *g)
 {
-    if (!g->h_words && hipHostMalloc((void **)&g->h_words, 16 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess)
-        g->h_words = nullptr;
-    return g->h_words;
+    if (!g->h_words.p) (void)pinned_take(g->h_words, 16 * sizeof(uint32_t));
+    return (uint32_t *)g->h_words.p;
 }
 
 int radix_sort_pairs_u64(sg_grid *g, uint64_t *keys, uint32_t *vals, uint64_t *keys_tmp, uint32_t *vals_tmp,

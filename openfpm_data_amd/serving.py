@@ -9,7 +9,8 @@ relative-residual tolerance.  The loop
    footprint fit the budget (``Admission``; the head blocks the queue, so no request is
    starved by smaller ones behind it);
 3. builds each admitted grid on the device (insert of whole chunks, flush, neighbour
-   table), frees its build temporaries (``sg_trim``) and books its measured resident bytes;
+   table), frees its build temporaries (``sg_trim``; small ones stay with the grid, see
+   ``KEEP_TEMPORARIES``) and books its measured bytes and the batch's;
    the builds run in a builder thread on a stream of their own, so that they overlap the
    batched steps of the grids already live (the library's calls release the GIL);
 4. runs one outer iteration of every live grid in shared launches (``sg_batch_step``):
@@ -35,6 +36,17 @@ from . import poisson as P
 SLOT_BYTES = 3 * 8 + 2 * 4 + 1
 # per chunk: chunk id (8 B) + NNStar table row (8 x 4 B)
 CHUNK_BYTES = 8 + 8 * 4
+
+
+# per chunk, in the batch while the grid is live: a second FP32 sweep buffer (512 x 4 B) and a
+# row of 20 neighbour positions
+BATCH_CHUNK_BYTES = 512 * 4 + 20 * 4
+# Freeing and reallocating some 35 blocks takes a small grid's build longer than its kernels
+# (0.75 ms against 0.5 ms), so temporaries of up to KEEP_TEMPORARIES stay with the grid, booked,
+# and pass to later grids when it closes; after KEEP_BYTES of grids built so, a trim returns
+# what nobody uses.
+KEEP_TEMPORARIES = 32 << 20
+KEEP_BYTES = 256 << 20
 
 
 def resident_bytes(nchunks):
@@ -126,25 +138,33 @@ class PoissonServer:
         self.adm = Admission(budget_bytes)
         self.keep = keep_solutions
         self.threaded = build_thread
+        self._kept = 0  # bytes of the grids built since the last trim
 
     def close(self):
         self.batch.close()
 
     def _build(self, req, stream):
-        """Builds the request's grid on `stream`; returns (grid, resident bytes) once the
-        grid is complete (sg_trim waits for the stream)."""
+        """Builds the request's grid on `stream`; returns (grid, bytes to book) once the grid is
+        complete."""
         torch = self.torch
         with torch.cuda.stream(stream):
             f = torch.from_numpy(np.ascontiguousarray(req["f"])).to("cuda", non_blocking=False)
             ids = torch.from_numpy(np.asarray(req["chunk_ids"], np.int64)).to("cuda")
             g = P.poisson_grid(req["size"], ids, f, stream)
             del f, ids
-        C.check(C.load().sg_trim(g._h))
+        n = len(req["chunk_ids"])
+        held = grid_device_bytes(g)
+        self._kept += held
+        if held - resident_bytes(n) > KEEP_TEMPORARIES or self._kept > KEEP_BYTES:
+            C.check(C.load().sg_trim(g._h))
+            self._kept = 0
+        else:
+            g.synchronize()
         if stream is not self.stream:
-            # later work on the grid runs on the batch's stream (the build stream is idle:
-            # sg_trim waited for it, so the switch does not wait)
+            # later work on the grid runs on the batch's stream (the build stream is idle, so
+            # the switch does not wait)
             g.set_stream(self.stream)
-        return g, grid_device_bytes(g)
+        return g, grid_device_bytes(g) + n * BATCH_CHUNK_BYTES
 
     def _builder(self, inq, outq):
         while True:
