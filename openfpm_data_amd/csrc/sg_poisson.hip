@@ -238,9 +238,11 @@ __global__ __launch_bounds__(64 * WAVES) void rbsor_batch_kernel(const PGrid *__
 // half the launches.  The kernel is bound by instructions (about 400 vector ones a chunk,
 // against 2 x 363 of two half sweeps); before the rows were kept split by colour, with a
 // select for every operand, it had 680 and a sweep of 48 grids took 115 us.  Those 48 grids
-// (58,600 chunks): 2 x 64 us a sweep in half sweeps, 74 us here; 152 chunks 2 x 4.8 -> 4.3 us.
-// 4 waves a workgroup (1: 12.2 ms a solve of the 48 instead of 11.3); plain stores 11.9 ms;
-// registers for 5 waves a SIMD spill (14.2 ms).
+// (58,600 chunks): 2 x 64 us a sweep in half sweeps, 66 us here; 152 chunks 2 x 4.8 -> 3.9 us.
+// Measured and not kept (ms a solve of the 48, 10.0 as it is): 1, 2 or 8 waves a workgroup
+// 10.4, 10.3, 10.2; plain stores 10.4; contiguous tile ranges per XCD 10.1; groups of grids of
+// 16,384 tiles one after the other, so that a group stays in the Infinity Cache, 11.6 (the
+// launches' tails cost more than the misses).
 constexpr int kNb = 20;  // entries per chunk: -x +x -y +y -z +z, xy, xz, yz edges, 2 unused
 // LDS row of the 10 x 10 rows of a chunk and its ring: the 4 points of the first colour, the 4
 // of the second, then x = -1 and x = 8 at 8 and 9.  Point j of a colour is at x = 2 j + s, s
@@ -484,21 +486,15 @@ __device__ __forceinline__ void fused_tile(const PGrid &g, uint32_t c, float *ti
 
     const float wgt = (float)g.omega;
     bool small = false;
-    float k0[4], k1[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        k0[j] = in.c0[j];
-        k1[j] = in.c1[j];
-    }
     fused_compute<false>(in, tile, lane, wgt, &small);
     if (__ballot(small) != 0) {
         // subnormal quotients somewhere in the chunk: again with true divisions.  The LDS rows'
         // second-colour points are as they were, the first colour's are rewritten.
+        R8<float> again;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            in.c0[j] = k0[j];
-            in.c1[j] = k1[j];
-        }
+        for (int i = 0; i < 8; ++i) again.v[i] = 0.f;
+        if (!zero_x) ld8(again, (const float *)((const char *)src + at));
+        split8(in.c0, in.c1, again, s);
         wave_sync_lds();
         fused_compute<true>(in, tile, lane, wgt, &small);
     }
@@ -519,8 +515,10 @@ __device__ __forceinline__ void fused_tile(const PGrid &g, uint32_t c, float *ti
     wave_sync_lds();
 }
 
-// sweep `sweep` of the live grids, both colours (work list as for rbsor_batch_kernel)
-template <int WAVES>
+// Sweep `sweep` of the live grids, both colours (work list as for rbsor_batch_kernel).  A tile
+// per wave, or with LOOP as many as the launch's size needs: without the loop the per-lane
+// offsets are not kept across it, which leaves registers for 5 waves a SIMD instead of 4.
+template <int WAVES, bool LOOP>
 __global__ __launch_bounds__(64 * WAVES) void rbsor_fused_kernel(const PGrid *__restrict__ grids,
                                                                 const int64_t *__restrict__ prefix,
                                                                 const int32_t *__restrict__ tile_grid,
@@ -529,14 +527,19 @@ __global__ __launch_bounds__(64 * WAVES) void rbsor_fused_kernel(const PGrid *__
     __shared__ __attribute__((aligned(16))) float tiles[WAVES][100 * kFS];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t nact = act[sweep];
-    const int64_t nwaves = (int64_t)gridDim.x * WAVES;
-    for (int64_t t = (int64_t)blockIdx.x * WAVES + w; t < nact; t += nwaves) {
+    auto tile = [&](int64_t t) __attribute__((always_inline)) {
         const int gi = tile_grid[t];
         const PGrid &g = grids[gi];
         // the block's last sweep writes x
         const bool to2 = ((g.nsweeps - 1 - sweep) & 1) != 0;
         float *x = (float *)as_global(g.x), *x2 = as_global(g.x2);
         fused_tile(g, (uint32_t)(t - prefix[gi]), tiles[w], lane, zero_x, to2 ? x : x2, to2 ? x2 : x);
+    };
+    int64_t t = (int64_t)blockIdx.x * WAVES + w;
+    if constexpr (LOOP) {
+        for (; t < nact; t += (int64_t)gridDim.x * WAVES) tile(t);
+    } else if (t < nact) {
+        tile(t);
     }
 }
 
@@ -851,10 +854,17 @@ template <typename T> int launch_sweep(sg_batch *b, int waves, unsigned nblk, in
     }
 }
 
-template <int W> int launch_fused_kernel(sg_batch *b, unsigned nblk, int zx, int s)
+// loop: fewer workgroups than tiles
+template <int W> int launch_fused_kernel(sg_batch *b, unsigned nblk, bool loop, int zx, int s)
 {
-    hipLaunchKernelGGL((rbsor_fused_kernel<W>), dim3(nblk), dim3(64 * W), 0, b->stream, (const PGrid *)b->d_grids,
-                       (const int64_t *)b->d_prefix, (const int32_t *)b->d_tg.p, (const int64_t *)b->d_act, zx, s);
+    if (loop)
+        hipLaunchKernelGGL((rbsor_fused_kernel<W, true>), dim3(nblk), dim3(64 * W), 0, b->stream,
+                           (const PGrid *)b->d_grids, (const int64_t *)b->d_prefix, (const int32_t *)b->d_tg.p,
+                           (const int64_t *)b->d_act, zx, s);
+    else
+        hipLaunchKernelGGL((rbsor_fused_kernel<W, false>), dim3(nblk), dim3(64 * W), 0, b->stream,
+                           (const PGrid *)b->d_grids, (const int64_t *)b->d_prefix, (const int32_t *)b->d_tg.p,
+                           (const int64_t *)b->d_act, zx, s);
     SG_HIP(hipGetLastError());
     return SG_OK;
 }
@@ -878,14 +888,15 @@ int launch_sweeps(sg_batch *b, int sweeps, bool first_zero)
     if (b->max_wgs > 0) nblk = std::min(nblk, b->max_wgs);
     const bool mixed = b->p.mode == SG_POISSON_MIXED;
     if (fused_ok(b, first_zero)) {
+        const bool loop = nblk * waves < nt;
         for (int s = 0; s < sweeps; ++s) {
             const int zx = s == 0 ? 1 : 0;
             int rc;
             switch (waves) {
-            case 1: rc = launch_fused_kernel<1>(b, (unsigned)nblk, zx, s); break;
-            case 2: rc = launch_fused_kernel<2>(b, (unsigned)nblk, zx, s); break;
-            case 8: rc = launch_fused_kernel<8>(b, (unsigned)nblk, zx, s); break;
-            default: rc = launch_fused_kernel<4>(b, (unsigned)nblk, zx, s); break;
+            case 1: rc = launch_fused_kernel<1>(b, (unsigned)nblk, loop, zx, s); break;
+            case 2: rc = launch_fused_kernel<2>(b, (unsigned)nblk, loop, zx, s); break;
+            case 8: rc = launch_fused_kernel<8>(b, (unsigned)nblk, loop, zx, s); break;
+            default: rc = launch_fused_kernel<4>(b, (unsigned)nblk, loop, zx, s); break;
             }
             if (rc) return rc;
         }
