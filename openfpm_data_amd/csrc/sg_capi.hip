@@ -555,14 +555,15 @@ int sg_get_prop(sg_grid *g, int prop, void *out, int mem)
 int sg_set_prop(sg_grid *g, int prop, const void *in, int mem)
 {
     if (!valid_prop(g, prop) || !in) return fail(SG_E_ARG, "bad property or input");
+    if (mem == SG_MEM_DEVICE) return set_prop_device(g, prop, in);
     if (g->nchunks) {
-        SG_HIP(hipMemcpyAsync(g->d_prop[prop], in, (size_t)g->nchunks * g->csz * g->ts[prop],
-                              mem == SG_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, g->stream));
+        SG_HIP(hipMemcpyAsync(g->d_prop[prop], in, (size_t)g->nchunks * g->csz * g->ts[prop], hipMemcpyHostToDevice,
+                              g->stream));
         // slots without a point hold the background
         int rc = normalize_prop(g, prop);
         if (rc) return rc;
     }
-    if (mem == SG_MEM_HOST) SG_HIP(hipStreamSynchronize(g->stream));
+    SG_HIP(hipStreamSynchronize(g->stream));
     return SG_OK;
 }
 

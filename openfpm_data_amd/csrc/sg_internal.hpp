@@ -363,6 +363,8 @@ int apply_stencil_impl(sg_grid *g, const sg_stencil_desc *d);
 int get_points_impl(sg_grid *g, int prop, int64_t n, const int64_t *keys, void *out, int mem);
 int fill_background_chunk(sg_grid *g, int prop);
 int normalize_prop(sg_grid *g, int prop);
+// the property's values from device memory, the background where no point is
+int set_prop_device(sg_grid *g, int prop, const void *in);
 // occupancy table of the 8^3 star stencils (sg_grid::d_occ_tab), rebuilt when stale
 int occ_table_impl(sg_grid *g);
 // EXIST bit-planes of 8^3 chunks (sg_grid::d_ebits), rebuilt when stale

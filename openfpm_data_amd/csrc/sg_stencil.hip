@@ -2144,6 +2144,32 @@ template <typename T> __global__ void normalize_kernel(T *p, const uint8_t *mask
     if (i < n && mask[i] == 0) p[i] = v;
 }
 
+// p = src where the mask is not 0, the background elsewhere, 16 bytes of values per thread
+// (src 16-byte aligned) and the last n % (16 / sizeof(T)) values one by one; not VEC: a value
+// per thread.  One pass instead of a copy and a second kernel over what it wrote.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(kWG) void set_values_kernel(T *p, const T *src, const uint8_t *mask, int64_t n, T v)
+{
+    constexpr int E = VEC ? 16 / (int)sizeof(T) : 1;
+    struct __attribute__((aligned(VEC ? 16 : sizeof(T)))) Vals {
+        T t[E];
+    };
+    struct __attribute__((aligned(VEC ? E : 1))) Masks {
+        uint8_t m[E];
+    };
+    const int64_t i = (int64_t)blockIdx.x * kWG + threadIdx.x, nv = n / E;
+    if (i < nv) {
+        Vals a = ((const Vals *)src)[i];
+        const Masks m = ((const Masks *)mask)[i];
+#pragma unroll
+        for (int e = 0; e < E; ++e) a.t[e] = m.m[e] ? a.t[e] : v;
+        ((Vals *)p)[i] = a;
+    } else if (i - nv < n - nv * E) {
+        const int64_t k = nv * E + (i - nv);
+        p[k] = mask[k] ? src[k] : v;
+    }
+}
+
 // countExistingElements (which 0: EXIST bits) / countBoundaryElements (which 1: EXIST and
 // PADDING), SparseGridGpu.hpp:2422-2470: 16 mask bytes per load, four bytes per popcount
 __device__ inline uint32_t count_word(uint32_t w, int which)
@@ -2717,6 +2743,31 @@ int normalize_prop(sg_grid *g, int p)
         memcpy(&v, g->bg[p], sizeof(T));
         hipLaunchKernelGGL(normalize_kernel<T>, dim3(grid_1d(total, kWG)), dim3(kWG), 0, g->stream, (T *)g->d_prop[p],
                            g->d_mask, total, v);
+    });
+    SG_HIP(hipGetLastError());
+    return SG_OK;
+}
+
+int set_prop_device(sg_grid *g, int p, const void *in)
+{
+    const int64_t total = g->nchunks * g->csz;
+    if (total == 0) return SG_OK;
+    if ((uintptr_t)in % (size_t)g->ts[p]) {
+        // not even aligned to a value
+        SG_HIP(hipMemcpyAsync(g->d_prop[p], in, (size_t)total * g->ts[p], hipMemcpyDeviceToDevice, g->stream));
+        return normalize_prop(g, p);
+    }
+    dispatch_type(g->dt[p], [&](auto tag) {
+        typedef decltype(tag) T;
+        T v;
+        memcpy(&v, g->bg[p], sizeof(T));
+        constexpr int64_t E = 16 / sizeof(T);
+        if (((uintptr_t)in & 15) == 0)
+            hipLaunchKernelGGL((set_values_kernel<T, true>), dim3(grid_1d(total / E + total % E, kWG)), dim3(kWG), 0,
+                               g->stream, (T *)g->d_prop[p], (const T *)in, g->d_mask, total, v);
+        else
+            hipLaunchKernelGGL((set_values_kernel<T, false>), dim3(grid_1d(total, kWG)), dim3(kWG), 0, g->stream,
+                               (T *)g->d_prop[p], (const T *)in, g->d_mask, total, v);
     });
     SG_HIP(hipGetLastError());
     return SG_OK;

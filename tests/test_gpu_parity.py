@@ -1080,3 +1080,28 @@ def test_flush_few_records_per_chunk(G, oracle, dim, edge, grow, dtypes):
     m = a.masks()
     for p in range(len(dtypes)):
         assert (a.prop(p)[m == 0] == p + 1).all()
+
+
+@pytest.mark.parametrize("edge,dim", [(8, 3), (3, 3), (5, 2)])
+@pytest.mark.parametrize("dtype", [np.uint8, np.int16, np.float32, np.float64, np.int64])
+def test_set_prop_from_device_memory(G, dtype, edge, dim):
+    """Values from device memory at any alignment: taken where the mask is not 0, the
+    background elsewhere; sizes that are no whole number of 16-byte vectors."""
+    import torch
+    rng = np.random.default_rng(edge)
+    size = [4 * edge + 1] * dim
+    pts = np.stack([rng.integers(0, s, 200) for s in size], 1).astype(np.int32)
+    g = G(dim, size, [dtype, np.float32], block_edge=edge)
+    g.set_background_value(0, 7)
+    g.insert_coords(pts, [np.zeros(200, dtype), np.zeros(200, np.float32)], rng.choice(np.array([1, 2, 3], np.uint8), 200))
+    g.flush(["smax", "smax"])
+    m = g.masks().reshape(-1)
+    n = m.size
+    size_b = np.dtype(dtype).itemsize
+    raw = torch.from_numpy(rng.integers(0, 100, (n + 16) * size_b).astype(np.uint8)).cuda()
+    for off in (0, size_b, 1):
+        part = raw[off:off + n * size_b]
+        C.check(g._lib.sg_set_prop(g._h, 0, ctypes.c_void_p(part.data_ptr()), C.SG_MEM_DEVICE))
+        want = part.cpu().numpy().view(dtype).copy()
+        want[m == 0] = 7
+        np.testing.assert_array_equal(g.prop(0).reshape(-1).view(np.uint8), want.view(np.uint8))
