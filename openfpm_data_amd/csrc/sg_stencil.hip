@@ -873,9 +873,9 @@ template <typename T> struct BoxIn {
 };
 
 template <typename T>
-__device__ inline void box_load(BoxIn<T> &in, int64_t c, const int32_t *__restrict__ nn,
+__device__ __forceinline__ void box_load(BoxIn<T> &in, int64_t c, const int32_t *__restrict__ nn,
                                 const uint8_t *__restrict__ mask, const T *__restrict__ src, int lane,
-                                bool skip_xm = false, bool skip_xp = false)
+                                         bool skip_xm = false, bool skip_xp = false)
 {
     const int32_t *row_nn = nn + c * 27;
     auto chunk_of = [&](int dx, int dy, int dz) -> int64_t {
@@ -885,7 +885,6 @@ __device__ inline void box_load(BoxIn<T> &in, int64_t c, const int32_t *__restri
     const T *sr = src + c * 512 + lane * 8;
 #pragma unroll
     for (int i = 0; i < 8; ++i) in.own[i] = sr[i];
-    // skip_xm / skip_xp: the -x / +x ghosts come from a chunk the caller holds
     if (!skip_xm) in.oxm = src[chunk_of(-1, 0, 0) * 512 + lane * 8 + 7];
     if (!skip_xp) in.oxp = src[chunk_of(1, 0, 0) * 512 + lane * 8 + 0];
     if (lane < 36) {
@@ -901,12 +900,56 @@ __device__ inline void box_load(BoxIn<T> &in, int64_t c, const int32_t *__restri
     }
 }
 
+// Workgroup b runs in XCD b & 7, each with an L2 of its own.  An XCD takes the work of
+// 2^sh consecutive workgroups, then of the next 2^sh after the other XCDs' (a grid of a
+// multiple of 8 * 2^sh workgroups): most of the 26 neighbours a chunk reads are then in
+// that L2, and the XCDs still walk the same part of memory.
+__device__ __forceinline__ int64_t xcd_run_block(int sh)
+{
+    const uint32_t q = blockIdx.x >> 3;
+    return ((int64_t)((q >> sh) * 8 + (blockIdx.x & 7)) << sh) + (q & ((1u << sh) - 1));
+}
+
+// Box coefficients in the property type and the points to write: uniform kernel
+// arguments, so that a product takes its coefficient from a scalar register.
+template <typename T> struct BoxArgs {
+    T cf[27];
+    T bg_dst;
+    int apply, use_box, zorder;
+    int lo[3], hi[3];
+    int64_t bsz0, bsz1;
+};
+
+// bytes of a mask row that are not zero, as 0x01 each
+__device__ __forceinline__ uint64_t row_nonzero(uint64_t m)
+{
+    return ((((m & 0x7F7F7F7F7F7F7F7Full) + 0x7F7F7F7F7F7F7F7Full) | m) >> 7) & 0x0101010101010101ull;
+}
+
+// 0xFF in the bytes of the row (y, z) of the chunk `key` whose points lie in the box
+template <typename T>
+__device__ __forceinline__ uint64_t box_row_bytes(const BoxArgs<T> &ba, int64_t key, int y, int z)
+{
+    ChunkLin L;
+    L.dim = 3;
+    L.zorder = ba.zorder;
+    L.bsz[0] = ba.bsz0;
+    L.bsz[1] = ba.bsz1;
+    L.bsz[2] = 1 << 30;
+    int64_t bc[3];
+    chunk_coords(L, key, bc);
+    const int64_t py = bc[1] * 8 + y, pz = bc[2] * 8 + z;
+    const int64_t x0 = ba.lo[0] - bc[0] * 8, x1 = ba.hi[0] - bc[0] * 8;  // first and last x of the row
+    if (py < ba.lo[1] || py > ba.hi[1] || pz < ba.lo[2] || pz > ba.hi[2] || x0 > 7 || x1 < 0 || x0 > x1) return 0;
+    const int f = x0 < 0 ? 0 : (int)x0, l = x1 > 7 ? 7 : (int)x1;
+    return (~0ull << (8 * f)) & (~0ull >> (8 * (7 - l)));
+}
+
 // Stages chunk c's 10 x 10 x 10 tile from `in`, sums the 3 x 3 x 3 box of each of the
 // lane's 8 points and writes the chunk back through the tile.
 template <typename T, bool UNI>
-__device__ inline void box_finish(const BoxIn<T> &in, int64_t c, T *tw, T *__restrict__ dst,
-                                  const int64_t *__restrict__ keys, int64_t bsz0, int64_t bsz1, T bg_dst,
-                                  const StencilArgs &sa, int lane)
+__device__ __forceinline__ void box_finish(const BoxIn<T> &in, int64_t c, T *tw, T *__restrict__ dst,
+                                           const int64_t *__restrict__ keys, const BoxArgs<T> &ba, int lane)
 {
     const int y = lane & 7, z = lane >> 3;
     {
@@ -934,103 +977,74 @@ __device__ inline void box_finish(const BoxIn<T> &in, int64_t c, T *tw, T *__res
     uint32_t fl = 0;
     T out[8];
     if (mrow != 0) {
-        bool inbox[8];
-#pragma unroll
-        for (int x = 0; x < 8; ++x) inbox[x] = true;
-        if (sa.use_box) {
-            ChunkLin L;
-            L.dim = 3;
-            L.zorder = sa.zorder;
-            L.bsz[0] = bsz0;
-            L.bsz[1] = bsz1;
-            L.bsz[2] = 1 << 30;
-            int64_t bc[3];
-            chunk_coords(L, keys[c], bc);
-            const int64_t py = bc[1] * 8 + y, pz = bc[2] * 8 + z;
-            const bool yz = py >= sa.lo[1] && py <= sa.hi[1] && pz >= sa.lo[2] && pz <= sa.hi[2];
-#pragma unroll
-            for (int x = 0; x < 8; ++x) {
-                const int64_t px = bc[0] * 8 + x;
-                inbox[x] = yz && px >= sa.lo[0] && px <= sa.hi[0];
-            }
-        }
-        T cf[27];
-#pragma unroll
-        for (int q = 0; q < 27; ++q) cf[q] = std::is_integral<T>::value ? (T)sa.icoef[q] : (T)sa.coef[q];
-        T isum[8];
+        uint64_t m = mrow;
+        if (ba.use_box) m &= box_row_bytes(ba, keys[c], y, z);
+        // active points of the row, a byte 0x01 each
+        const uint64_t act = (ba.apply == SG_APPLY_EXISTING)
+                                 ? row_nonzero(m)
+                                 : (m & ~(m >> 1) & 0x0101010101010101ull);  // SG_EXIST without SG_PADDING
+        const uint32_t act_lo = (uint32_t)act, act_hi = (uint32_t)(act >> 32);
         if constexpr (std::is_integral<T>::value) {
             // wrapping integer sums do not depend on the order of the terms, so each of the
             // 9 rows of the 3 x 3 (y, z) neighbourhood is read from LDS once (10 values)
             // instead of once per tap
 #pragma unroll
-            for (int x = 0; x < 8; ++x) isum[x] = 0;
-            if constexpr (UNI) {
-                // every tap has the same coefficient: c (a + b + ...) = c a + c b + ... in
-                // wrapping arithmetic, so the 27 values are summed (row triples first) and
-                // multiplied once, no multiply per tap
+            for (int x = 0; x < 8; ++x) out[x] = 0;
 #pragma unroll
-                for (int j = 0; j < 3; ++j)
+            for (int j = 0; j < 3; ++j)
 #pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        const T *row = tw + ((z + k) * 10 + (y + j)) * 10;
-                        T r[10];
+                for (int k = 0; k < 3; ++k) {
+                    const T *row = tw + ((z + k) * 10 + (y + j)) * 10;
+                    T r[10];
 #pragma unroll
-                        for (int q = 0; q < 10; ++q) r[q] = row[q];
+                    for (int q = 0; q < 10; ++q) r[q] = row[q];
+                    if constexpr (UNI) {
+                        // every tap has the same coefficient: c (a + b + ...) = c a + c b + ...
+                        // in wrapping arithmetic, so the 27 values are summed (row triples
+                        // first) and multiplied once, no multiply per tap
 #pragma unroll
                         for (int x = 0; x < 8; ++x)
-                            isum[x] = dev_add<T>(isum[x], dev_add<T>(dev_add<T>(r[x], r[x + 1]), r[x + 2]));
-                    }
+                            out[x] = dev_add<T>(out[x], dev_add<T>(dev_add<T>(r[x], r[x + 1]), r[x + 2]));
+                        // a row's sums are done before the next row's: regrouped over all
+                        // rows, as the compiler would, the 90 values stay live at once
 #pragma unroll
-                for (int x = 0; x < 8; ++x) isum[x] = dev_mul<T>(isum[x], cf[0]);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 3; ++j)
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        const T *row = tw + ((z + k) * 10 + (y + j)) * 10;
-                        T r[10];
-#pragma unroll
-                        for (int q = 0; q < 10; ++q) r[q] = row[q];
+                        for (int x = 0; x < 8; ++x) asm volatile("" : "+v"(out[x]));
+                    } else {
 #pragma unroll
                         for (int i = 0; i < 3; ++i)
 #pragma unroll
                             for (int x = 0; x < 8; ++x)
-                                isum[x] = dev_add<T>(isum[x], dev_mul<T>(r[x + i], cf[i * 9 + j * 3 + k]));
+                                out[x] = dev_add<T>(out[x], dev_mul<T>(r[x + i], ba.cf[i * 9 + j * 3 + k]));
                     }
-            }
-        }
-        bool act[8];
-        bool whole = true;
+                }
+            if constexpr (UNI) {
 #pragma unroll
-        for (int x = 0; x < 8; ++x) {
-            uint8_t cm = (uint8_t)(mrow >> (8 * x));
-            if (!inbox[x]) cm = 0;
-            act[x] = (sa.apply == SG_APPLY_EXISTING) ? (cm != 0) : ((cm & SG_EXIST) && !(cm & SG_PADDING));
-            const uint8_t raw = (uint8_t)(mrow >> (8 * x));
-            whole = whole && (act[x] || raw == 0);
-            T tot = 0;
-            if constexpr (std::is_integral<T>::value) {
-                tot = isum[x];
-            } else {
-                // floating point: the reference order (x offset outermost, z innermost)
+                for (int x = 0; x < 8; ++x) out[x] = dev_mul<T>(out[x], ba.cf[0]);
+            }
+        } else {
+            // floating point: the reference order (x offset outermost, z innermost)
+#pragma unroll
+            for (int x = 0; x < 8; ++x) {
+                T tot = 0;
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
 #pragma unroll
                     for (int j = 0; j < 3; ++j)
 #pragma unroll
                         for (int k = 0; k < 3; ++k)
-                            tot = dev_add<T>(tot,
-                                             dev_mul<T>(tw[((z + k) * 10 + (y + j)) * 10 + (x + i)], cf[i * 9 + j * 3 + k]));
+                            tot = dev_add<T>(tot, dev_mul<T>(tw[((z + k) * 10 + (y + j)) * 10 + (x + i)],
+                                                             ba.cf[i * 9 + j * 3 + k]));
+                out[x] = tot;
             }
-            out[x] = act[x] ? tot : bg_dst;
         }
-        if (whole) {
-            fl = 1;
-        } else {
-            fl = 2;
 #pragma unroll
-            for (int x = 0; x < 8; ++x) fl |= (uint32_t)act[x] << (8 + x);
-        }
+        for (int x = 0; x < 8; ++x)
+            out[x] = (((x < 4 ? act_lo : act_hi) >> (8 * (x & 3))) & 1u) ? out[x] : ba.bg_dst;
+        // whole: every point of the row is active or empty; else the bytes' bits gathered
+        // into bits 8-15 (b << 24, 17, 10, 3 do not overlap)
+        fl = (act == row_nonzero(mrow)) ? 1u
+                                        : 2u | (((act_lo * 0x01020408u) >> 24) & 15u) << 8 |
+                                              (((act_hi * 0x01020408u) >> 24) & 15u) << 12;
     }
     // the tile is free once every lane has summed its points: stage the rows there and
     // write the chunk back contiguously
@@ -1047,46 +1061,58 @@ __device__ inline void box_finish(const BoxIn<T> &in, int64_t c, T *tw, T *__res
     store_chunk_contig(dst + c * 512, tw, fl, lane);
 }
 
-// One wave per chunk (lane = x-row).  Every load of the chunk (source rows, ghosts, mask
-// row) is issued into registers before any is used, then the 10 x 10 x 10 tile of the
-// source (rows (z, y) in [-1, 8]^2, 10 values with the x ghosts, from the chunk and its 26
-// neighbours; a missing chunk is the background chunk) is staged in LDS and each lane
-// sums its 8 points over the 3 x 3 x 3 box in stencil_generic_kernel's order (x offset
+constexpr int kBoxRunLog = 7;  // chunks an XCD takes in a row: 128, fewer on small grids
+template <typename T> constexpr int kBoxWaves = std::is_same<T, double>::value ? 5 : 1;
+
+// One wave and workgroup per chunk (lane = x-row).  Every load of the chunk (source rows,
+// ghosts, mask row) is issued into registers before any is used, then the 10 x 10 x 10 tile
+// of the source (rows (z, y) in [-1, 8]^2, 10 values with the x ghosts, from the chunk and
+// its 26 neighbours; a missing chunk is the background chunk) is staged in LDS and each
+// lane sums its 8 points over the 3 x 3 x 3 box in stencil_generic_kernel's order (x offset
 // outermost, z innermost).  Rows whose points are all active or empty are stored whole
 // (empty points take the destination background); other rows point by point.
-template <typename T, int WAVES, bool UNI>
-__global__ __launch_bounds__(64 * WAVES) void box8_kernel(int64_t n, const int32_t *__restrict__ nn,
+//
+// The bound is the traffic between L2 and memory: about 100 lines of 128 bytes per chunk
+// are touched for 2-4 KB of own values.  FP32 on 23,600 chunks (0.11 GB), us: chunks dealt
+// to the XCDs workgroup by workgroup 46; runs of 8 chunks 31, 32 28, 128 27, 512 28, one
+// range per XCD 27.  On 190,000 chunks (0.88 GB): 352; 234, 233, 231, 239, 250.  Pairs of
+// chunks in round-robin workgroups of 8 took 42 and 269.  Arithmetic (two roundings per
+// tap: 432 vector instructions per lane and chunk) is about 17 us of it; coefficients in the
+// property type as kernel arguments instead of converted from FP64 by each wave, and
+// activity as byte masks, took it from 940 to 730 instructions.
+template <typename T, bool UNI>
+__global__ __launch_bounds__(64, kBoxWaves<T>) void box8_kernel(int64_t n, const int32_t *__restrict__ nn,
                                                          const uint8_t *__restrict__ mask, const T *__restrict__ src,
                                                          T *__restrict__ dst, const int64_t *__restrict__ keys,
-                                                         int64_t bsz0, int64_t bsz1, T bg_dst, StencilArgs sa)
+                                                         int sh, BoxArgs<T> ba)
 {
-    __shared__ T tile[WAVES][100 * 10];
-    // uniform wave index: the neighbour-table row is read by scalar loads
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t c = (int64_t)blockIdx.x * WAVES + w;
-    if (c >= n) return;  // waves are independent
+    __shared__ T tile[100 * 10];
+    const int64_t c = xcd_run_block(sh);  // uniform: the neighbour-table row is read by scalar loads
+    if (c >= n) return;
     BoxIn<T> a;
-    box_load<T>(a, c, nn, mask, src, lane);
-    box_finish<T, UNI>(a, c, tile[w], dst, keys, bsz0, bsz1, bg_dst, sa, lane);
+    box_load<T>(a, c, nn, mask, src, threadIdx.x);
+    box_finish<T, UNI>(a, c, tile, dst, keys, ba, threadIdx.x);
 }
+
+template <typename T>
+constexpr int kBoxPairWaves = std::is_same<T, float>::value ? 5 : std::is_same<T, double>::value ? 3 : 1;
 
 // Two consecutive chunks c0 = 2p, c1 = 2p + 1 per wave.  When c1 is c0's +x neighbour (the
 // table says so; consecutive chunk ids along x sort next to each other), the x ghosts
 // between them are not gathered: c0's +x ghosts of its own and ghost rows are x = 0 of
 // c1's same rows, c1's -x ghosts x = 7 of c0's, all in the lane's own registers (a ghost
 // row of c1 comes from the chunk at (1, dy, dz) from c0, whose row c0's +x ghost is).
-// Those gathers of single values from 64 or 36 rows each are most of the kernel's
-// texture-addresser work.  Otherwise each chunk gathers its own.
-template <typename T, int WAVES, bool UNI>
-__global__ __launch_bounds__(64 * WAVES) void box8_pair_kernel(int64_t n, const int32_t *__restrict__ nn,
-                                                              const uint8_t *__restrict__ mask,
-                                                              const T *__restrict__ src, T *__restrict__ dst,
-                                                              const int64_t *__restrict__ keys, int64_t bsz0,
-                                                              int64_t bsz1, T bg_dst, StencilArgs sa)
+// Otherwise each chunk gathers its own.  Fewer waves are in flight, but each has twice the
+// lines of HBM on the way: for arrays far larger than the caches.
+template <typename T, bool UNI>
+__global__ __launch_bounds__(128, kBoxPairWaves<T>) void box8_pair_kernel(
+    int64_t n, const int32_t *__restrict__ nn, const uint8_t *__restrict__ mask, const T *__restrict__ src,
+    T *__restrict__ dst, const int64_t *__restrict__ keys, int sh, BoxArgs<T> ba)
 {
-    __shared__ T tile[WAVES][100 * 10];
+    __shared__ T tile[2][100 * 10];
+    // uniform wave index: the neighbour-table rows are read by scalar loads
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t c0 = ((int64_t)blockIdx.x * WAVES + w) * 2, c1 = c0 + 1;
+    const int64_t c0 = (xcd_run_block(sh) * 2 + w) * 2, c1 = c0 + 1;
     if (c0 >= n) return;  // waves are independent
     const bool two = c1 < n;
     // full table entry (dx + 1) + 3 (dy + 1) + 9 (dz + 1) of (+1, 0, 0): 14
@@ -1102,13 +1128,13 @@ __global__ __launch_bounds__(64 * WAVES) void box8_pair_kernel(int64_t n, const 
             b.gxm = a.gr[7];
         }
     }
-    box_finish<T, UNI>(a, c0, tile[w], dst, keys, bsz0, bsz1, bg_dst, sa, lane);
+    box_finish<T, UNI>(a, c0, tile[w], dst, keys, ba, lane);
     if (two) {
         // the tile is staged again: every lane's reads of the first chunk come first
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        box_finish<T, UNI>(b, c1, tile[w], dst, keys, bsz0, bsz1, bg_dst, sa, lane);
+        box_finish<T, UNI>(b, c1, tile[w], dst, keys, ba, lane);
     }
 }
 
@@ -2496,21 +2522,39 @@ int apply_stencil_impl(sg_grid *g, const sg_stencil_desc *d)
         dispatch_type(dt, [&](auto tag) {
             typedef decltype(tag) T;
             if constexpr (sizeof(T) >= 4) {
-                T bgd;
-                memcpy(&bgd, g->bg[d->dst[0]], sizeof(T));
+                BoxArgs<T> ba;
+                memcpy(&ba.bg_dst, g->bg[d->dst[0]], sizeof(T));
+                for (int q = 0; q < 27; ++q) ba.cf[q] = std::is_integral<T>::value ? (T)sa.icoef[q] : (T)sa.coef[q];
+                ba.apply = sa.apply;
+                ba.use_box = sa.use_box;
+                ba.zorder = sa.zorder;
+                for (int q = 0; q < 3; ++q) ba.lo[q] = sa.lo[q], ba.hi[q] = sa.hi[q];
+                ba.bsz0 = g->bsz[0];
+                ba.bsz1 = g->bsz[1];
                 // integer boxes whose 27 coefficients are equal (as T) sum first, multiply once
                 bool uni = std::is_integral<T>::value;
                 for (int q = 1; q < 27 && uni; ++q) uni = (T)d->icoef[q] == (T)d->icoef[0];
+                // Pairs only where the arrays are far larger than the 256 MB Infinity Cache
+                // (the line lies where both take the same: 0.7 GB in FP64).  FP32 and FP64 on
+                // shells, one chunk / pairs: 0.11 GB 27 / 32 us, 0.27 GB 55 / 61, 0.41 GB
+                // 79 / 85, 0.88 GB 231 / 199; 0.51 GB 105 / 119, 0.77 GB 185 / 184, 1.65 GB
+                // 391 / 372.
+                const bool pairs = g->box_pairs >= 0 ? g->box_pairs != 0
+                                                     : n * 512 * (int64_t)(2 * sizeof(T) + 1) > (int64_t)640 << 20;
                 auto launch = [&](auto u) {
                     constexpr bool U = decltype(u)::value;
-                    if (g->box_pairs)
-                        hipLaunchKernelGGL((box8_pair_kernel<T, 4, U>), dim3((unsigned)((n + 7) / 8)), dim3(256), 0,
-                                           g->stream, n, g->d_nn[type], g->d_mask, (const T *)g->d_prop[d->src[0]],
-                                           (T *)g->d_prop[d->dst[0]], g->d_keys, g->bsz[0], g->bsz[1], bgd, sa);
+                    // every XCD gets at least 4 runs, a pair kernel's workgroup 4 chunks
+                    int run = kBoxRunLog;
+                    while (run > (pairs ? 2 : 0) && n < ((int64_t)32 << run)) --run;
+                    const unsigned runs = (unsigned)((n + (8 << run) - 1) / (8 << run) * 8);
+                    if (pairs)
+                        hipLaunchKernelGGL((box8_pair_kernel<T, U>), dim3(runs << (run - 2)), dim3(128), 0, g->stream, n,
+                                           g->d_nn[type], g->d_mask, (const T *)g->d_prop[d->src[0]],
+                                           (T *)g->d_prop[d->dst[0]], g->d_keys, run - 2, ba);
                     else
-                        hipLaunchKernelGGL((box8_kernel<T, 4, U>), dim3((unsigned)((n + 3) / 4)), dim3(256), 0,
-                                           g->stream, n, g->d_nn[type], g->d_mask, (const T *)g->d_prop[d->src[0]],
-                                           (T *)g->d_prop[d->dst[0]], g->d_keys, g->bsz[0], g->bsz[1], bgd, sa);
+                        hipLaunchKernelGGL((box8_kernel<T, U>), dim3(runs << run), dim3(64), 0, g->stream, n,
+                                           g->d_nn[type], g->d_mask, (const T *)g->d_prop[d->src[0]],
+                                           (T *)g->d_prop[d->dst[0]], g->d_keys, run, ba);
                 };
                 if (uni) launch(std::true_type());
                 else launch(std::false_type());

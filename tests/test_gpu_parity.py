@@ -747,6 +747,33 @@ def test_tag_and_box_8cubed_random(G, oracle, seed, pairs):
         S.assert_same_state(a, b, exist_only=False)
 
 
+@pytest.mark.parametrize("pairs", [1, 0, None])
+@pytest.mark.parametrize("edge,dt", [(8, np.float64), (40, np.float32), (73, np.int32), (136, np.float32),
+                                     (137, np.int64)])
+def test_box_8cubed_chunk_runs(G, oracle, edge, dt, pairs):
+    """The chunks dealt to the XCDs in runs: 1 chunk, fewer and more than 8 * 128, an odd
+    last run; one chunk or two per wave, or by size.  Bit-exact against the oracle."""
+    rng = np.random.default_rng(edge)
+    pts = rng.integers(0, edge, (40 * edge, 3)).astype(np.int32)
+    val = rng.integers(-50, 50, pts.shape[0]).astype(dt)
+    coef = rng.integers(-3, 4, 27)
+    grids = []
+    for cls in (G, oracle.SparseGridCpu):
+        g = cls(3, (edge,) * 3, [dt, dt])
+        g.insert_coords(pts, [val, np.zeros_like(val)])
+        g.flush(["smax", "smax"])
+        g.set_nn_type(C.NN_FULL)
+        if cls is G and pairs is not None:
+            g.set_tuning(C.TUNE_BOX_PAIRS, pairs)
+        for box in (None, ((1, 2, 3), (edge - 2, edge - 1, edge // 2 + 3))):
+            if np.issubdtype(np.dtype(dt), np.integer):
+                g.apply_stencil(C.make_desc(C.ST_BOX, [0], [1], C.APPLY_EXISTING, box, (), [int(v) for v in coef]))
+            else:
+                g.apply_stencil(C.make_desc(C.ST_BOX, [0], [1], C.APPLY_EXISTING, box, [v / 3 for v in coef]))
+        grids.append(g)
+    S.assert_same_state(*grids)
+
+
 @pytest.mark.parametrize("variant,cpw", [(0, 1), (1, 1), (1, 2), (1, 4)])
 @pytest.mark.parametrize("nn", [C.NN_STAR, C.NN_FULL])
 def test_tag_boundaries_chunks_per_wave(G, oracle, variant, cpw, nn):
