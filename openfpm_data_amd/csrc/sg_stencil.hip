@@ -244,6 +244,30 @@ struct StencilArgs {
     int64_t icoef[27];
 };
 
+// Workgroup b runs in XCD b & 7, each with an L2 of its own.  An XCD takes the work of
+// 2^sh consecutive workgroups, then of the next 2^sh after the other XCDs' (a grid of a
+// multiple of 8 * 2^sh workgroups): most of the 26 neighbours a chunk reads are then in
+// that L2, and the XCDs still walk the same part of memory.
+__device__ __forceinline__ int64_t xcd_run_block(int sh)
+{
+    const uint32_t q = blockIdx.x >> 3;
+    return ((int64_t)((q >> sh) * 8 + (blockIdx.x & 7)) << sh) + (q & ((1u << sh) - 1));
+}
+
+constexpr int kBoxRunLog = 7;  // 27-point box and 2D kernels: 128 chunks in a row
+
+// Runs of up to 2^max_log workgroups, at least 4 for every XCD where there are that many.
+struct XcdRuns {
+    int sh;
+    unsigned grid;
+};
+XcdRuns xcd_runs(int64_t nwg, int max_log)
+{
+    int sh = max_log;
+    while (sh > 0 && nwg < ((int64_t)32 << sh)) --sh;
+    return {sh, (unsigned)((nwg + (8 << sh) - 1) / (8 << sh) * (8 << sh))};
+}
+
 // generic stencil: one workgroup per chunk, enlarged blocks of up to two
 // properties in dynamic LDS.  dst_alias[q] != 0 means dst q is also a source: it is
 // then written for every slot (new value where active, the old value elsewhere)
@@ -900,16 +924,6 @@ __device__ __forceinline__ void box_load(BoxIn<T> &in, int64_t c, const int32_t 
     }
 }
 
-// Workgroup b runs in XCD b & 7, each with an L2 of its own.  An XCD takes the work of
-// 2^sh consecutive workgroups, then of the next 2^sh after the other XCDs' (a grid of a
-// multiple of 8 * 2^sh workgroups): most of the 26 neighbours a chunk reads are then in
-// that L2, and the XCDs still walk the same part of memory.
-__device__ __forceinline__ int64_t xcd_run_block(int sh)
-{
-    const uint32_t q = blockIdx.x >> 3;
-    return ((int64_t)((q >> sh) * 8 + (blockIdx.x & 7)) << sh) + (q & ((1u << sh) - 1));
-}
-
 // Box coefficients in the property type and the points to write: uniform kernel
 // arguments, so that a product takes its coefficient from a scalar register.
 template <typename T> struct BoxArgs {
@@ -1061,7 +1075,6 @@ __device__ __forceinline__ void box_finish(const BoxIn<T> &in, int64_t c, T *tw,
     store_chunk_contig(dst + c * 512, tw, fl, lane);
 }
 
-constexpr int kBoxRunLog = 7;  // chunks an XCD takes in a row: 128, fewer on small grids
 template <typename T> constexpr int kBoxWaves = std::is_same<T, double>::value ? 5 : 1;
 
 // One wave and workgroup per chunk (lane = x-row).  Every load of the chunk (source rows,
@@ -1843,22 +1856,27 @@ __device__ inline void group_step(GroupLds<T, KIND, W, ONE> &L, int64_t grp, int
     process_chunk<T, KIND, ONE>(in, c, L.tiles0[w], L.tiles1[w], dst0, dst1, alias, sa, keys, bsz0, bsz1, lane);
 }
 
-// one group per workgroup; group g runs in XCD g's slot (g & 7 of the launch order)
+// Chunks an XCD takes in a row (a power of two; xcd_run_block), FP32 128 and FP64 64: the
+// same bytes.  Gray-Scott on a shell of 512^3 in FP32, one range per XCD 159 us for two
+// steps; runs of 32 chunks 162, 64 151, 128 148, 256 148, 512 153.  On a shell of 391^3 in
+// FP64 (variant 6) 189; 179, 178, 181, 179, 181; of 200^3 42; 41, 41, 44, 44, 44.
+template <typename T> constexpr int kStarRunLog = sizeof(T) == 8 ? 6 : 7;
+
+// one group per workgroup
 template <typename T, int KIND, int W, bool ONE>
 __global__ __launch_bounds__(64 * W) void stencil_group_kernel(const int32_t *__restrict__ nn, int64_t n,
                                                                const uint8_t *__restrict__ mask,
                                                                const T *__restrict__ src0, const T *__restrict__ src1,
                                                                T *__restrict__ dst0, T *__restrict__ dst1, int alias,
                                                                StencilArgs sa, const int64_t *__restrict__ keys,
-                                                               int64_t bsz0, int64_t bsz1, int64_t groups_per_xcd)
+                                                               int64_t bsz0, int64_t bsz1, int sh)
 {
     __shared__ GroupLds<T, KIND, W, ONE> L;
     // the wave index is uniform: with it in a scalar register the neighbour-table row is
     // read by scalar loads, which the ghost loads wait for without waiting for the own
     // rows (vector loads complete in order)
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t b = blockIdx.x;
-    const int64_t grp = (b & 7) * groups_per_xcd + (b >> 3);
+    const int64_t grp = xcd_run_block(sh);
     group_step<T, KIND, W, ONE>(L, grp, w, lane, nn, n, mask, src0, src1, dst0, dst1, alias, sa, keys, bsz0, bsz1);
 }
 
@@ -1871,12 +1889,11 @@ __global__ __launch_bounds__(64 * W) void rbsor_group_kernel(const int32_t *__re
                                                             const uint8_t *__restrict__ mask, T *u,
                                                             const T *__restrict__ f, StencilArgs sa,
                                                             const int64_t *__restrict__ keys, int64_t bsz0, int64_t bsz1,
-                                                            int64_t groups_per_xcd)
+                                                            int sh)
 {
     __shared__ GroupLds<T, SG_ST_RBSOR, W, false> L;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t b = blockIdx.x;
-    const int64_t grp = (b & 7) * groups_per_xcd + (b >> 3);
+    const int64_t grp = xcd_run_block(sh);
     group_step<T, SG_ST_RBSOR, W, false>(L, grp, w, lane, nn, n, mask, u, f, u, nullptr, 0, sa, keys, bsz0, bsz1);
 }
 
@@ -1888,8 +1905,7 @@ __global__ __launch_bounds__(64 * W) void rbsor_group_kernel(const int32_t *__re
 // LDS copy of the chunk, x neighbours from the lane's piece and that copy; the rows above and
 // below the chunk are one load by the lanes of rows 0 and 15, the columns beside it one
 // gather by the lanes at the row ends, unless the neighbour is in the group (its column is
-// then read from its LDS copy).  All loads are issued before the barrier.  Workgroup b runs
-// in XCD b & 7, which walks its own contiguous range of the chunks.
+// then read from its LDS copy).  All loads are issued before the barrier.
 // A heat step on a ring of 4001^2 (8.2 M points, FP32) took 114.7 us with the generic kernel
 // (a value per lane and load, the ghost cells by division) and takes 18.3 us: 4.4 TB/s of the
 // slots' 9 bytes.  Two chunks a wave, all their loads first: 18.7 us; four: 20.0 us.
@@ -1900,7 +1916,7 @@ __global__ __launch_bounds__(256) void star2d16_kernel(const int32_t *__restrict
                                                       const uint8_t *__restrict__ mask, const T *src0,
                                                       const T *__restrict__ src1, T *dst0, T *dst1, int alias,
                                                       StencilArgs sa, const int64_t *__restrict__ keys, int64_t bsz0,
-                                                      int64_t per_xcd)
+                                                      int sh)
 {
     constexpr bool kTwo = (KIND == SG_ST_GRAY_SCOTT);
     constexpr bool kRhs = (KIND == SG_ST_RBSOR || KIND == SG_ST_RESIDUAL);
@@ -1913,7 +1929,7 @@ __global__ __launch_bounds__(256) void star2d16_kernel(const int32_t *__restrict
     };
     __shared__ __attribute__((aligned(16))) T tile[G][NP][16 * S];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t c = ((int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3)) * G + w;
+    const int64_t c = xcd_run_block(sh) * G + w;
     const T *src[2] = {src0, src1};
     Piece own[NP][PP], gy[NP][PP], rhs[PP];
     T gx[NP][PP];
@@ -2543,18 +2559,15 @@ int apply_stencil_impl(sg_grid *g, const sg_stencil_desc *d)
                                                      : n * 512 * (int64_t)(2 * sizeof(T) + 1) > (int64_t)640 << 20;
                 auto launch = [&](auto u) {
                     constexpr bool U = decltype(u)::value;
-                    // every XCD gets at least 4 runs, a pair kernel's workgroup 4 chunks
-                    int run = kBoxRunLog;
-                    while (run > (pairs ? 2 : 0) && n < ((int64_t)32 << run)) --run;
-                    const unsigned runs = (unsigned)((n + (8 << run) - 1) / (8 << run) * 8);
+                    const XcdRuns r = pairs ? xcd_runs((n + 3) / 4, kBoxRunLog - 2) : xcd_runs(n, kBoxRunLog);
                     if (pairs)
-                        hipLaunchKernelGGL((box8_pair_kernel<T, U>), dim3(runs << (run - 2)), dim3(128), 0, g->stream, n,
+                        hipLaunchKernelGGL((box8_pair_kernel<T, U>), dim3(r.grid), dim3(128), 0, g->stream, n,
                                            g->d_nn[type], g->d_mask, (const T *)g->d_prop[d->src[0]],
-                                           (T *)g->d_prop[d->dst[0]], g->d_keys, run - 2, ba);
+                                           (T *)g->d_prop[d->dst[0]], g->d_keys, r.sh, ba);
                     else
-                        hipLaunchKernelGGL((box8_kernel<T, U>), dim3(runs << run), dim3(64), 0, g->stream, n,
-                                           g->d_nn[type], g->d_mask, (const T *)g->d_prop[d->src[0]],
-                                           (T *)g->d_prop[d->dst[0]], g->d_keys, run, ba);
+                        hipLaunchKernelGGL((box8_kernel<T, U>), dim3(r.grid), dim3(64), 0, g->stream, n, g->d_nn[type],
+                                           g->d_mask, (const T *)g->d_prop[d->src[0]], (T *)g->d_prop[d->dst[0]],
+                                           g->d_keys, r.sh, ba);
                 };
                 if (uni) launch(std::true_type());
                 else launch(std::false_type());
@@ -2589,30 +2602,34 @@ int apply_stencil_impl(sg_grid *g, const sg_stencil_desc *d)
             if (fast) {
                 const int64_t per_xcd = (n + 7) / 8;
                 const int al = alias[0] != 0;
-                const int64_t gpx4 = ((n + 3) / 4 + 7) / 8;
+                const XcdRuns r4 = xcd_runs((n + 3) / 4, kStarRunLog<T> - 2);
                 // red-black SOR and the residual run in groups of 4 chunks only: the launch
                 // shapes of the variants are tuned for the other three
                 if (kind == SG_ST_RBSOR) {
-                    hipLaunchKernelGGL((rbsor_group_kernel<T, 4>), dim3((unsigned)(gpx4 * 8)), dim3(256), 0, g->stream,
-                                       fnn, n, g->d_mask, o0, s1, sa, g->d_keys, g->bsz[0], g->bsz[1], gpx4);
+                    hipLaunchKernelGGL((rbsor_group_kernel<T, 4>), dim3(r4.grid), dim3(256), 0, g->stream,
+                                       fnn, n, g->d_mask, o0, s1, sa, g->d_keys, g->bsz[0], g->bsz[1], r4.sh);
                     return;
                 }
                 if (kind == SG_ST_RESIDUAL) {
-                    hipLaunchKernelGGL((stencil_group_kernel<T, SG_ST_RESIDUAL, 4, false>), dim3((unsigned)(gpx4 * 8)),
+                    hipLaunchKernelGGL((stencil_group_kernel<T, SG_ST_RESIDUAL, 4, false>), dim3(r4.grid),
                                        dim3(256), 0, g->stream, fnn, n, g->d_mask, s0, s1, o0, o1, al, sa, g->d_keys,
-                                       g->bsz[0], g->bsz[1], gpx4);
+                                       g->bsz[0], g->bsz[1], r4.sh);
                     return;
                 }
                 auto launch = [&](auto kind_tag) {
                     constexpr int K = decltype(kind_tag)::value;
-                    if (g->fast_variant == 0) {
+                    // two FP64 tiles per wave leave 2 waves a SIMD (164 VGPRs), one tile 3:
+                    // Gray-Scott on a shell of 391^3 203 -> 178 us; FP32 148 and 150 us
+                    const int variant = g->fast_variant >= 0 ? g->fast_variant
+                                        : (K == SG_ST_GRAY_SCOTT && sizeof(T) == 8) ? 6 : 3;
+                    if (variant == 0) {
                         // one chunk per 64-lane workgroup
                         hipLaunchKernelGGL((stencil_wave_kernel<T, K>), dim3((unsigned)(per_xcd * 8)), dim3(64), 0,
                                            g->stream, fnn, n, g->d_mask, s0, s1, o0, o1, al, sa, g->d_keys,
                                            g->bsz[0], g->bsz[1], per_xcd);
                         return;
                     }
-                    if (g->fast_variant >= 3) {
+                    if (variant >= 3) {
                         // groups of W consecutive chunks sharing x faces through LDS
                         // (variants 6 / 7 / 8: the same with one LDS tile per wave for both
                         // Gray-Scott properties)
@@ -2620,14 +2637,13 @@ int apply_stencil_impl(sg_grid *g, const sg_stencil_desc *d)
                             constexpr int GW = decltype(wtag)::value;
                             constexpr bool ONE = decltype(onetag)::value;
                             const int64_t ngroups = (n + GW - 1) / GW;
-                            const int64_t gpx = (ngroups + 7) / 8;
-                            hipLaunchKernelGGL((stencil_group_kernel<T, K, GW, ONE>), dim3((unsigned)(gpx * 8)),
-                                               dim3(64 * GW), 0, g->stream, fnn, n, g->d_mask, s0, s1, o0,
-                                               o1, al, sa, g->d_keys, g->bsz[0], g->bsz[1], gpx);
+                            const XcdRuns r = xcd_runs(ngroups, kStarRunLog<T> - (GW == 8 ? 3 : GW == 4 ? 2 : 1));
+                            hipLaunchKernelGGL((stencil_group_kernel<T, K, GW, ONE>), dim3(r.grid), dim3(64 * GW), 0, g->stream, fnn, n, g->d_mask, s0, s1, o0,
+                                               o1, al, sa, g->d_keys, g->bsz[0], g->bsz[1], r.sh);
                         };
                         const std::false_type two_tiles;
                         const std::true_type one_tile;
-                        switch (g->fast_variant) {
+                        switch (variant) {
                         case 3: grouped(std::integral_constant<int, 4>(), two_tiles); break;
                         case 4: grouped(std::integral_constant<int, 8>(), two_tiles); break;
                         case 5: grouped(std::integral_constant<int, 2>(), two_tiles); break;
@@ -2643,7 +2659,7 @@ int apply_stencil_impl(sg_grid *g, const sg_stencil_desc *d)
                         std::max<int64_t>(1, std::min<int64_t>(g->fast_wg_per_xcd, (per_xcd + 3) / 4));
                     const int64_t per_wave = (per_xcd + wg_per_xcd * 4 - 1) / (wg_per_xcd * 4);
                     const unsigned nblk = (unsigned)(wg_per_xcd * 8);
-                    if (g->fast_variant == 1)
+                    if (variant == 1)
                         hipLaunchKernelGGL((stencil_fast_kernel<T, K, 1>), dim3(nblk), dim3(256), 0, g->stream,
                                            fnn, n, g->d_mask, s0, s1, o0, o1, al, sa, g->d_keys, g->bsz[0],
                                            g->bsz[1], per_xcd, per_wave);
@@ -2662,10 +2678,10 @@ int apply_stencil_impl(sg_grid *g, const sg_stencil_desc *d)
             if (fast2) {
                 auto launch = [&](auto kind_tag) {
                     constexpr int K = decltype(kind_tag)::value;
-                    const int64_t per_xcd = ((n + 3) / 4 + 7) / 8;
-                    hipLaunchKernelGGL((star2d16_kernel<T, K>), dim3((unsigned)(per_xcd * 8)), dim3(256), 0,
+                    const XcdRuns r = xcd_runs((n + 3) / 4, kBoxRunLog - 2);
+                    hipLaunchKernelGGL((star2d16_kernel<T, K>), dim3(r.grid), dim3(256), 0,
                                        g->stream, fnn, n, g->d_mask, s0, s1, o0, o1, (int)(alias[0] != 0), sa,
-                                       g->d_keys, g->bsz[0], per_xcd);
+                                       g->d_keys, g->bsz[0], r.sh);
                 };
                 switch (kind) {
                 case SG_ST_LAP: launch(std::integral_constant<int, SG_ST_LAP>()); break;

@@ -96,3 +96,28 @@ def test_many_workgroups(G, oracle, dim, edge, n):
         a.apply_stencil(d)
         b.apply_stencil(d)
     S.assert_same_state(a, b)
+
+
+@pytest.mark.parametrize("dim,edge,dtype", [(3, 8, np.float32), (3, 8, np.float64), (2, 16, np.float32)])
+@pytest.mark.parametrize("nb", [1, 5, 17])
+def test_chunk_runs(G, oracle, dim, edge, dtype, nb):
+    """Chunks dealt to the XCDs in runs: fewer and more than the longest run takes (17^3 and
+    65^2 chunks), with a last run that is not full.  Bit-exact against the oracle."""
+    nb = {17: 65}.get(nb, nb) if dim == 2 else nb
+    size = [nb * edge - 3] * dim
+    rng = np.random.default_rng(nb)
+    pts = rng.integers(0, size[0], (nb ** dim * 9, dim)).astype(np.int32)
+    pts = np.concatenate([pts, pts + np.eye(dim, dtype=np.int32)[0]]).clip(0, size[0] - 1)
+    vals = [rng.uniform(-1, 1, len(pts)).astype(dtype) for _ in range(3)]
+    a, b = (cls(dim, size, [dtype] * 3, block_edge=edge) for cls in (G, oracle.SparseGridCpu))
+    for g in (a, b):
+        g.insert_coords(pts, vals)
+        g.flush(["smax"] * 3)
+        g.find_neighbours(C.NN_STAR)
+    for d in [C.make_desc(C.ST_HEAT, [0], [2], C.APPLY_EXISTING, None, [0.1]),
+              C.make_desc(C.ST_GRAY_SCOTT, [0, 1], [2, 1], C.APPLY_EXISTING, None, [0.2, 0.1, 0.04, 0.06, 0.5]),
+              C.make_desc(C.ST_RBSOR, [2, 0], [], C.APPLY_EXISTING, None, [1.3], [1]),
+              C.make_desc(C.ST_RESIDUAL, [2, 0], [1], C.APPLY_EXISTING, None)]:
+        for g in (a, b):
+            g.apply_stencil(d)
+        S.assert_same_state(a, b)
