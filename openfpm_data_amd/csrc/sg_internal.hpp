@@ -269,6 +269,29 @@ template <typename T> __device__ inline void store_chunk_contig(T *dst, const T 
     }
 }
 
+// Workgroup b runs in XCD b & 7, each with an L2 of its own.  An XCD takes the work of
+// 2^sh consecutive workgroups, then of the next 2^sh after the other XCDs' (a grid of a
+// multiple of 8 * 2^sh workgroups): what neighbouring work shares, lines read by several chunks or
+// written in parts by several tiles, is then in one L2, and the XCDs still walk the same
+// part of memory.
+__device__ __forceinline__ int64_t xcd_run_block(int sh)
+{
+    const uint32_t q = blockIdx.x >> 3;
+    return ((int64_t)((q >> sh) * 8 + (blockIdx.x & 7)) << sh) + (q & ((1u << sh) - 1));
+}
+
+// Runs of up to 2^max_log workgroups, at least 4 for every XCD where there are that many.
+struct XcdRuns {
+    int sh;
+    unsigned grid;
+};
+inline XcdRuns xcd_runs(int64_t nwg, int max_log)
+{
+    int sh = max_log;
+    while (sh > 0 && nwg < ((int64_t)32 << sh)) --sh;
+    return {sh, (unsigned)((nwg + (8 << sh) - 1) / (8 << sh) * (8 << sh))};
+}
+
 // ---- chunk linearizers -----------------------------------------------------------
 // grid_smb (src/Grid/Geometry/grid_smb.hpp:175-297): chunk id row-major, x fastest.
 // grid_zmb (src/Grid/Geometry/grid_zmb.hpp:65-106, util/zmorton.hpp): chunk id = Morton

@@ -244,29 +244,7 @@ struct StencilArgs {
     int64_t icoef[27];
 };
 
-// Workgroup b runs in XCD b & 7, each with an L2 of its own.  An XCD takes the work of
-// 2^sh consecutive workgroups, then of the next 2^sh after the other XCDs' (a grid of a
-// multiple of 8 * 2^sh workgroups): most of the 26 neighbours a chunk reads are then in
-// that L2, and the XCDs still walk the same part of memory.
-__device__ __forceinline__ int64_t xcd_run_block(int sh)
-{
-    const uint32_t q = blockIdx.x >> 3;
-    return ((int64_t)((q >> sh) * 8 + (blockIdx.x & 7)) << sh) + (q & ((1u << sh) - 1));
-}
-
 constexpr int kBoxRunLog = 7;  // 27-point box and 2D kernels: 128 chunks in a row
-
-// Runs of up to 2^max_log workgroups, at least 4 for every XCD where there are that many.
-struct XcdRuns {
-    int sh;
-    unsigned grid;
-};
-XcdRuns xcd_runs(int64_t nwg, int max_log)
-{
-    int sh = max_log;
-    while (sh > 0 && nwg < ((int64_t)32 << sh)) --sh;
-    return {sh, (unsigned)((nwg + (8 << sh) - 1) / (8 << sh) * (8 << sh))};
-}
 
 // generic stencil: one workgroup per chunk, enlarged blocks of up to two
 // properties in dynamic LDS.  dst_alias[q] != 0 means dst q is also a source: it is
