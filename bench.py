@@ -230,8 +230,9 @@ def run_poisson_secondary():
     t_pb, r_pb = timed(C.POISSON_PLAIN_FP64, True, True, tuning)
     sw = np.array([r["sweeps"] for r in r_mix])
     # sweep kernel rate: one outer iteration of K FP32 red-black sweeps over all 256 grids
-    # (no graph: 2 K launches of rbsor_batch_kernel and two defect passes).  Algorithmic bytes
-    # per slot: 13 per half sweep (x read and written, f read, mask), 33 per defect pass.
+    # (no graph: K launches of rbsor_fused_kernel, both colours in one pass, and two defect
+    # passes).  Algorithmic bytes per slot: 13 per sweep (x read and written, f read, mask), 33
+    # per defect pass.
     K = 40
     slots = int(sum(s["chunk_ids"].size for s in specs)) * 512
     gs = grids()
@@ -246,7 +247,7 @@ def run_poisson_secondary():
     for g in gs:
         g.close()
     assert all(r["sweeps"] == K for r in rk)
-    sweep_bytes = slots * (2 * K * 13 + 2 * 33)
+    sweep_bytes = slots * (K * 13 + 2 * 33)
     sweep_gbs = sweep_bytes / t_k / 1e9
     return {"workload": "poisson_batch256", "grids": len(specs),
             "chunks": int(sum(s["chunk_ids"].size for s in specs)), "tol": 1e-10,

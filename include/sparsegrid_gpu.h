@@ -237,7 +237,7 @@ typedef struct {
     int32_t first_sweeps;  /* sweeps of the first block (default 24) */
     int32_t max_sweeps;    /* per grid (default 20000) */
     int32_t max_outer;     /* per grid (default 100) */
-    int32_t use_graph;     /* capture the inner sweep sequence in a hipGraph */
+    int32_t use_graph;     /* capture an inner sweep sequence that comes again in a hipGraph */
 } sg_poisson_params;
 
 typedef struct {

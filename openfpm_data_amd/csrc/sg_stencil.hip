@@ -1885,8 +1885,9 @@ __global__ __launch_bounds__(64 * W) void rbsor_group_kernel(const int32_t *__re
 // gather by the lanes at the row ends, unless the neighbour is in the group (its column is
 // then read from its LDS copy).  All loads are issued before the barrier.
 // A heat step on a ring of 4001^2 (8.2 M points, FP32) took 114.7 us with the generic kernel
-// (a value per lane and load, the ghost cells by division) and takes 18.3 us: 4.4 TB/s of the
-// slots' 9 bytes.  Two chunks a wave, all their loads first: 18.7 us; four: 20.0 us.
+// (a value per lane and load, the ghost cells by division) and takes 17.6 us: 4.5 TB/s of the
+// slots' 9 bytes (18.3 us with one range of chunks per XCD; then, two chunks a wave, all their
+// loads first, 18.7 us and four 20.0 us).
 // src0 is not restrict: red-black SOR writes it in place (other-colour values keep their
 // bits, and only those are used by other waves).
 template <typename T, int KIND>
