@@ -922,15 +922,18 @@ struct FoldState {
     int voff[kMaxProps];
 };
 
+constexpr uint32_t kOutside = 0xffffu;
+
 // Device-coordinate point inserts staged straight as the grouped flush's (chunk id,
 // record) pairs, in insertion order, so that the flush has no insert-buffer pass: the
 // chunk id (as stage_coords_kernel computes the key), then the record: slot offset, mask
 // (masks or EXIST) and each property's value (the source's, or the background) at the
-// layout's offsets.  A coordinate outside the grid gives chunk id 0xffffffff and sets
-// *bad.  A block takes kWG * kStageItems consecutive records, a thread every kWG-th; the
+// layout's offsets.  A coordinate outside the grid gives chunk id 0, slot offset kOutside (no
+// chunk has that many slots) and sets *bad: every staged id is then one of the domain's, so a
+// sort by the domain's id bits leaves no more runs of equal ids than the domain has chunks.
+// A block takes kWG * kStageItems consecutive records, a thread every kWG-th; the
 // records are assembled in registers (the layout is uniform) and stored as 16-byte
 // vectors, a wave's stores covering consecutive records.
-
 template <int NV>
 __global__ __launch_bounds__(kWG) void stage_coord_records_kernel(const int32_t *__restrict__ coords,
                                                                   const uint8_t *__restrict__ masks, int64_t n,
@@ -959,8 +962,9 @@ __global__ __launch_bounds__(kWG) void stage_coord_records_kernel(const int32_t 
         bool ok = i < n;
 #pragma unroll
         for (int d = 0; d < 3; ++d) ok = ok && (d >= dim || (c[t][d] >= 0 && c[t][d] < sz[d]));
-        uint32_t id = 0xffffffffu, l = 0;
+        uint32_t id = 0, l = kOutside;
         if (ok) {
+            l = 0;
             int64_t bc[3] = {0, 0, 0};
 #pragma unroll
             for (int d = 2; d >= 0; --d) {
@@ -1007,8 +1011,8 @@ __global__ __launch_bounds__(kWG) void stage_coord_records_kernel(const int32_t 
     }
 }
 
-// staged (chunk id, record) pairs -> the point insert buffer (key -1 for chunk id
-// 0xffffffff, the mask, each property's value into V.dst)
+// staged (chunk id, record) pairs -> the point insert buffer (key -1 for slot offset
+// kOutside, the mask, each property's value into V.dst)
 __global__ __launch_bounds__(kWG) void point_records_to_buffer_kernel(const uint32_t *__restrict__ ck,
                                                                       const unsigned char *__restrict__ rec, int64_t n,
                                                                       int csz, RecLayout R, StageVals V,
@@ -1018,8 +1022,8 @@ __global__ __launch_bounds__(kWG) void point_records_to_buffer_kernel(const uint
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const unsigned char *d = rec + i * R.bytes;
-    const uint32_t id = ck[i];
-    keys[i] = id == 0xffffffffu ? (int64_t)-1 : (int64_t)id * csz + *(const uint16_t *)d;
+    const uint32_t l = *(const uint16_t *)d;
+    keys[i] = l == kOutside ? (int64_t)-1 : (int64_t)ck[i] * csz + l;
     mask[i] = d[2];
     for (int q = 0; q < V.np; ++q) {
         const unsigned char *f = d + R.off[q];
@@ -1902,7 +1906,7 @@ bool point_record_layout(const sg_grid *g, RecLayout *R, FoldState *S, int *cbit
     int cb = 0;
     while (cb < 63 && (((int64_t)1 << cb) < nblocks)) ++cb;
     *cbits = cb;
-    if (cb > 32 || csz > 65536) return false;
+    if (cb > 32 || csz >= (int)kOutside) return false;
     int at = 3;
     for (int p = 0; p < g->np; ++p) {
         at = (at + g->ts[p] - 1) / g->ts[p] * g->ts[p];
@@ -2760,11 +2764,12 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
     // chunk list.  Up to kBound touched chunks can be expected (by the records and the
     // domain), all of it is queued before the one wait of the flush, on arrays and launches of
     // that bound; beyond, the host waits for their number first (2^20 entries are 46 MB of
-    // temporaries; a wait is some 15 us).  Ids outside the grid lead to no access outside the
-    // arrays: staged ones are one more distinct id, 0xffffffff.
+    // temporaries; a wait is some 15 us).  Records outside the grid carry chunk id 0 (both
+    // kinds), so the runs are distinct ids of the domain, at most its chunks; the flags read
+    // after the wait keep such records from being folded.
     const int64_t rtiles = (n + kRunTile - 1) / kRunTile;
     constexpr int64_t kBound = 1 << 20;
-    int64_t bound = std::min<int64_t>(n, limit / csz + 1);
+    int64_t bound = std::min<int64_t>(n, limit / csz);
     const bool queued = bound <= kBound;
     DevBuf &b_h = g->scratch[4];
     if ((rc = ensure(g->pool, b_h, (size_t)rtiles * 8 + 64))) return rc;

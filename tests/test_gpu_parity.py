@@ -1054,6 +1054,41 @@ def test_device_coordinates_outside_the_grid(G, oracle):
     o.close()
 
 
+@pytest.mark.parametrize("dim,edge,nb,nprop", [(3, 8, 1, 1), (3, 8, 4, 1), (3, 8, 8, 5), (2, 16, 16, 2), (2, 6, 5, 1)])
+@pytest.mark.parametrize("lin", ["smb", "zmb"])
+def test_many_device_coordinates_outside_the_grid(G, oracle, dim, edge, nb, nprop, lin):
+    """Coordinates outside the grid in turn with points of the domain's last chunk (and of
+    others), many more of them than the domain has chunks, in domains of one chunk, of a power
+    of two and of another number: reported and counted, the grid unchanged, the others merged
+    by the next flush as the oracle merges them alone."""
+    import torch
+    from openfpm_data_amd._capi import SgError
+    rng = np.random.default_rng(dim * 100 + nb)
+    side, n = edge * nb, 6000
+    last = rng.integers(side - edge, side, (n, dim))
+    outside = np.where(rng.random((n, dim)) < 0.5, -1 - rng.integers(0, 9, (n, dim)), side + rng.integers(0, 9, (n, dim)))
+    coords = np.stack([last, outside, rng.integers(0, side, (n, dim))], 1).reshape(-1, dim)[:3 * n - 1].astype(np.int32)
+    keep = np.all((coords >= 0) & (coords < side), axis=1)
+    dtypes = [np.float32, np.int32, np.float64, np.uint8, np.int16][:nprop]  # 16-byte records, 32-byte ones with 5
+    vals = [rng.integers(0, 100, len(coords)).astype(t) for t in dtypes]
+    g = G(dim, [side] * dim, dtypes, block_edge=edge, linearizer=lin)
+    o = oracle.SparseGridCpu(dim, [side] * dim, dtypes, block_edge=edge, linearizer=lin)
+    for x in (g, o):
+        x.insert_coords(coords[keep][:7], [v[keep][:7] for v in vals])
+        x.flush(["smax"] * nprop)
+    before = [g.chunk_ids(), g.masks()] + [g.prop(p) for p in range(nprop)]
+    g.insert_coords(torch.from_numpy(coords).cuda(), [torch.from_numpy(v).cuda() for v in vals])
+    with pytest.raises(SgError, match="%d inserted points outside the grid" % n):
+        g.flush(["smax"] * nprop)
+    assert g.pending_inserts() == int(keep.sum())
+    for a, b in zip(before, [g.chunk_ids(), g.masks()] + [g.prop(p) for p in range(nprop)]):
+        np.testing.assert_array_equal(a, b)
+    g.flush(["smax"] * nprop)
+    o.insert_coords(coords[keep], [v[keep] for v in vals])
+    o.flush(["smax"] * nprop)
+    S.assert_same_state(g, o)
+
+
 def test_flush_known_answers_of_the_reference(G):
     """BlockMapGpu_tests.cu:126-264 and BlockMapGpu_kernels_tests.cu:16-492 (segmented fold
     with old data, merge maps, conflict resolution), end to end through insert + flush on
