@@ -2683,7 +2683,7 @@ int flush_chunks_impl(sg_grid *g, const int32_t *ops)
                        g->d_cins_mask, g->d_mask);
     SG_HIP(hipGetLastError());
     g->cins_n = 0;
-    g->nn_valid[0] = g->nn_valid[1] = false;
+    g->chunks_changed();
     g->occ_tab_valid = false;
     g->ebits_valid = false;
     g->ep_valid = false;
@@ -2941,7 +2941,7 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
     finish_merge(g, df);
     g->ins_n = 0;
     g->pins_n = 0;
-    g->nn_valid[0] = g->nn_valid[1] = false;
+    g->chunks_changed();
     g->occ_tab_valid = false;
     g->ebits_valid = planes;
     g->ep_valid = false;
@@ -3141,7 +3141,7 @@ int flush_impl(sg_grid *g, const int32_t *ops)
     }
     g->ins_n = 0;
     // flush marks the neighbour table stale (SparseGridGpu.hpp:778), and the point list
-    g->nn_valid[0] = g->nn_valid[1] = false;
+    g->chunks_changed();
     g->occ_tab_valid = false;
     g->ebits_valid = false;
     g->ep_valid = false;
@@ -3238,7 +3238,7 @@ int set_chunks_impl(sg_grid *g, int64_t n, const int64_t *ids, const uint8_t *ma
     for (int p = 0; p < g->np; ++p) g->d_prop[p] = nprop[p];
     g->nchunks = n;
     g->cap = ncap;
-    g->nn_valid[0] = g->nn_valid[1] = false;
+    g->chunks_changed();
     g->occ_tab_valid = false;
     g->ebits_valid = false;
     g->ep_valid = false;

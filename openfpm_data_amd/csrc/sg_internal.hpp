@@ -116,6 +116,13 @@ struct sg_grid {
     int32_t *d_nn[2] = {nullptr, nullptr};
     int64_t nn_cap[2] = {0, 0};
     bool nn_valid[2] = {false, false};
+    // counts the changes of the chunk set: tables made from it elsewhere compare it
+    uint64_t chunks_gen = 0;
+    void chunks_changed()
+    {
+        nn_valid[0] = nn_valid[1] = false;
+        ++chunks_gen;
+    }
     int ghost_type = SG_NN_STAR;
 
     // insert buffer (point records)

@@ -41,7 +41,7 @@ struct PGrid {
     double omega;
     int64_t n;            // chunks
     int32_t nsweeps;      // sweeps of this grid in the current inner block
-    // fused sweeps (mixed form): x's second buffer, the chunks' 18 neighbours, and whether both
+    // fused sweeps (mixed form): x's second buffer, the chunks' 18 neighbours, and whether they
     // are still to be set up
     float *x2;
     int32_t *nb;
@@ -251,9 +251,10 @@ constexpr int kNb = 20;  // entries per chunk: -x +x -y +y -z +z, xy, xz, yz edg
 // 16-byte read of each of the four, with no selection.
 constexpr int kFS = 12;
 
-// neighbour tables and zeroed second buffers of the grids that joined the batch (one wave
-// per chunk): edge neighbour (a, b) is b's neighbour of a's neighbour, or where that is
-// missing a's of b's; the background chunk where neither exists
+// neighbour tables and the second buffers' background chunks of the grids that joined the
+// batch or whose chunk set changed (one wave per chunk): edge neighbour (a, b) is b's
+// neighbour of a's neighbour, or where that is missing a's of b's; the background chunk where
+// neither exists.  The second buffers' other chunks are first written by the sweeps.
 __global__ __launch_bounds__(256) void fused_prep_kernel(const PGrid *__restrict__ grids,
                                                          const int64_t *__restrict__ prefix,
                                                          const int32_t *__restrict__ tile_grid, int64_t ntiles)
@@ -265,11 +266,8 @@ __global__ __launch_bounds__(256) void fused_prep_kernel(const PGrid *__restrict
     const PGrid &g = grids[gi];
     if (!g.prep) return;
     const int64_t c = t - prefix[gi];
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 *p = (float4 *)(g.x2 + c * 512);
-    p[lane] = zero;
-    p[64 + lane] = zero;
     if (c == 0) {
+        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
         float4 *b = (float4 *)(g.x2 + g.n * 512);
         b[lane] = zero;
         b[64 + lane] = zero;
@@ -409,9 +407,10 @@ __device__ __forceinline__ void fused_compute(FusedIn &in, float *tile, int lane
     sor_row<EXACT>(in.c1, in.c0, in.b1, xn, !s, tile + own, in.mrow, wgt, small);
 }
 
-// both colours on chunk c of grid g (fewer than 2^21 chunks: 32-bit byte offsets): src -> dst
+// both colours on chunk c of grid g (fewer than 2^21 chunks: 32-bit byte offsets): src -> dst,
+// the rows with a point and those of `every`
 __device__ __forceinline__ void fused_tile(const PGrid &g, uint32_t c, float *tile, int lane, int zero_x,
-                                           const float *src, float *dst)
+                                           const float *src, float *dst, uint64_t every)
 {
     const int32_t *nb = as_global(g.nb) + (size_t)c * kNb;
     const float *rhs = (const float *)as_global(g.rhs);
@@ -498,9 +497,9 @@ __device__ __forceinline__ void fused_tile(const PGrid &g, uint32_t c, float *ti
         wave_sync_lds();
         fused_compute<true>(in, tile, lane, wgt, &small);
     }
-    const uint64_t rows = __ballot(in.mrow != 0);
+    const uint64_t rows = __ballot(in.mrow != 0) | every;
     wave_sync_lds();
-    // back in row order, and out as lane-contiguous 16-byte stores of the rows with a point
+    // back in row order, and out as lane-contiguous 16-byte stores
     *(float4 *)(tile + lane * 8) = make_float4(sel(s, in.c1[0], in.c0[0]), sel(s, in.c0[0], in.c1[0]),
                                                sel(s, in.c1[1], in.c0[1]), sel(s, in.c0[1], in.c1[1]));
     *(float4 *)(tile + lane * 8 + 4) = make_float4(sel(s, in.c1[2], in.c0[2]), sel(s, in.c0[2], in.c1[2]),
@@ -530,10 +529,12 @@ __global__ __launch_bounds__(64 * WAVES) void rbsor_fused_kernel(const PGrid *__
     auto tile = [&](int64_t t) __attribute__((always_inline)) {
         const int gi = tile_grid[t];
         const PGrid &g = grids[gi];
-        // the block's last sweep writes x
+        // the block's last sweep writes x.  The rows without a point hold zeros in x, but in x2
+        // whatever they held when they last had one: a block's first sweep into x2 writes all rows
         const bool to2 = ((g.nsweeps - 1 - sweep) & 1) != 0;
         float *x = (float *)as_global(g.x), *x2 = as_global(g.x2);
-        fused_tile(g, (uint32_t)(t - prefix[gi]), tiles[w], lane, zero_x, to2 ? x : x2, to2 ? x2 : x);
+        fused_tile(g, (uint32_t)(t - prefix[gi]), tiles[w], lane, zero_x, to2 ? x : x2, to2 ? x2 : x,
+                   to2 && sweep < 2 ? ~0ull : 0ull);
     };
     int64_t t = (int64_t)blockIdx.x * WAVES + w;
     if constexpr (LOOP) {
@@ -699,10 +700,11 @@ struct sg_batch {
         int inner = 0;  // inner sweeps for the next outer iteration
         double tol = 0.0;
         // fused sweeps: second x buffer and neighbour table (from the batch's pool; null: the
-        // grid cannot take them), still to be set up
+        // grid cannot take them) for the chunk set of that count, still to be set up
         float *x2 = nullptr;
         int32_t *nb = nullptr;
         bool prep = false;
+        uint64_t chunks_gen = 0;
     };
     std::vector<Entry> live;
     std::vector<std::pair<int64_t, sg_poisson_result>> done;
@@ -996,6 +998,48 @@ double omega_from_rate(double rho, double w0)
     return 2.0 / (1.0 + std::sqrt(1.0 - mu * mu));
 }
 
+void free_fused(sg_batch *b, sg_batch::Entry &en)
+{
+    // stream order: reused only by work queued on the batch's stream after this
+    b->pool.free(en.x2);
+    b->pool.free(en.nb);
+    en.x2 = nullptr;
+    en.nb = nullptr;
+}
+
+// What the batch keeps for a grid's fused sweeps, when the grid joins and before each step: a
+// program may change a live grid between two steps, and the second buffer and the neighbour
+// table are those of one chunk set.  Fused sweeps keep e = 0 where no point is, and take 2.1 KB
+// a chunk of the batch's memory; a grid that does not fit makes its steps run half sweeps.
+int fused_state(sg_batch *b, sg_batch::Entry &en)
+{
+    sg_grid *g = en.g;
+    const sg_poisson_params &p = b->p;
+    const bool changed = en.chunks_gen != g->chunks_gen;
+    if (changed) {
+        if (!g->nn_valid[SG_NN_STAR]) {
+            const int rc = find_neighbours_impl(g, SG_NN_STAR);
+            if (rc) return rc;
+        }
+        // the grid's own queued work must be done before the batch stream uses it
+        SG_HIP(hipStreamSynchronize(g->stream));
+    }
+    static const unsigned char zero[8] = {};
+    const bool fits = p.mode == SG_POISSON_MIXED && g->nchunks > 0 && g->nchunks < (1 << 21) - 1 &&
+                      memcmp(g->bg[p.e_prop], zero, sizeof(float)) == 0;
+    if (!changed && (fits || !en.x2)) return SG_OK;
+    ++b->version;
+    free_fused(b, en);
+    en.prep = false;
+    en.chunks_gen = g->chunks_gen;
+    if (!fits) return SG_OK;
+    en.x2 = (float *)b->pool.alloc((size_t)(g->nchunks + 1) * 512 * sizeof(float));
+    en.nb = (int32_t *)b->pool.alloc((size_t)g->nchunks * kNb * sizeof(int32_t));
+    if (!en.x2 || !en.nb) free_fused(b, en);
+    en.prep = en.x2 != nullptr;
+    return SG_OK;
+}
+
 void retire(sg_batch *b, size_t i, int converged)
 {
     sg_batch::Entry &en = b->live[i];
@@ -1007,11 +1051,7 @@ void retire(sg_batch *b, size_t i, int converged)
     r.omega = en.omega;
     r.solution_prop = en.cur_u;
     b->done.emplace_back(en.tag, r);
-    // stream order: reused only by work queued on the batch's stream after this
-    b->pool.free(en.x2);
-    b->pool.free(en.nb);
-    en.x2 = nullptr;
-    en.nb = nullptr;
+    free_fused(b, en);
 }
 
 }  // namespace
@@ -1065,12 +1105,6 @@ int sg_batch_add(sg_batch *b, sg_grid *g, int64_t tag, double tol)
     if (!need(p.u_prop, SG_F64) || !need(p.f_prop, SG_F64) ||
         (mixed && (!need(p.u2_prop, SG_F64) || !need(p.e_prop, SG_F32) || !need(p.r_prop, SG_F32))))
         return fail(SG_E_ARG, "grid properties do not match the solver layout (u, u2, f: f64; e, r: f32)");
-    if (!g->nn_valid[SG_NN_STAR]) {
-        int rc = find_neighbours_impl(g, SG_NN_STAR);
-        if (rc) return rc;
-    }
-    // the grid's own queued work must be done before the batch stream uses it
-    SG_HIP(hipStreamSynchronize(g->stream));
     sg_batch::Entry en;
     en.g = g;
     en.tag = tag;
@@ -1078,21 +1112,9 @@ int sg_batch_add(sg_batch *b, sg_grid *g, int64_t tag, double tol)
     en.omega = (p.omega > 0.0) ? p.omega : p.omega0;
     en.inner = p.first_sweeps;
     en.tol = (tol > 0.0) ? tol : p.tol;
-    // Fused sweeps keep e = 0 where no point is (as the second buffer has it), and take
-    // 2.1 KB a chunk of the batch's memory; a grid that does not fit makes its steps run half
-    // sweeps.
-    static const unsigned char zero[8] = {};
-    if (mixed && g->nchunks > 0 && g->nchunks < (1 << 21) - 1 && memcmp(g->bg[p.e_prop], zero, sizeof(float)) == 0) {
-        en.x2 = (float *)b->pool.alloc((size_t)(g->nchunks + 1) * 512 * sizeof(float));
-        en.nb = (int32_t *)b->pool.alloc((size_t)g->nchunks * kNb * sizeof(int32_t));
-        if (!en.x2 || !en.nb) {
-            b->pool.free(en.x2);
-            b->pool.free(en.nb);
-            en.x2 = nullptr;
-            en.nb = nullptr;
-        }
-        en.prep = en.x2 != nullptr;
-    }
+    en.chunks_gen = g->chunks_gen + 1;
+    const int rc = fused_state(b, en);
+    if (rc) return rc;
     b->live.push_back(en);
     b->dirty = true;
     ++b->version;
@@ -1127,8 +1149,10 @@ int sg_batch_step(sg_batch *b)
     if (b->live.empty()) return SG_OK;
     const bool mixed = b->p.mode == SG_POISSON_MIXED;
     std::vector<double> norms;
-    int rc = defect_and_norms(b, norms, true);
-    if (rc) return rc;
+    int rc;
+    for (auto &en : b->live)
+        if ((rc = fused_state(b, en))) return rc;
+    if ((rc = defect_and_norms(b, norms, true))) return rc;
     // convergence / retirement
     std::vector<sg_batch::Entry> keep;
     for (size_t i = 0; i < b->live.size(); ++i) {

@@ -209,3 +209,61 @@ def test_grids_without_fused_sweeps(P, oracle):
     rm = P.solve(mixed, P.make_params(tol=1e-8, max_outer=30))
     assert ra[0]["converged"] and rm[0]["converged"] and ra[0]["sweeps"] == rm[0]["sweeps"]
     np.testing.assert_array_equal(alone[0].prop(ra[0]["solution_prop"]), mixed[0].prop(rm[0]["solution_prop"]))
+
+
+@pytest.mark.parametrize("sweeps", [1, 2, 5, 8])
+def test_live_grid_changed_between_steps(P, sweeps):
+    """Points removed (whole rows and a whole chunk), a chunk set that grows, shrinks again and
+    a background of e that comes and goes, each between two steps of a live grid: the bits of
+    half sweeps, which a mate with another background of e makes the step run."""
+    import torch
+    rng = np.random.default_rng(sweeps)
+    n = 48
+    boxes = [(0, 0, 0), (1, 0, 0), (1, 1, 0), (1, 1, 1), (2, 1, 1), (4, 4, 4)]
+    cells = np.stack(np.meshgrid(*[np.arange(8)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    pts = np.concatenate([cells + 8 * np.array(b) for b in boxes]).astype(np.int32)
+    more = np.concatenate([cells + 8 * np.array(b) for b in [(2, 0, 0), (0, 1, 1), (5, 5, 5)]]).astype(np.int32)
+    f, f2 = rng.uniform(-1, 1, len(pts)), rng.uniform(-1, 1, len(more))
+    mate_spec = _small_grids(1, 5, 32)[0]
+
+    def grid_values(half):
+        from openfpm_data_amd import SparseGridGpu
+        g = SparseGridGpu(3, (n,) * 3, P.POISSON_PROPS)
+        put = lambda c, v: (g.insert_coords(c, [0 * v, 0 * v, v] + [np.zeros(len(c), np.float32)] * 2),  # noqa: E731
+                            g.flush(["sright"] * 5))
+        put(pts, f)
+        b = P.PoissonBatch(P.make_params(tol=1e-300, omega=1.4, first_sweeps=sweeps, inner_target=0.3, max_outer=9,
+                                         use_graph=sweeps % 2 == 0))
+        b.add(g, 0)
+        mate = P.poisson_grid(mate_spec["size"], mate_spec["chunk_ids"], mate_spec["f"])
+        if half:
+            mate.set_background_value(P.E, 0.5)
+        b.add(mate, 1)
+        seen = []
+        for step in range(8):
+            b.step()
+            torch.cuda.synchronize()
+            seen.append([g.prop(P.U), g.prop(P.U2), g.prop(P.E), g.prop(P.R)])
+            if step == 1:  # rows and a chunk without a point
+                gone = pts[(pts[:, 1] % 8 == 3) | (pts[:, 0] >= 32) | ((pts[:, 0] < 8) & (pts[:, 2] > 2))]
+                g.remove_points(g.lin_id(gone))
+            elif step == 3:
+                put(more, f2)
+            elif step == 4:
+                g.set_background_value(P.E, 0.25)
+            elif step == 5:
+                g.set_background_value(P.E, 0.0)
+            elif step == 6:
+                keep = np.ascontiguousarray(g.chunk_ids()[::2])
+                m = np.ascontiguousarray(g.masks()[::2])
+                vals = [g.prop(p)[::2] for p in range(5)]
+                C.check(g._lib.sg_set_chunks(g._h, len(keep), keep.ctypes.data, m.ctypes.data, C.SG_MEM_HOST))
+                for p in range(5):
+                    g.set_prop(p, vals[p])
+            torch.cuda.synchronize()
+        b.close()
+        return seen
+
+    for a, h in zip(grid_values(False), grid_values(True)):
+        for x, y in zip(a, h):
+            np.testing.assert_array_equal(x.view(np.uint8), y.view(np.uint8))
