@@ -2787,13 +2787,32 @@ int normalize_prop(sg_grid *g, int p)
     return SG_OK;
 }
 
+// whether the `bytes` bytes at p lie in one allocation of the device that holds `own`
+static bool in_device_memory(const void *p, size_t bytes, const void *own)
+{
+    hipPointerAttribute_t a, o;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess && hipPointerGetAttributes(&o, own) == hipSuccess &&
+        a.type == hipMemoryTypeDevice && a.device == o.device &&
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) == hipSuccess)
+        return (const char *)p + bytes <= (const char *)base + size;
+    (void)hipGetLastError();
+    return false;
+}
+
 int set_prop_device(sg_grid *g, int p, const void *in)
 {
     const int64_t total = g->nchunks * g->csz;
     if (total == 0) return SG_OK;
-    if ((uintptr_t)in % (size_t)g->ts[p]) {
-        // not even aligned to a value
-        SG_HIP(hipMemcpyAsync(g->d_prop[p], in, (size_t)total * g->ts[p], hipMemcpyDeviceToDevice, g->stream));
+    if ((uintptr_t)in % (size_t)g->ts[p] || !in_device_memory(in, (size_t)total * g->ts[p], g->d_prop[p])) {
+        // Not even aligned to a value, or not all in this device's memory: the runtime copies
+        // what it can reach (host memory, another device's) and refuses the rest.
+        const hipError_t e = hipMemcpyAsync(g->d_prop[p], in, (size_t)total * g->ts[p], hipMemcpyDeviceToDevice, g->stream);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();  // reported here, not by the caller's next call
+            return fail(SG_E_HIP, std::string("set_prop from device memory: ") + hipGetErrorString(e));
+        }
         return normalize_prop(g, p);
     }
     dispatch_type(g->dt[p], [&](auto tag) {

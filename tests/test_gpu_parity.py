@@ -1167,3 +1167,56 @@ def test_set_prop_from_device_memory(G, dtype, edge, dim):
         want = part.cpu().numpy().view(dtype).copy()
         want[m == 0] = 7
         np.testing.assert_array_equal(g.prop(0).reshape(-1).view(np.uint8), want.view(np.uint8))
+
+
+def test_set_prop_checks_device_memory(G):
+    """A tensor without room for the values is refused before any of it is read, as is memory
+    that ends before them in the C call; larger tensors, other types of the same bytes and
+    pinned host memory are taken, also in a captured graph."""
+    import torch
+    rng = np.random.default_rng(3)
+    g = G(3, (64, 64, 64), [np.float32])
+    g.insert_coords(rng.integers(0, 64, (4000, 3)).astype(np.int32), [np.zeros(4000, np.float32)])
+    g.flush(["smax"])
+    m = g.masks().reshape(-1) != 0
+    n = m.size
+    x = torch.from_numpy(rng.uniform(1, 2, n + 100).astype(np.float32)).cuda()
+    for short in (x[101:], torch.zeros(1, device="cuda").expand(n), x[:n // 2].clone(), x.to(torch.float16)):
+        with pytest.raises(ValueError):
+            g.set_prop(0, short)
+    assert (g.prop(0) == 0).all()
+
+    def check(start):
+        np.testing.assert_array_equal(g.prop(0).reshape(-1), np.where(m, x.cpu().numpy()[start:start + n], 0))
+
+    g.set_prop(0, x)
+    check(0)
+    g.set_prop(0, x[100:].view(torch.int32))
+    check(100)
+    pin = torch.empty(n, dtype=torch.float32, pin_memory=True)
+    pin.copy_(x[7:n + 7])
+    C.check(g._lib.sg_set_prop(g._h, 0, ctypes.c_void_p(pin.data_ptr()), C.SG_MEM_DEVICE))
+    check(7)
+    # an allocation of its own that ends before the values do
+    raw, small = G(2, (16, 16), [np.float32], block_edge=16), 16 * 16
+    raw.insert_coords([[0, 0]], [np.ones(1, np.float32)])
+    raw.flush(["smax"])
+    assert n > 100 * small
+    from openfpm_data_amd._capi import SgError
+    with pytest.raises(SgError):
+        C.check(g._lib.sg_set_prop(g._h, 0, ctypes.c_void_p(raw.device_ptr(0)), C.SG_MEM_DEVICE))
+    check(7)
+    s = torch.cuda.Stream()
+    g.set_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        g.set_prop(0, x[4:])
+    g.synchronize()
+    check(7)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        check(4)
+        g.set_prop(0, x)
+        g.synchronize()
+        check(0)
