@@ -173,6 +173,19 @@ void DevicePool::free(void *p)
     cache_.emplace(it->second, p);
 }
 
+void DevicePool::hand_back(void *p)
+{
+    auto it = p ? sizes_.find(p) : sizes_.end();
+    if (it == sizes_.end()) return;
+    {
+        std::lock_guard<std::mutex> lk(g_idle_mu);
+        g_idle.emplace(it->second, std::make_pair(p, devs_[p]));
+    }
+    live_ -= it->second;
+    sizes_.erase(it);
+    devs_.erase(p);
+}
+
 void DevicePool::release()
 {
     {

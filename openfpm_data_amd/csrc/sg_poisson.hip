@@ -998,11 +998,13 @@ double omega_from_rate(double rho, double w0)
     return 2.0 / (1.0 + std::sqrt(1.0 - mu * mu));
 }
 
+// The batch's stream is idle: the blocks go where every pool can take them and sg_trim frees
+// them.  In the batch's own pool they would stay as long as the batch lives, which a server's
+// does, and only other grids of about their size could use them.
 void free_fused(sg_batch *b, sg_batch::Entry &en)
 {
-    // stream order: reused only by work queued on the batch's stream after this
-    b->pool.free(en.x2);
-    b->pool.free(en.nb);
+    b->pool.hand_back(en.x2);
+    b->pool.hand_back(en.nb);
     en.x2 = nullptr;
     en.nb = nullptr;
 }
@@ -1029,7 +1031,10 @@ int fused_state(sg_batch *b, sg_batch::Entry &en)
                       memcmp(g->bg[p.e_prop], zero, sizeof(float)) == 0;
     if (!changed && (fits || !en.x2)) return SG_OK;
     ++b->version;
-    free_fused(b, en);
+    if (en.x2) {
+        SG_HIP(hipStreamSynchronize(b->stream));  // sweeps of the last step
+        free_fused(b, en);
+    }
     en.prep = false;
     en.chunks_gen = g->chunks_gen;
     if (!fits) return SG_OK;
@@ -1040,6 +1045,7 @@ int fused_state(sg_batch *b, sg_batch::Entry &en)
     return SG_OK;
 }
 
+// after the wait for the norms that decide it
 void retire(sg_batch *b, size_t i, int converged)
 {
     sg_batch::Entry &en = b->live[i];

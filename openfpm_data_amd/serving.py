@@ -43,8 +43,9 @@ CHUNK_BYTES = 8 + 8 * 4
 BATCH_CHUNK_BYTES = 512 * 4 + 20 * 4
 # Freeing and reallocating some 35 blocks takes a small grid's build longer than its kernels
 # (0.75 ms against 0.5 ms), so temporaries of up to KEEP_TEMPORARIES stay with the grid, booked,
-# and pass to later grids when it closes; after KEEP_BYTES of grids built so, a trim returns
-# what nobody uses.
+# and pass to later grids when it closes.  What served grids gave back is held idle, unbooked,
+# until a build's trim frees it: with KEEP_BYTES of it, or as soon as it and the booked bytes
+# pass the budget.
 KEEP_TEMPORARIES = 32 << 20
 KEEP_BYTES = 256 << 20
 
@@ -65,7 +66,8 @@ def build_bytes(nchunks):
 class Admission:
     """FIFO admission against a byte budget.  ``reserve`` is booked at admission (footprint
     while building), ``settle`` replaces it with the measured resident size, ``release``
-    returns it."""
+    returns it; the device memory itself then counts as idle until a trim (``take_trim``,
+    called by the thread that builds)."""
 
     def __init__(self, budget_bytes):
         self.budget = int(budget_bytes)
@@ -73,6 +75,8 @@ class Admission:
         self.peak = 0
         self.queue = collections.deque()
         self.booked = {}
+        self.idle = 0  # bytes given back since the last trim
+        self.lock = threading.Lock()
 
     def arrive(self, req):
         self.queue.append(req)
@@ -106,7 +110,18 @@ class Admission:
         self.peak = max(self.peak, self.used)
 
     def release(self, req_id):
-        self.used -= self.booked.pop(req_id)
+        n = self.booked.pop(req_id)
+        self.used -= n
+        with self.lock:
+            self.idle += n
+
+    def take_trim(self, force=False):
+        """Whether the idle memory is to be freed now; it then counts as freed."""
+        with self.lock:
+            due = force or self.idle > KEEP_BYTES or self.used + self.idle > self.budget
+            if due:
+                self.idle = 0
+            return due
 
 
 def grid_device_bytes(grid):
@@ -138,7 +153,6 @@ class PoissonServer:
         self.adm = Admission(budget_bytes)
         self.keep = keep_solutions
         self.threaded = build_thread
-        self._kept = 0  # bytes of the grids built since the last trim
 
     def close(self):
         self.batch.close()
@@ -154,10 +168,8 @@ class PoissonServer:
             del f, ids
         n = len(req["chunk_ids"])
         held = grid_device_bytes(g)
-        self._kept += held
-        if held - resident_bytes(n) > KEEP_TEMPORARIES or self._kept > KEEP_BYTES:
+        if self.adm.take_trim(force=held - resident_bytes(n) > KEEP_TEMPORARIES):
             C.check(C.load().sg_trim(g._h))
-            self._kept = 0
         else:
             g.synchronize()
         if stream is not self.stream:

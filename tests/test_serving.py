@@ -46,6 +46,64 @@ def test_admission_head_of_line_and_reject():
     assert [r["id"] for r in got] == [0]
 
 
+def test_idle_memory_is_bounded():
+    """What served grids of uneven sizes give back is trimmed by a build: with KEEP_BYTES of it,
+    or where it and the booked bytes would pass the budget."""
+    a = S.Admission(4 * S.KEEP_BYTES)
+    sizes = [S.KEEP_BYTES // 3, S.KEEP_BYTES // 3, S.KEEP_BYTES, 3 * S.KEEP_BYTES, S.KEEP_BYTES // 2]
+    for i, n in enumerate(sizes):
+        a.booked[i] = n
+    a.used = sum(sizes[:3])
+    assert not a.take_trim()
+    a.release(0)
+    a.release(1)
+    assert a.idle == sizes[0] + sizes[1] and not a.take_trim()  # two thirds: kept
+    a.release(2)
+    assert a.take_trim() and a.idle == 0 and not a.take_trim()
+    a.used = sizes[3] + sizes[4]
+    a.release(4)
+    assert not a.take_trim()  # half of KEEP_BYTES, and the budget has room
+    a.used += S.KEEP_BYTES // 2 + 1
+    assert a.take_trim()
+    a.booked[5] = 1
+    a.release(5)
+    assert a.take_trim(force=True) and a.idle == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("build_thread", [True, False])
+def test_served_memory_is_returned(build_thread):
+    """While a server lives, the device memory of the grids that it served, its batch's sweep
+    buffers among it, can be freed by a trim: nothing of it stays with the batch."""
+    import torch
+    from openfpm_data_amd import _capi as C
+    from openfpm_data_amd import poisson as P
+
+    rng = np.random.default_rng(2)
+    tiny = P.poisson_grid((32,) * 3, np.arange(64), rng.uniform(-1, 1, (64, 512)))
+    srv = S.PoissonServer(budget_bytes=8 << 30, build_thread=build_thread)
+    reqs = []
+    for i, edge in enumerate((96, 224, 64, 160, 128)):
+        n = (edge // 8) ** 3
+        reqs.append({"id": i, "size": (edge,) * 3, "chunk_ids": np.arange(n),
+                     "f": rng.uniform(-1, 1, (n, 512)).astype(np.float32), "tol": 1e-2})
+    srv.run(reqs[2:3], [0.0])  # code objects, streams
+
+    def free_bytes():
+        C.check(C.load().sg_trim(tiny._h))
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        return torch.cuda.mem_get_info()[0]
+
+    before = free_bytes()
+    recs, summ = srv.run(reqs, [0.0] * len(reqs))
+    assert summ["served"] == len(reqs)
+    # the batch's sweep buffers of the grids are 75 MB; its work lists may grow by 0.8 MB
+    chunks = sum(len(r["chunk_ids"]) for r in reqs)
+    assert before - free_bytes() < min(16 << 20, chunks * S.BATCH_CHUNK_BYTES // 4)
+    srv.close()
+
+
 def test_arrivals_are_poisson():
     t = S.poisson_arrivals(20000, 50.0, 7)
     gaps = np.diff(np.concatenate([[0.0], t]))
