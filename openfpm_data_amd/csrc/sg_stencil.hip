@@ -2566,7 +2566,15 @@ int apply_stencil_impl(sg_grid *g, const sg_stencil_desc *d)
     const bool fast2 = g->dim == 2 && g->edge == 16 && type == SG_NN_STAR && kind != SG_ST_BOX && alias_ok && !sor_self;
     // the fast kernels take the star table, or with lskip >= 2 the occupancy table
     const int32_t *fnn = g->d_nn[type];
-    if (fast && g->fast_lskip >= 2) {
+    if (fast && (kind == SG_ST_RBSOR || kind == SG_ST_RESIDUAL) && sa.lskip >= 2) {
+        // A captured sweep or residual reads the masks when it is replayed, as the generic kernel
+        // that took these before does: the occupancy table is built by the host, once, and
+        // building it may allocate.
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (g->stream) SG_HIP(hipStreamIsCapturing(g->stream, &cap));
+        if (cap != hipStreamCaptureStatusNone) sa.lskip = 0;
+    }
+    if (fast && sa.lskip >= 2) {
         if ((rc = occ_table_impl(g))) return rc;
         fnn = g->d_occ_tab;
         sa.mplanes = g->d_mplanes;

@@ -121,3 +121,36 @@ def test_chunk_runs(G, oracle, dim, edge, dtype, nb):
         for g in (a, b):
             g.apply_stencil(d)
         S.assert_same_state(a, b)
+
+
+@pytest.mark.parametrize("skip", [0, 1, 2, 3, 4])
+def test_captured_sweeps_follow_the_masks(G, oracle, skip):
+    """A sweep and a residual captured before any table of the skip modes exists, replayed after
+    tags and points have changed: every replay does what the oracle does on the masks of then."""
+    import torch
+    a, b = _pair(G, oracle, 3, 8, (41, 30, 25), np.float64, 9, tag=False)
+    s = torch.cuda.Stream()
+    a.set_stream(s)
+    a.set_tuning(C.TUNE_STENCIL_SKIP_EMPTY_ROWS, skip)
+    descs = [C.make_desc(C.ST_RBSOR, [2, 0], [], C.APPLY_INTERIOR, None, [1.3], [0]),
+             C.make_desc(C.ST_RBSOR, [2, 0], [], C.APPLY_INTERIOR, None, [1.3], [1]),
+             C.make_desc(C.ST_RESIDUAL, [2, 0], [1], C.APPLY_INTERIOR)]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        for d in descs:
+            a.apply_stencil(d)
+    rng = np.random.default_rng(2)
+    for step in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        for d in descs:
+            b.apply_stencil(d)
+        S.assert_same_state(a, b)
+        if step == 0:
+            for g in (a, b):
+                g.tag_boundaries(C.NN_STAR)
+        else:
+            keys = rng.choice(a.num_chunks() * 512, 900, replace=False)
+            keys = a.chunk_ids()[keys // 512] * 512 + keys % 512
+            for g in (a, b):
+                g.remove_points(keys)
