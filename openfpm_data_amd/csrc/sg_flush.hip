@@ -2817,6 +2817,9 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
     // records a chunk a wave per chunk reads and writes it whole at the copy's rate.
     const bool few = n <= kFewRecords * nnew && (int64_t)hw[0] < nnew && ((csz % 16) == 0 || hw[0] == 0);
     df.copy_touched = few;
+    // the list of chunks with more records: allocated before the chunk set changes, so that a
+    // failure leaves the grid and the pending records as they are
+    if (few && (rc = ensure(g->pool, g->scratch[8], (size_t)(nnew + 1) * 4))) return rc;
     int64_t *cpos = nullptr;
     if ((rc = merge_grow(g, ML, nnew, hw[0], &cpos, &df))) return rc;
     const bool planes = df.planes;
@@ -2893,7 +2896,6 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
     const bool use_few = few && (df.nfresh == 0 || fresh_ok);
     uint32_t *list = nullptr;
     if (use_few) {
-        if ((rc = ensure(g->pool, g->scratch[8], (size_t)(nnew + 1) * 4))) return rc;
         list = (uint32_t *)g->scratch[8].p;
         hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(1), dim3(64), 0, g->stream, list, 0u, (int64_t)1);
         auto launch = [&](auto kern) {
