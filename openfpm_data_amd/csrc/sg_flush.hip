@@ -1184,6 +1184,7 @@ __device__ inline uint32_t exist_byte(uint64_t row)
 // and written once, contiguously.  Where the chunk set did not grow the chunk stays in
 // place, and only the 16-byte vectors a record reached are read and written (the records
 // of fold_few_records_kernel's figures took 114 us with every chunk written whole, 101 us so).
+// In place omask is I.smask, and the values are read and written through one array too.
 template <int NV>
 __global__ __launch_bounds__(256) void fold_chunk_records_kernel(const uint4 *__restrict__ rec,
                                                                  const uint32_t *__restrict__ ustart,
@@ -1192,7 +1193,7 @@ __global__ __launch_bounds__(256) void fold_chunk_records_kernel(const uint4 *__
                                                                  const uint32_t *__restrict__ isnew, int64_t nnew,
                                                                  int csz, int obits, int waves, FoldState S,
                                                                  FoldProps F, RecLayout R, FusedImg I,
-                                                                 uint8_t *__restrict__ omask, int skip_fresh,
+                                                                 uint8_t *omask, int skip_fresh,
                                                                  uint64_t *__restrict__ eb,
                                                                  const uint32_t *__restrict__ list)
 {
