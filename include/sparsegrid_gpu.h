@@ -258,7 +258,8 @@ int sg_batch_destroy(sg_batch *b);
 int sg_batch_add(sg_batch *b, sg_grid *g, int64_t tag, double tol);
 int sg_batch_live(sg_batch *b);
 /* launch shape of the batched sweep kernel: waves (64 lanes, one chunk tile each) per
- * workgroup, 1 / 2 / 4 / 8 (LDS tile per wave: 3.2 KB FP32, 6.4 KB FP64), default 4 */
+ * workgroup, 1 / 2 / 4 / 8, or 0 (default): 1 up to 1024 tiles, 4 beyond.  LDS tile per wave:
+ * 4.8 KB where both colours of an FP32 sweep run in one pass, else 3.2 KB FP32, 6.4 KB FP64 */
 #define SG_TUNE_BATCH_WAVES 5
 /* at most this many workgroups per launch, waves then loop over tiles; 0 (default): one
  * tile per wave */

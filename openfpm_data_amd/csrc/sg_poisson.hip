@@ -1134,7 +1134,8 @@ int sg_batch_set_tuning(sg_batch *b, int key, int64_t value)
     if (!b) return fail(SG_E_ARG, "null batch");
     switch (key) {
     case SG_TUNE_BATCH_WAVES:
-        if (value != 1 && value != 2 && value != 4 && value != 8) return fail(SG_E_ARG, "waves must be 1, 2, 4 or 8");
+        if (value != 0 && value != 1 && value != 2 && value != 4 && value != 8)
+            return fail(SG_E_ARG, "waves must be 0 (by size), 1, 2, 4 or 8");
         b->waves = (int)value;
         break;
     case SG_TUNE_BATCH_MAX_WGS:

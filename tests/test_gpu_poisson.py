@@ -267,3 +267,29 @@ def test_live_grid_changed_between_steps(P, sweeps):
     for a, h in zip(grid_values(False), grid_values(True)):
         for x, y in zip(a, h):
             np.testing.assert_array_equal(x.view(np.uint8), y.view(np.uint8))
+
+
+def test_waves_by_size_can_be_restored(P):
+    """0 waves, the default (by the number of tiles), is accepted after another setting; the
+    solutions do not depend on it."""
+    import torch
+    from openfpm_data_amd._capi import SgError
+    spec = _small_grids(1, 7, 64)[0]
+    out = []
+    for settings in ((), (4,), (8, 0)):
+        g = P.poisson_grid(spec["size"], spec["chunk_ids"], spec["f"])
+        b = P.PoissonBatch(P.make_params(tol=1e-8), torch.cuda.current_stream())
+        for w in settings:
+            b.set_tuning(C.TUNE_BATCH_WAVES, w)
+        for w in (-1, 3, 16):
+            with pytest.raises(SgError):
+                b.set_tuning(C.TUNE_BATCH_WAVES, w)
+        b.add(g, 0)
+        while b.live():
+            b.step()
+        res = b.poll()[0][1]
+        b.close()
+        out.append((res["sweeps"], g.prop(res["solution_prop"])))
+    for sweeps, u in out[1:]:
+        assert sweeps == out[0][0]
+        np.testing.assert_array_equal(u, out[0][1])
