@@ -173,17 +173,15 @@ void DevicePool::free(void *p)
     cache_.emplace(it->second, p);
 }
 
-void DevicePool::hand_back(void *p)
+void DevicePool::release_cached()
 {
-    auto it = p ? sizes_.find(p) : sizes_.end();
-    if (it == sizes_.end()) return;
-    {
-        std::lock_guard<std::mutex> lk(g_idle_mu);
-        g_idle.emplace(it->second, std::make_pair(p, devs_[p]));
+    std::lock_guard<std::mutex> lk(g_idle_mu);
+    for (auto &kv : cache_) {
+        g_idle.emplace(kv.first, std::make_pair(kv.second, devs_[kv.second]));
+        sizes_.erase(kv.second);
+        devs_.erase(kv.second);
     }
-    live_ -= it->second;
-    sizes_.erase(it);
-    devs_.erase(p);
+    cache_.clear();
 }
 
 void DevicePool::release()

@@ -65,7 +65,8 @@ public:
     void *alloc(size_t bytes);
     void free(void *p);
     void release();   // every block of this handle to the process-wide idle cache
-    void hand_back(void *p);  // one block there (the same holds: the handle's stream is idle)
+    void release_cached();  // the blocks not in use there (the same holds: the stream is idle)
+    size_t cached_bytes() const { return held_bytes() - live_; }
     void trim();      // hipFree this handle's cached blocks and the idle cache of the device
     size_t live_bytes() const { return live_; }
     size_t held_bytes() const;

@@ -48,6 +48,8 @@ BATCH_CHUNK_BYTES = 512 * 4 + 20 * 4
 # pass the budget.
 KEEP_TEMPORARIES = 32 << 20
 KEEP_BYTES = 256 << 20
+# what the batch keeps of retired grids' buffers, which no trim frees
+BATCH_CACHE = 64 << 20
 
 
 def resident_bytes(nchunks):
@@ -116,11 +118,12 @@ class Admission:
             self.idle += n
 
     def take_trim(self, force=False):
-        """Whether the idle memory is to be freed now; it then counts as freed."""
+        """Whether the idle memory is to be freed now; it then counts as freed, but for what the
+        batch may keep."""
         with self.lock:
             due = force or self.idle > KEEP_BYTES or self.used + self.idle > self.budget
             if due:
-                self.idle = 0
+                self.idle = min(self.idle, BATCH_CACHE)
             return due
 
 

@@ -59,22 +59,22 @@ def test_idle_memory_is_bounded():
     a.release(1)
     assert a.idle == sizes[0] + sizes[1] and not a.take_trim()  # two thirds: kept
     a.release(2)
-    assert a.take_trim() and a.idle == 0 and not a.take_trim()
+    assert a.take_trim() and a.idle == S.BATCH_CACHE and not a.take_trim()
     a.used = sizes[3] + sizes[4]
     a.release(4)
-    assert not a.take_trim()  # half of KEEP_BYTES, and the budget has room
-    a.used += S.KEEP_BYTES // 2 + 1
-    assert a.take_trim()
-    a.booked[5] = 1
-    a.release(5)
-    assert a.take_trim(force=True) and a.idle == 0
+    assert not a.take_trim()  # half of KEEP_BYTES more, and the budget has room
+    a.used += a.budget - a.used - a.idle
+    assert not a.take_trim()
+    a.used += 1
+    assert a.take_trim() and a.idle == S.BATCH_CACHE
+    assert a.take_trim(force=True)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("build_thread", [True, False])
 def test_served_memory_is_returned(build_thread):
     """While a server lives, the device memory of the grids that it served, its batch's sweep
-    buffers among it, can be freed by a trim: nothing of it stays with the batch."""
+    buffers among it, can be freed by a trim but for the bytes a batch may keep."""
     import torch
     from openfpm_data_amd import _capi as C
     from openfpm_data_amd import poisson as P
@@ -83,10 +83,12 @@ def test_served_memory_is_returned(build_thread):
     tiny = P.poisson_grid((32,) * 3, np.arange(64), rng.uniform(-1, 1, (64, 512)))
     srv = S.PoissonServer(budget_bytes=8 << 30, build_thread=build_thread)
     reqs = []
-    for i, edge in enumerate((96, 224, 64, 160, 128)):
+    for i, edge in enumerate((96, 232, 64, 224, 216, 208)):
         n = (edge // 8) ** 3
         reqs.append({"id": i, "size": (edge,) * 3, "chunk_ids": np.arange(n),
                      "f": rng.uniform(-1, 1, (n, 512)).astype(np.float32), "tol": 1e-2})
+    chunks = sum(len(r["chunk_ids"]) for r in reqs)
+    assert chunks * S.BATCH_CHUNK_BYTES > 2 * S.BATCH_CACHE
     srv.run(reqs[2:3], [0.0])  # code objects, streams
 
     def free_bytes():
@@ -98,9 +100,7 @@ def test_served_memory_is_returned(build_thread):
     before = free_bytes()
     recs, summ = srv.run(reqs, [0.0] * len(reqs))
     assert summ["served"] == len(reqs)
-    # the batch's sweep buffers of the grids are 75 MB; its work lists may grow by 0.8 MB
-    chunks = sum(len(r["chunk_ids"]) for r in reqs)
-    assert before - free_bytes() < min(16 << 20, chunks * S.BATCH_CHUNK_BYTES // 4)
+    assert before - free_bytes() < S.BATCH_CACHE + (16 << 20)  # the work lists: 2 MB
     srv.close()
 
 
