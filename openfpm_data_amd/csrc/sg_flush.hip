@@ -2815,7 +2815,10 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
     df.planes = g->dim == 3 && g->edge == 8 && (g->ebits_valid || g->nchunks == 0);
     // few records a touched chunk (8 on average at most) and old chunks among them: those are
     // folded slot by slot in place, after the old chunks have moved if the set grows.  With more
-    // records a chunk a wave per chunk reads and writes it whole at the copy's rate.
+    // records a chunk a wave per chunk reads and writes it whole at the copy's rate.  Merges into
+    // 20,000 of 40,000 chunks, us with few / without: 7 records in each 130 / 162, 9 in each 194 /
+    // 160, 16 203 / 169; with 2% of the touched chunks new 7 232 / 252, 9 307 / 252, 16 319 / 258.
+    // The average misses uneven ones: 2 records in most and 720 in 1% (9 on average) 157 / 182.
     const bool few = n <= kFewRecords * nnew && (int64_t)hw[0] < nnew && ((csz % 16) == 0 || hw[0] == 0);
     df.copy_touched = few;
     // the list of chunks with more records: allocated before the chunk set changes, so that a
@@ -2925,8 +2928,9 @@ int flush_grouped_impl(sg_grid *g, const int32_t *ops, bool *taken)
     if (!fresh_ok || df.nfresh < nnew) {
         // chunks that existed before (and new ones when the image path is not taken)
         const int waves = std::max(1, std::min(4, 65536 / S.bytes));
-        // one wave per touched chunk (a wave's loop then runs once)
-        // (with a list: at most n / (kFewRecords + 1) chunks are on it, waves loop over it)
+        // Without a list one wave per touched chunk, whose loop runs once.  The list's length is
+        // not known here: at most n / (kFewRecords + 1) chunks, which up to 2048 workgroups of
+        // waves loop over.
         const int64_t most = list ? std::min<int64_t>(2048 * waves, n / (kFewRecords + 1) + 1) : nnew;
         const int64_t groups = (most + waves - 1) / waves;
         const dim3 fgrid((unsigned)groups), fblk(64 * waves);

@@ -12,7 +12,7 @@
 // Batching: every launch covers all live grids; workgroup waves take tiles of a (grid,
 // chunk) work list (per-grid prefix sums of chunk counts, binary-searched per wave), so
 // grids of uneven size share launches and small grids cost no launches of their own.
-// The inner sweep sequence can be captured once per live set in a hipGraph and replayed.
+// An inner sweep sequence that comes again is captured in a hipGraph and replayed.
 // Grids join and leave the batch between outer iterations (continuous batching).
 //
 // SOR relaxation: omega is estimated per grid from the residual reduction rho of each
@@ -239,7 +239,7 @@ __global__ __launch_bounds__(64 * WAVES) void rbsor_batch_kernel(const PGrid *__
 // against 2 x 363 of two half sweeps); before the rows were kept split by colour, with a
 // select for every operand, it had 680 and a sweep of 48 grids took 115 us.  Those 48 grids
 // (58,600 chunks): 2 x 64 us a sweep in half sweeps, 66 us here; 152 chunks 2 x 4.8 -> 3.9 us.
-// Measured and not kept (ms a solve of the 48, 10.0 as it is): 1, 2 or 8 waves a workgroup
+// Measured and not kept (ms a solve of the 48, 10.0 then as it is): 1, 2 or 8 waves a workgroup
 // 10.4, 10.3, 10.2; plain stores 10.4; contiguous tile ranges per XCD 10.1; groups of grids of
 // 16,384 tiles one after the other, so that a group stays in the Infinity Cache, 11.6 (the
 // launches' tails cost more than the misses).
@@ -516,7 +516,8 @@ __device__ __forceinline__ void fused_tile(const PGrid &g, uint32_t c, float *ti
 
 // Sweep `sweep` of the live grids, both colours (work list as for rbsor_batch_kernel).  A tile
 // per wave, or with LOOP as many as the launch's size needs: without the loop the per-lane
-// offsets are not kept across it, which leaves registers for 5 waves a SIMD instead of 4.
+// offsets are not kept across it, 75 registers instead of 104, which allow 6 waves a SIMD
+// instead of 4.
 template <int WAVES, bool LOOP>
 __global__ __launch_bounds__(64 * WAVES) void rbsor_fused_kernel(const PGrid *__restrict__ grids,
                                                                 const int64_t *__restrict__ prefix,
@@ -828,9 +829,9 @@ int upload_worklist(sg_batch *b, bool defect_view, const std::vector<int> &order
     return SG_OK;
 }
 
-// waves per workgroup of the sweeps: 4 (neighbour chunks share a CU's cache: 48 grids 11.3 ms,
-// 12.2 ms with 1), or 1 while the tiles are fewer than would give every CU 4 waves (152
-// tiles: 4.3 us a sweep with 4 waves on 38 CUs, 3.9 us with 1 on 152)
+// waves per workgroup of the sweeps: 4 (neighbour chunks share a CU's cache: the 48 grids above
+// 10.0 ms, 10.4 ms with 1), or 1 while the tiles are fewer than would give every CU 4 waves
+// (152 tiles: 4.3 us a sweep with 4 waves on 38 CUs, 3.9 us with 1 on 152)
 int sweep_waves(const sg_batch *b, int64_t nt)
 {
     if (b->waves > 0) return b->waves;

@@ -876,9 +876,10 @@ template <typename T> struct BoxIn {
 
 template <typename T>
 __device__ __forceinline__ void box_load(BoxIn<T> &in, int64_t c, const int32_t *__restrict__ nn,
-                                const uint8_t *__restrict__ mask, const T *__restrict__ src, int lane,
+                                         const uint8_t *__restrict__ mask, const T *__restrict__ src, int lane,
                                          bool skip_xm = false, bool skip_xp = false)
 {
+    // skip_xm / skip_xp: the -x / +x ghosts come from a chunk the caller holds
     const int32_t *row_nn = nn + c * 27;
     auto chunk_of = [&](int dx, int dy, int dz) -> int64_t {
         return (dx == 0 && dy == 0 && dz == 0) ? c : (int64_t)row_nn[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)];

@@ -68,11 +68,13 @@ def _descs(rng, dim, size):
     return out
 
 
-# chunk counts around the workgroups' 8 (2D) and 4 (3D) chunks, ragged last chunks
+# chunk counts around the workgroups' 4 chunks (1, 3, 4, 5, 4 k + 1 and others), ragged last chunks
 @pytest.mark.parametrize("lin", ["smb", "zmb"])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("dim,edge,size", [(2, 16, (16, 16)), (2, 16, (130, 17)), (2, 16, (75, 91)), (2, 16, (200, 170)),
-                                           (3, 8, (8, 8, 8)), (3, 8, (33, 9, 17)), (3, 8, (41, 30, 25))])
+                                           (2, 16, (48, 16)), (2, 16, (30, 31)), (2, 16, (16, 77)), (2, 16, (269, 13)),
+                                           (3, 8, (8, 8, 8)), (3, 8, (33, 9, 17)), (3, 8, (41, 30, 25)),
+                                           (3, 8, (24, 7, 8)), (3, 8, (15, 16, 8)), (3, 8, (8, 8, 37)), (3, 8, (133, 5, 6))])
 def test_star_kernels_match_the_oracle(G, oracle, dim, edge, size, dtype, lin):
     rng = np.random.default_rng(dim * 1000 + size[0])
     a, b = _pair(G, oracle, dim, edge, size, dtype, 31 + size[0], lin)
