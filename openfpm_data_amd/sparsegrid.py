@@ -305,10 +305,12 @@ class SparseGridGpu:
     def set_prop(self, p, data):
         if _is_device(data):
             # values are taken from the tensor's memory as it lies, so that has to hold them all
-            need = self.num_chunks() * self.chunk_size * self.dtypes[p].itemsize
-            have = data.untyped_storage().nbytes() - data.storage_offset() * data.element_size()
-            if have < need:
-                raise ValueError("property %d: %d bytes from the tensor's start where %d are expected" % (p, have, need))
+            # (objects that only look like tensors are left to the C call's own check)
+            if hasattr(data, "untyped_storage"):
+                need = self.num_chunks() * self.chunk_size * self.dtypes[p].itemsize
+                have = data.untyped_storage().nbytes() - data.storage_offset() * data.element_size()
+                if have < need:
+                    raise ValueError("property %d: %d bytes from the tensor's start where %d are expected" % (p, have, need))
             C.check(self._lib.sg_set_prop(self._h, p, _ptr(data), C.SG_MEM_DEVICE))
             return
         a = np.ascontiguousarray(np.asarray(data, dtype=self.dtypes[p]))

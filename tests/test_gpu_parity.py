@@ -1193,6 +1193,12 @@ def test_set_prop_checks_device_memory(G):
     check(0)
     g.set_prop(0, x[100:].view(torch.int32))
     check(100)
+    class Handle:  # device memory that is no tensor
+        is_cuda = True
+        data_ptr = staticmethod(x[50:].data_ptr)
+
+    g.set_prop(0, Handle())
+    check(50)
     pin = torch.empty(n, dtype=torch.float32, pin_memory=True)
     pin.copy_(x[7:n + 7])
     C.check(g._lib.sg_set_prop(g._h, 0, ctypes.c_void_p(pin.data_ptr()), C.SG_MEM_DEVICE))

@@ -92,7 +92,8 @@ def test_star_kernels_match_the_oracle(G, oracle, dim, edge, size, dtype, lin):
 
 @pytest.mark.parametrize("dim,edge,n", [(2, 16, 600), (3, 8, 72)])
 def test_many_workgroups(G, oracle, dim, edge, n):
-    """More chunks than one workgroup per XCD: the XCD-ranged chunk order covers them all."""
+    """More chunks than one workgroup per XCD: the order in which they are dealt to the XCDs covers
+    them all."""
     a, b = _pair(G, oracle, dim, edge, (n,) * dim, np.float32, 5, tag=False)
     for d in _descs(np.random.default_rng(1), dim, (n,) * dim)[12:]:
         a.apply_stencil(d)
